@@ -313,6 +313,9 @@ struct ModeWeights {
   DeviceBuffer tail_bias;
   DeviceBuffer body_consts;        // epilogue constants of the fused body (kBodyConsts floats)
   DeviceBuffer fp32;               // FP32 policy: the whole weight image (kernels.hpp kF32*)
+  // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
+  DeviceBuffer f32_refine, f32_tail;
+  F32SplitScale f32_refine_scale{}, f32_tail_scale{};
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -327,6 +330,17 @@ struct ModeWeights {
     fn(tail_bias);
     fn(body_consts);
     fn(fp32);
+    fn(f32_refine);
+    fn(f32_tail);
+  }
+  F32Weights f32_weights() const {
+    F32Weights W;
+    W.image = fp32.as<float>();
+    W.refine = f32_refine.ptr;
+    W.tail = f32_tail.ptr;
+    W.refine_scale = f32_refine_scale;
+    W.tail_scale = f32_tail_scale;
+    return W;
   }
   size_t bytes() const {
     size_t n = 0;
@@ -498,12 +512,43 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
       img[off + size_t(ks * ks) * cin * cout + o] = b[o];
     }
   };
+  // hi / lo FP16 fragments of a layer's weights, scaled so that the largest lies in [2^14, 2^15): chunk f of
+  // `chunks`, row m, slot s is the weight at(f, m, s); the fragment order is chunk, then hi and lo
+  auto split = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, int chunks, auto at, DeviceBuffer& dst) {
+    const float* w = w32(l, cout, cin, ks);
+    const float* b = a.need(l + ".bias", kF32, {cout}).f32();
+    double top = 0, gain = 0, offset = 0;
+    const size_t per = size_t(cin) * ks * ks;
+    for (uint32_t o = 0; o < cout; ++o) {
+      double sum = 0;
+      for (size_t i = 0; i < per; ++i) {
+        top = std::max(top, std::fabs((double)w[o * per + i]));
+        sum += std::fabs((double)w[o * per + i]);
+      }
+      gain = std::max(gain, sum);
+      offset = std::max(offset, std::fabs((double)b[o]));
+    }
+    F32SplitScale sc;
+    sc.exponent = top > 0 ? std::min(std::max(14 - std::ilogb(top), -60), 24) : 0;
+    sc.gain = (float)(1.001 * gain);
+    sc.offset = (float)(1.001 * offset);
+    dst.upload(pack_frags<uint16_t>(2 * chunks, 8, [&](int f, int m, int s) {
+      const float v = std::ldexp(w[at(f / 2, m, s)], sc.exponent);
+      const uint16_t hi = f32_to_f16_bits(v);
+      return f % 2 ? f32_to_f16_bits(v - f16_bits_to_f32(hi)) : hi;
+    }));
+    return sc;
+  };
   layer("project", 32, 32, 1, kF32Project, 0.1f);
   layer("compress", 64, 128, 1, kF32Compress, 0.1f);
   for (int l = 0; l < 4; ++l) layer("bottleneck" + std::to_string(l), 64, 32, 3, kF32Grouped + l * kF32GroupedStride, 0.1f);
   layer("expand", 128, 64, 1, kF32Expand, 0.1f);
   layer("refine", 64, 32, 3, kF32Refine, 0.1f);
   layer("tail", 64, 64, 1, kF32Tail, 1.0f);
+  rt.f32_refine_scale = split("refine", 64, 32, 3, 36,
+                              [](int f, int m, int s) { return ((16 * (f / 9) + m) * 32 + s) * 9 + f % 9; }, rt.f32_refine);
+  rt.f32_tail_scale = split("tail", 64, 64, 1, 8,
+                            [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; }, rt.f32_tail);
   for (int i = 0; i < 100; ++i) img[kF32Base + i] = base[i];
   for (int i = 0; i < 1600; ++i) img[kF32Basis + i] = basis[i];
   for (int i = 0; i < 24; ++i) img[kF32Analysis + i] = rt.analysis[i];
@@ -1026,9 +1071,9 @@ static void enqueue_fp32(const ModeWeights& w, const Geometry& g, const Scratch&
   if (ev) check_hip(hipEventRecord(ev[0], s), "hipEventRecord");
   float* lows[5];
   for (int i = 0; i < 5; ++i) lows[i] = static_cast<float*>(sc.low[i]);
-  check_launch(launch_f32_controller(g.in_fp32, d_in, w.fp32.as<float>(), static_cast<float*>(sc.skip), lows[0], lows[1],
+  check_launch(launch_f32_controller(g.in_fp32, d_in, w.f32_weights(), static_cast<float*>(sc.skip), lows[0], lows[1],
                                      g.nlow == 5 ? lows : nullptr, static_cast<float*>(sc.work), static_cast<float*>(sc.meta),
-                                     g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, s, ev),
+                                     g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, g.cus, s, ev),
                "FP32 controller launch", s);
   check_launch(launch_f32_head(g.in_fp32, g.out_fp32, d_in, static_cast<const float*>(sc.meta), w.fp32.as<float>(), d_out,
                                g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, sc.nonfinite, s),
@@ -1067,7 +1112,7 @@ static std::string startup_report(const Runtime& rt) {
     << " body=" << (g.fused ? (g.fused_rgb ? "fused-analysis-project-compress-4x-grouped-expand"
                                            : "project+fused-compress-4x-grouped-expand")
                             : "per-layer-kernels")
-    << " body_mfma=" << (rt.mode == 0 ? "f16" : rt.mode == 1 ? "fp8" : rt.mode == 2 ? "i8" : rt.mode == 3 ? "f16-on-e4m3-values" : "none-fp32-fma")
+    << " body_mfma=" << (rt.mode == 0 ? "f16" : rt.mode == 1 ? "fp8" : rt.mode == 2 ? "i8" : rt.mode == 3 ? "f16-on-e4m3-values" : "f16-hi-lo-splits-of-fp32")
     << " head=" << (g.fused ? "fused-refine-tail-reconstruction" : "refine-tail+reconstruction")
     << " source=" << g.W << 'x' << g.H << " batch=" << g.batch << " padded=" << g.Wp << 'x' << g.Hp
     << " packed=" << g.Wq << 'x' << g.Hq << " low=" << g.Wl << 'x' << g.Hl << " source_pad=" << g.px << ','

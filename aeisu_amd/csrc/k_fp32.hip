@@ -7,11 +7,15 @@
 //   meta  [B][Hq][Wq][64]   refine 3x3 + LeakyReLU -> tail 1x1 (the packed coefficients)
 // and the head writes the clipped 2x frame.
 //
-// One thread per output pixel holds all its output channels in registers and walks the input
-// channels; the weights, laid out [tap][ci][co] (kernels.hpp kF32*), are read at wave-uniform
-// addresses, so they come through the scalar cache and feed the FMAs as scalar operands.  Every
-// product is an FP32 fmaf; the sums run over input channels (and taps) in a fixed order, which
-// differs from the reference's convolution order only by FP32 rounding.
+// Two forms of kernel:
+//  * one thread per output pixel holds all its output channels in registers and walks the input
+//    channels; the weights, laid out [tap][ci][co] (kernels.hpp kF32*), are read at wave-uniform
+//    addresses, so they come through the scalar cache and feed the FP32 FMAs as scalar operands;
+//  * products of hi / lo FP16 splits on the MFMA (below), FP32 sums.
+// The sums run in a fixed order, which differs from the reference's convolution order only by FP32
+// rounding.
+#include <algorithm>
+
 #include "common.hpp"
 #include "features.hpp"
 #include "kernels.hpp"
@@ -198,63 +202,236 @@ __global__ __launch_bounds__(kF32Threads) void f32_expand_kernel(const float* __
   }
 }
 
-// ---- refine 3x3 (32 -> 64) + LeakyReLU + tail 1x1 (64 -> 64): a 16 x 16 tile of packed pixels per
-// block (one pixel per thread), its 18 x 18 input halo (32 channels, 36 floats apart) staged in LDS
-// as in the grouped layers; the tail in two halves of 32 outputs (64 + 32 accumulators within 128
-// VGPRs: four waves per SIMD; all 64 + 64 took 129)
-__global__ __launch_bounds__(kF32Threads) void f32_refine_tail_kernel(const float* __restrict__ work,
-                                                                      const float* __restrict__ wimg,
-                                                                      float* __restrict__ meta, int Hq, int Wq, int batch) {
-  __shared__ __attribute__((aligned(16))) float tile[kF32GH * kF32GH * kF32GPix];
-  const int tx_n = (Wq + kF32GT - 1) / kF32GT, ty_n = (Hq + kF32GT - 1) / kF32GT;
-  const int b = (int)blockIdx.x / (tx_n * ty_n), rem = (int)blockIdx.x - b * tx_n * ty_n;
-  const int y0 = (rem / tx_n) * kF32GT, x0 = (rem % tx_n) * kF32GT;
-  const int tid = threadIdx.x;
-  for (int i = tid; i < kF32GH * kF32GH * 8; i += kF32Threads) {
-    const int pix = i >> 3, q = i & 7, py = pix / kF32GH, px = pix - py * kF32GH;
-    const int y = y0 + py - 1, x = x0 + px - 1;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (y >= 0 && y < Hq && x >= 0 && x < Wq)
-      v = *reinterpret_cast<const float4*>(work + (((size_t)b * Hq + y) * Wq + x) * 32 + 4 * q);
-    *reinterpret_cast<float4*>(&tile[pix * kF32GPix + 4 * q]) = v;
-  }
-  __syncthreads();
-  const int ty = tid / kF32GT, tx = tid - ty * kF32GT;
-  const float* wr = wimg + kF32Refine;
-  const float* wt = wimg + kF32Tail;
-  float r[64];
+// ---- split products on the FP16 MFMA ----------------------------------------------------------------
+// An FP32 operand x is scaled by a power of two and written as hi + lo, hi = fp16(x), lo = fp16(x - hi),
+// and a product is hi hi' + (hi lo' + lo hi'): three FP16 MFMAs in place of the FP32 FMAs, at 5 times the
+// rate of the FP32 MFMA and 10 times that of the unpacked FMA.  hi + lo carries 22 to 23 bits, and the
+// MFMA rounds its FP32 accumulator once per 8 products where the FMA chain rounds at every one, so the
+// result is nearer to the exact sum than the chain's (64 x 96 frames of three kinds, both checkpoints,
+// against 64 bits: coefficients 0.72 to 0.98 of the chain's error).  The cross terms go to an accumulator
+// of their own: added to the main sum they would be rounded at its magnitude.
+//
+// The scale keeps FP32's range: the largest magnitude of the tile (finite values only) goes to
+// [2^14, 2^15), so nothing overflows FP16, and a value is cut off at 2^-38 of the tile's largest.
+__device__ __forceinline__ float residual_lo(float v, unsigned w) {   // v - (low half of w), exact
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
+  return r;
+}
+__device__ __forceinline__ float residual_hi(float v, unsigned w) {
+  float r;
+  asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
+  return r;
+}
+// Four values -> their hi halves (two dwords) and lo halves.
+__device__ __forceinline__ void split4(float a, float b, float c, float d, u2& hi, u2& lo) {
+  const unsigned h0 = pack_h2(a, b), h1 = pack_h2(c, d);
+  hi = u2{h0, h1};
+  lo = u2{pack_h2(residual_lo(a, h0), residual_hi(b, h0)), pack_h2(residual_lo(c, h1), residual_hi(d, h1))};
+}
+__device__ __forceinline__ float pow2f(int e) { return __builtin_bit_cast(float, (unsigned)(e + 127) << 23); }
+// Exponent e with m 2^e in [2^14, 2^15), for a finite m >= 0 (clamped for tiny m).
+__device__ __forceinline__ int scale_exponent(float m) {
+  return min(14 + 127 - (int)(__builtin_bit_cast(unsigned, m) >> 23), 100);
+}
+__device__ __forceinline__ float finite_abs(float v) {
+  const float a = fabsf(v);
+  return a < __builtin_inff() ? a : 0.f;
+}
+__device__ __forceinline__ float inverse_scale(int e) { return pow2f(-min(max(e, -126), 126)); }
+__device__ __forceinline__ float wave_max(float m) {
 #pragma unroll
-  for (int co = 0; co < 64; ++co) r[co] = 0.f;
+  for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+  return m;
+}
+
+// ---- 3x3 layers: persistent blocks of four waves over tiles of 16 x TH pixels -----------------------
+// Wave w serves output channels 32 (w & 1) .. + 31 (two MFMA row tiles) of the pixel rows of its half
+// (w >> 1), and keeps its 36 weight fragments (9 taps x 2 tiles x hi, lo: 144 VGPRs) for the launch: from
+// LDS or L2 the fragments would be read once per pixel row and more often than the activations.  The tile's
+// input halo is staged in LDS as hi and lo halves, split once per value.  Two blocks per CU (two waves per
+// SIMD at 256 VGPRs): one block's staging and barriers overlap the other's products.
+constexpr int kConvTW = 16, kConvPW = kConvTW + 2;
+constexpr int kConvThreads = 256;
+
+__device__ __forceinline__ void conv_weights(h8 (&A)[9][2][2], const h8* __restrict__ frag, int role, int lane) {
+#pragma unroll
+  for (int T = 0; T < 2; ++T)
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+      for (int part = 0; part < 2; ++part) A[tap][T][part] = frag[(((2 * role + T) * 9 + tap) * 2 + part) * 64 + lane];
+}
+
+// One row of 16 pixels: acc[T] = sum over the 9 taps of the wave's two row tiles.  p: the lane's operand of
+// the top left tap (hi; lo is `lo` bytes further), rows `row` bytes apart, pixels `pix`.
+__device__ __forceinline__ void conv_row(const unsigned char* p, int lo, int row, int pix, const h8 (&A)[9][2][2],
+                                         f4 (&acc)[2]) {
+  f4 small[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+  acc[0] = acc[1] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
   for (int tap = 0; tap < 9; ++tap) {
-    const float* src = &tile[((ty + tap / 3) * kF32GH + tx + tap % 3) * kF32GPix];
-    for (int c0 = 0; c0 < 32; c0 += 4) {
-      const float4 x4 = *reinterpret_cast<const float4*>(src + c0);
-      const float xs[4] = {x4.x, x4.y, x4.z, x4.w};
+    const unsigned char* q = p + (tap / 3) * row + (tap % 3) * pix;
+    const h8 bh = *reinterpret_cast<const h8*>(q), bl = *reinterpret_cast<const h8*>(q + lo);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float* w = wr + (tap * 32 + c0 + e) * 64;
+    for (int T = 0; T < 2; ++T) acc[T] = mfma_f16(A[tap][T][0], bh, acc[T]);
 #pragma unroll
-        for (int co = 0; co < 64; ++co) r[co] = fmaf(xs[e], w[co], r[co]);
-      }
+    for (int T = 0; T < 2; ++T) small[T] = mfma_f16(A[tap][T][0], bl, small[T]);
+#pragma unroll
+    for (int T = 0; T < 2; ++T) small[T] = mfma_f16(A[tap][T][1], bh, small[T]);
+  }
+#pragma unroll
+  for (int T = 0; T < 2; ++T) acc[T] += small[T];
+}
+
+// The tile's largest finite magnitude over all waves, through `red` (one float per wave).  Ends with a
+// block barrier, before which every wave has left the previous tile's LDS data.
+__device__ __forceinline__ float block_max(float m, float* red, int wave, int lane) {
+  m = wave_max(m);
+  if (lane == 0) red[wave] = m;
+  lds_barrier();
+  const float4 r = *reinterpret_cast<const float4*>(red);
+  return fmaxf(fmaxf(r.x, r.y), fmaxf(r.z, r.w));
+}
+
+template <int TH>
+struct RefineLayout {
+  static constexpr int Rows = TH + 2, Pix = 144, Chunks = Rows * kConvPW * 8;   // float4 chunks of the halo
+  static constexpr int Per = (Chunks + kConvThreads - 1) / kConvThreads;
+  static constexpr int RPix = 272;                   // refine outputs: 64 channels hi, 64 lo, pad
+  static constexpr int OffR = Rows * kConvPW * Pix, OffRed = OffR + TH * kConvTW * RPix;
+  static constexpr int Lds = OffRed + 16;
+};
+struct F32ConvTiles {
+  int H, W, tiles_x, tiles_y, num;
+};
+template <int PER, int CH>
+__device__ __forceinline__ void conv_fetch(float4 (&v)[PER], const float* __restrict__ in, const F32ConvTiles& G, int tidx,
+                                           int th, int chunks, int tid) {
+  const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per;
+  const int ty = rem / G.tiles_x, y0 = ty * th - 1, x0 = (rem - ty * G.tiles_x) * kConvTW - 1;
+  const float* f = in + (size_t)b * G.H * G.W * CH;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = tid + k * kConvThreads, pix = i / (CH / 4), c = i % (CH / 4);
+    const int py = pix / kConvPW, y = y0 + py, x = x0 + pix - py * kConvPW;
+    const bool in_grid = (unsigned)y < (unsigned)G.H && (unsigned)x < (unsigned)G.W && i < chunks;
+    v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (in_grid) v[k] = *reinterpret_cast<const float4*>(f + ((size_t)y * G.W + x) * CH + 4 * c);
+  }
+}
+template <int PER>
+__device__ __forceinline__ float chunk_max(const float4 (&v)[PER]) {
+  float m = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) m = fmaxf(m, fmaxf(fmaxf(fabsf(v[k].x), fabsf(v[k].y)), fmaxf(fabsf(v[k].z), fabsf(v[k].w))));
+  if (!(m < __builtin_inff())) {                     // an infinity somewhere: the largest finite value
+    m = 0.f;
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      m = fmaxf(m, fmaxf(fmaxf(finite_abs(v[k].x), finite_abs(v[k].y)), fmaxf(finite_abs(v[k].z), finite_abs(v[k].w))));
+  }
+  return m;
+}
+// Splits the staged chunks into LDS: pixel stride `pix`, hi halves of the CH channels first, lo halves after.
+template <int PER, int CH>
+__device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char* lds, int pix_bytes, float s, int chunks,
+                                           int tid) {
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = tid + k * kConvThreads, pix = i / (CH / 4), c = i % (CH / 4);
+    if (i < chunks) {
+      u2 hi, lo;
+      split4(v[k].x * s, v[k].y * s, v[k].z * s, v[k].w * s, hi, lo);
+      unsigned char* d = lds + pix * pix_bytes + 8 * c;
+      *reinterpret_cast<u2*>(d) = hi;
+      *reinterpret_cast<u2*>(d + 2 * CH) = lo;
     }
   }
-  const int qy = y0 + ty, qx = x0 + tx;
-  if (qy >= Hq || qx >= Wq) return;
+}
+
+// refine 3x3 (32 -> 64) + LeakyReLU + tail 1x1 (64 -> 64).  One thread per pixel with FP32 FMAs was bound by
+// their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 86 and 9.5.  Its 210 MB take 41 us
+// of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (416 KB per tile), which
+// two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
+// (scaled by a bound of their magnitude from the tile's input maximum and the weights) and wave w computes
+// tail channels 16 w .. + 15 from them.
+template <int TH>
+__global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const float* __restrict__ work,
+                                                                          const h8* __restrict__ rfrag,
+                                                                          const h8* __restrict__ tfrag,
+                                                                          const float* __restrict__ rbias,
+                                                                          const float* __restrict__ tbias,
+                                                                          float* __restrict__ meta, F32ConvTiles G,
+                                                                          F32SplitScale rs, F32SplitScale ts) {
+  typedef RefineLayout<TH> LY;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  float* red = reinterpret_cast<float*>(smem + LY::OffRed);
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, role = wave & 1, half = wave >> 1;
+  const int n = lane & 15, g = lane >> 4;
+  float4 v[LY::Per];
+  int tidx = tile_of(0, G.num);
+  if (tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
+  h8 A[9][2][2], At[2][2];
+  conv_weights(A, rfrag, role, lane);
 #pragma unroll
-  for (int ci = 0; ci < 64; ++ci) r[ci] = leaky01(r[ci] + wr[18432 + ci]);
-  float* out = meta + (((size_t)b * Hq + qy) * Wq + qx) * 64;
-  for (int h = 0; h < 64; h += 32) {
-    float t[32];
+  for (int k = 0; k < 2; ++k)
 #pragma unroll
-    for (int co = 0; co < 32; ++co) t[co] = 0.f;
+    for (int part = 0; part < 2; ++part) At[k][part] = tfrag[((wave * 2 + k) * 2 + part) * 64 + lane];
+  f4 rb[2];
 #pragma unroll
-    for (int ci = 0; ci < 64; ++ci)
+  for (int T = 0; T < 2; ++T) rb[T] = *reinterpret_cast<const f4*>(rbias + 32 * role + 16 * T + 4 * g);
+  const f4 tb = *reinterpret_cast<const f4*>(tbias + 16 * wave + 4 * g);
+  const int iters = tile_iters(G.num);
+  for (int it = 0; it < iters; ++it) {
+    if (tidx >= G.num) break;                        // block-uniform
+    const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per;
+    const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
+    const float m = block_max(chunk_max(v), red, wave, lane);
+    const int ex = scale_exponent(m);
+    conv_stage<LY::Per, 32>(v, smem, LY::Pix, pow2f(ex), LY::Chunks, tid);
+    tidx = tile_of(it + 1, G.num);
+    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
+    lds_barrier();
+    // |refine output| <= gain m + offset
+    const int er = scale_exponent(fminf(fmaf(rs.gain, m, rs.offset), 0x1p126f));
+    const float inv = inverse_scale(ex + rs.exponent), sr = pow2f(er);
+    for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); ++row) {
+      f4 acc[2];
+      conv_row(smem + (row * kConvPW + n) * LY::Pix + 16 * g, 64, kConvPW * LY::Pix, LY::Pix, A, acc);
+      unsigned char* d = smem + LY::OffR + (row * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
 #pragma unroll
-      for (int co = 0; co < 32; ++co) t[co] = fmaf(r[ci], wt[ci * 64 + h + co], t[co]);
+      for (int T = 0; T < 2; ++T) {
+        float r[4];
 #pragma unroll
-    for (int co = 0; co < 32; co += 4)
-      *reinterpret_cast<float4*>(out + h + co) = make_float4(t[co] + wt[4096 + h + co], t[co + 1] + wt[4097 + h + co],
-                                                             t[co + 2] + wt[4098 + h + co], t[co + 3] + wt[4099 + h + co]);
+        for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[T][i], inv, rb[T][i]), 0.1f) * sr;
+        u2 hi, lo;
+        split4(r[0], r[1], r[2], r[3], hi, lo);
+        *reinterpret_cast<u2*>(d + 32 * T) = hi;
+        *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
+      }
+    }
+    lds_barrier();
+    const float tinv = inverse_scale(er + ts.exponent);
+#pragma unroll 2
+    for (int row = 0; row < TH; ++row) {
+      const unsigned char* p = smem + LY::OffR + (row * kConvTW + n) * LY::RPix + 16 * g;
+      f4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const h8 bh = *reinterpret_cast<const h8*>(p + 64 * k), bl = *reinterpret_cast<const h8*>(p + 64 * k + 128);
+        acc = mfma_f16(At[k][0], bh, acc);
+        small = mfma_f16(At[k][0], bl, small);
+        small = mfma_f16(At[k][1], bh, small);
+      }
+      const int qy = y0 + row, qx = x0 + n;
+      if (qy < G.H && qx < G.W) {
+        f4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = fmaf(acc[i] + small[i], tinv, tb[i]);
+        *reinterpret_cast<f4*>(meta + (((size_t)b * G.H + qy) * G.W + qx) * 64 + 16 * wave + 4 * g) = o;
+      }
+    }
   }
 }
 
@@ -340,10 +517,31 @@ __global__ __launch_bounds__(kF32Threads) void f32_head_kernel(const Tin* __rest
 // ---- launchers ---------------------------------------------------------------------------------------
 static int f32_grid(long n) { return (int)((n + kF32Threads - 1) / kF32Threads); }
 
-hipError_t launch_f32_controller(int in_fp32, const void* src, const float* wimg, float* skip, float* low0, float* low1,
+template <int TH>
+static hipError_t launch_refine_t(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch, int cus,
+                                  hipStream_t stream) {
+  F32ConvTiles G{Hq, Wq, (Wq + kConvTW - 1) / kConvTW, (Hq + TH - 1) / TH, 0};
+  G.num = batch * G.tiles_x * G.tiles_y;
+  int grid = std::min(G.num, 2 * cus);
+  if (grid >= 8) grid -= grid % 8;
+  hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(grid), dim3(kConvThreads), RefineLayout<TH>::Lds, stream, work,
+                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32Refine + 18432, W.image + kF32Tail + 4096, meta,
+                     G, W.refine_scale, W.tail_scale);
+  return hipGetLastError();
+}
+static hipError_t launch_f32_refine_tail(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch,
+                                         int cus, hipStream_t stream) {
+  // tiles of 8 rows where they fill the 2 x cus resident blocks, else of 2 rows (more blocks, less work each)
+  const long tiles8 = (long)batch * ((Wq + kConvTW - 1) / kConvTW) * ((Hq + 7) / 8);
+  return tiles8 >= 2 * cus ? launch_refine_t<8>(work, W, meta, Hq, Wq, batch, cus, stream)
+                           : launch_refine_t<2>(work, W, meta, Hq, Wq, batch, cus, stream);
+}
+
+hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights& wts, float* skip, float* low0, float* low1,
                                  float* const* lows, float* work, float* meta, int H, int W, int Hq, int Wq, int py, int px,
-                                 int batch, hipStream_t stream, hipEvent_t* ev) {
+                                 int batch, int cus, hipStream_t stream, hipEvent_t* ev) {
   const int Hl = Hq / 2, Wl = Wq / 2;
+  const float* wimg = wts.image;
   const long packed = (long)batch * Hq * Wq, lowpx = (long)batch * Hl * Wl;
   if (in_fp32)
     hipLaunchKernelGGL(f32_project_kernel<float>, dim3(f32_grid(packed)), dim3(kF32Threads), 0, stream,
@@ -372,9 +570,7 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const float* wimg
                      (const float*)skip, wimg, work, Hl, Wl, batch);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[4], stream)) != hipSuccess) return e;
-  const int rtiles = batch * ((Hq + kF32GT - 1) / kF32GT) * ((Wq + kF32GT - 1) / kF32GT);
-  hipLaunchKernelGGL(f32_refine_tail_kernel, dim3(rtiles), dim3(kF32Threads), 0, stream, (const float*)work,
-                     wimg, meta, Hq, Wq, batch);
+  if ((e = launch_f32_refine_tail(work, wts, meta, Hq, Wq, batch, cus, stream)) != hipSuccess) return e;
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[5], stream)) != hipSuccess) return e;
   return hipSuccess;

@@ -124,12 +124,24 @@ constexpr int kF32Base = kF32Tail + 64 * 64 + 64;
 constexpr int kF32Basis = kF32Base + 25 * 4;
 constexpr int kF32Analysis = kF32Basis + 25 * 16 * 4;
 constexpr int kF32Floats = kF32Analysis + 24;
+// A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent, and an output's
+// magnitude is at most gain * (largest input magnitude) + offset.
+struct F32SplitScale {
+  int exponent;
+  float gain, offset;
+};
+// The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
+struct F32Weights {
+  const float* image;
+  const void *refine, *tail;               // [T][tap][part], [T][k][part]
+  F32SplitScale refine_scale, tail_scale;
+};
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong
 // between low0 and low1)
-hipError_t launch_f32_controller(int in_fp32, const void* src, const float* wimg, float* skip, float* low0, float* low1,
+hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights& wts, float* skip, float* low0, float* low1,
                                  float* const* lows, float* work, float* meta, int H, int W, int Hq, int Wq, int py, int px,
-                                 int batch, hipStream_t stream, hipEvent_t* ev);
+                                 int batch, int cus, hipStream_t stream, hipEvent_t* ev);
 hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const float* wimg, void* out,
                            int H, int W, int Hq, int Wq, int py, int px, int batch, unsigned* nonfinite,
                            hipStream_t stream);

@@ -1,0 +1,115 @@
+"""FP32 policy: every stage against the same stage in 64 bits on the GPU's own input, at the edges of the
+kernels' tiles and over FP32's range.
+
+The convolutions run as hi / lo FP16 splits on the MFMA (k_fp32.hip).  The bound of an output is
+2^-22 P sum |w||x| with P = 3 + 4 K / 8 at K products: each operand is held to 2^-22 (two operands and the
+dropped lo lo' product: 3), and the FP32 accumulators round once per 8 products, in three chains of which
+one is at the main sum's magnitude (2^-24 a rounding, taken as 2^-22 for terms that the MFMA cuts off when it
+aligns them).  FP32 FMA chains stay within it too.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.nn import functional as F
+
+from oracle import model as M
+from tests._util import WEIGHTS
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def R(gpu):
+    from aeisu_amd import runtime
+    return runtime
+
+
+@pytest.fixture(scope="module", params=["aeisu_area", "aeisu_div2k_l1"])
+def model(R, request):
+    return R.load_model(WEIGHTS / f"{request.param}.pt", precision="fp32"), M.load_folded(WEIGHTS / f"{request.param}.pt")
+
+
+def stages(model, frames):
+    """skip, low0..4, work, meta of a run that keeps them (NCHW, CPU)."""
+    from aeisu_amd import _lib as L
+    b, _, h, w = frames.shape
+    flags = L.FLAG_KEEP_INTERMEDIATES
+    hd = model.handle(b, h, w, torch.float32, torch.float32, flags)
+    model.run(frames.cuda().contiguous(), flags=flags, check_finite=False)
+    torch.cuda.synchronize()
+    _, _, _, _, hq, wq = model.geometry(hd)
+
+    def fetch(which, hh, ww, c):
+        t = model.intermediate(hd, which).cpu().view(torch.float32)
+        return t.reshape(b, hh, ww, c).permute(0, 3, 1, 2).contiguous()
+
+    return (fetch(L.BUF_SKIP, hq, wq, 32), [fetch(L.BUF_LOW0 + i, hq // 2, wq // 2, 64) for i in range(5)],
+            fetch(L.BUF_WORK, hq, wq, 32), fetch(L.BUF_META, hq, wq, 64))
+
+
+def conv64(x, state, name, slope=0.1):
+    """(LeakyReLU of the convolution in 64 bits, its error bound)."""
+    w, b = state[name + ".weight"].double(), state[name + ".bias"].double()
+    pad, k = w.shape[-1] // 2, w[0].numel()
+    y = F.conv2d(x.double(), w, b, padding=pad)
+    size = F.conv2d(x.double().abs(), w.abs(), b.abs(), padding=pad)
+    return torch.where(y >= 0, y, slope * y), 2.0 ** -22 * (3 + 4 * k / 8) * size
+
+
+def check(name, got, ref, bound):
+    over = (got.double() - ref).abs() - bound
+    assert torch.isfinite(got).all(), name
+    assert over.max().item() <= 0, f"{name}: {over.max().item():.3g} over the bound"
+
+
+def compare(model, state, frames):
+    skip, low, work, meta = stages(model, frames)
+    check("compress", low[0], *conv64(F.pixel_unshuffle(skip, 2), state, "compress_270"))
+    for i in range(1, 5):
+        for n, part in (("a", slice(0, 32)), ("b", slice(32, 64))):
+            check(f"bottleneck {i}{n}", low[i][:, part], *conv64(low[i - 1][:, part], state, f"bottleneck_270_{n}{i}"))
+    up, bound = conv64(low[4], state, "expand_270")
+    ref = skip.double() + F.pixel_shuffle(up, 2)
+    check("expand", work, ref, F.pixel_shuffle(bound, 2) + 2.0 ** -23 * ref.abs())
+    r, rb = conv64(work, state, "refine_540")
+    ref, tb = conv64(r, state, "metadata_head", slope=1.0)
+    through = F.conv2d(rb, state["metadata_head.weight"].double().abs())
+    check("refine + tail", meta, ref, tb + through)
+
+
+# one tile and less, ragged tiles, tile multiples, many frames (the large-launch variants), one long row
+SIZES = [(1, 1, 1), (1, 33, 65), (2, 96, 128), (1, 97, 31), (40, 70, 90), (3, 150, 1030)]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_stages_against_64_bits(model, size):
+    b, h, w = size
+    print(f"case: FP32 stages {size}", flush=True)
+    compare(*model, torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(h * w)))
+
+
+@pytest.mark.parametrize("gain", [0.0, 1e-30, 1e-6, 3e5, 1e12])
+def test_stages_over_the_range(model, gain):
+    """Frames far outside [0, 1]: the scaled splits neither overflow FP16 nor lose the small values."""
+    print(f"case: FP32 stages, frame values up to {gain:g}", flush=True)
+    frames = gain * (2 * torch.rand(1, 3, 45, 70, generator=torch.Generator().manual_seed(5)) - 1)
+    frames[:, :, :20] *= 1e-3                       # tiles that hold both
+    compare(*model, frames)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_nonfinite_input_stays_local(model, bad):
+    """A non-finite pixel makes its own surroundings non-finite and leaves pixels that it cannot reach (32 or
+    more away) at their values: it does not enter the scale of the tiles that it lies in."""
+    m, _ = model
+    print(f"case: FP32 frame with one pixel at {bad}", flush=True)
+    frames = torch.rand(1, 3, 80, 150, generator=torch.Generator().manual_seed(7))
+    clean = m.run(frames.cuda(), check_finite=False).cpu()
+    frames[0, 1, 40, 70] = bad
+    got = m.run(frames.cuda(), check_finite=False).cpu()
+    with pytest.raises(FloatingPointError):
+        m.run(frames.cuda())
+    far = torch.ones(160, 300, dtype=torch.bool)
+    far[2 * (40 - 32):2 * (40 + 33), 2 * (70 - 32):2 * (70 + 33)] = False
+    assert (got - clean).abs()[..., far].max().item() <= 2e-5
