@@ -314,8 +314,8 @@ struct ModeWeights {
   DeviceBuffer body_consts;        // epilogue constants of the fused body (kBodyConsts floats)
   DeviceBuffer fp32;               // FP32 policy: the whole weight image (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
-  DeviceBuffer f32_refine, f32_tail;
-  F32SplitScale f32_refine_scale{}, f32_tail_scale{};
+  DeviceBuffer f32_grouped[4], f32_refine, f32_tail;
+  F32SplitScale f32_grouped_scale[4] = {}, f32_refine_scale{}, f32_tail_scale{};
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -330,12 +330,17 @@ struct ModeWeights {
     fn(tail_bias);
     fn(body_consts);
     fn(fp32);
+    for (DeviceBuffer& b : f32_grouped) fn(b);
     fn(f32_refine);
     fn(f32_tail);
   }
   F32Weights f32_weights() const {
     F32Weights W;
     W.image = fp32.as<float>();
+    for (int l = 0; l < 4; ++l) {
+      W.grouped[l] = f32_grouped[l].ptr;
+      W.grouped_scale[l] = f32_grouped_scale[l];
+    }
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
     W.refine_scale = f32_refine_scale;
@@ -545,8 +550,10 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   layer("expand", 128, 64, 1, kF32Expand, 0.1f);
   layer("refine", 64, 32, 3, kF32Refine, 0.1f);
   layer("tail", 64, 64, 1, kF32Tail, 1.0f);
-  rt.f32_refine_scale = split("refine", 64, 32, 3, 36,
-                              [](int f, int m, int s) { return ((16 * (f / 9) + m) * 32 + s) * 9 + f % 9; }, rt.f32_refine);
+  auto conv3 = [](int f, int m, int s) { return ((16 * (f / 9) + m) * 32 + s) * 9 + f % 9; };
+  for (int l = 0; l < 4; ++l)
+    rt.f32_grouped_scale[l] = split("bottleneck" + std::to_string(l), 64, 32, 3, 36, conv3, rt.f32_grouped[l]);
+  rt.f32_refine_scale = split("refine", 64, 32, 3, 36, conv3, rt.f32_refine);
   rt.f32_tail_scale = split("tail", 64, 64, 1, 8,
                             [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; }, rt.f32_tail);
   for (int i = 0; i < 100; ++i) img[kF32Base + i] = base[i];

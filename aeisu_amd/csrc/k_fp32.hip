@@ -108,56 +108,6 @@ __global__ __launch_bounds__(kF32Threads) void f32_compress_kernel(const float* 
                     leaky01(acc[co + 2] + wc[8194 + co]), leaky01(acc[co + 3] + wc[8195 + co]));
 }
 
-// ---- grouped 3x3 (2 groups of 32 -> 32, zero padding) + LeakyReLU: a 16 x 16 tile of low pixels
-// per block (one pixel per thread) and one conv group (blockIdx.y), its 18 x 18 input halo staged in
-// LDS with coalesced loads (the group's 32 channels of a pixel, 36 floats apart: conflict-free
-// 16-byte reads), the weight rows block-uniform (scalar loads).  Read straight from memory, each
-// thread's 72 strided 16-byte loads made the layer 4x slower.
-constexpr int kF32GT = 16, kF32GH = kF32GT + 2, kF32GPix = 36;
-__global__ __launch_bounds__(kF32Threads) void f32_grouped_kernel(const float* __restrict__ in, const float* __restrict__ wl,
-                                                                  float* __restrict__ out, int Hl, int Wl, int batch) {
-  __shared__ __attribute__((aligned(16))) float tile[kF32GH * kF32GH * kF32GPix];
-  const int tx_n = (Wl + kF32GT - 1) / kF32GT, ty_n = (Hl + kF32GT - 1) / kF32GT;
-  const int b = (int)blockIdx.x / (tx_n * ty_n), rem = (int)blockIdx.x - b * tx_n * ty_n;
-  const int y0 = (rem / tx_n) * kF32GT, x0 = (rem % tx_n) * kF32GT;
-  const int grp = blockIdx.y, tid = threadIdx.x;
-  // stage: 18 x 18 pixels x 8 float4 (the group's 32 channels), zero outside the low grid
-  for (int i = tid; i < kF32GH * kF32GH * 8; i += kF32Threads) {
-    const int pix = i >> 3, q = i & 7, py = pix / kF32GH, px = pix - py * kF32GH;
-    const int y = y0 + py - 1, x = x0 + px - 1;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (y >= 0 && y < Hl && x >= 0 && x < Wl)
-      v = *reinterpret_cast<const float4*>(in + (((size_t)b * Hl + y) * Wl + x) * 64 + 32 * grp + 4 * q);
-    *reinterpret_cast<float4*>(&tile[pix * kF32GPix + 4 * q]) = v;
-  }
-  __syncthreads();
-  const int ty = tid / kF32GT, tx = tid - ty * kF32GT;
-  float acc[32];
-#pragma unroll
-  for (int o = 0; o < 32; ++o) acc[o] = 0.f;
-  for (int tap = 0; tap < 9; ++tap) {
-    const float* src = &tile[((ty + tap / 3) * kF32GH + tx + tap % 3) * kF32GPix];
-    for (int c0 = 0; c0 < 32; c0 += 4) {
-      const float4 x4 = *reinterpret_cast<const float4*>(src + c0);
-      const float xs[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float* wr = wl + (tap * 32 + c0 + e) * 64 + 32 * grp;
-#pragma unroll
-        for (int o = 0; o < 32; ++o) acc[o] = fmaf(xs[e], wr[o], acc[o]);
-      }
-    }
-  }
-  const int ly = y0 + ty, lx = x0 + tx;
-  if (ly >= Hl || lx >= Wl) return;
-  float* dst = out + (((size_t)b * Hl + ly) * Wl + lx) * 64 + 32 * grp;
-#pragma unroll
-  for (int o = 0; o < 32; o += 4)
-    *reinterpret_cast<float4*>(dst + o) = make_float4(
-        leaky01(acc[o] + wl[18432 + 32 * grp + o]), leaky01(acc[o + 1] + wl[18433 + 32 * grp + o]),
-        leaky01(acc[o + 2] + wl[18434 + 32 * grp + o]), leaky01(acc[o + 3] + wl[18435 + 32 * grp + o]));
-}
-
 // ---- expand 1x1 (64 -> 128) + LeakyReLU, pixel_shuffle, + skip: one low pixel per thread ----------
 // Expand output channel c * 4 + 2i + j goes to channel c of packed pixel (2ly + i, 2lx + j).
 __global__ __launch_bounds__(kF32Threads) void f32_expand_kernel(const float* __restrict__ low, const float* __restrict__ skip,
@@ -246,12 +196,12 @@ __device__ __forceinline__ float wave_max(float m) {
 }
 
 // ---- 3x3 layers: persistent blocks of four waves over tiles of 16 x TH pixels -----------------------
-// Wave w serves output channels 32 (w & 1) .. + 31 (two MFMA row tiles) of the pixel rows of its half
-// (w >> 1), and keeps its 36 weight fragments (9 taps x 2 tiles x hi, lo: 144 VGPRs) for the launch: from
-// LDS or L2 the fragments would be read once per pixel row and more often than the activations.  The tile's
+// A wave serves 32 output channels (two MFMA row tiles) of some of the tile's pixel rows and keeps their 36
+// weight fragments (9 taps x 2 tiles x hi, lo: 144 VGPRs) for the launch: from LDS or L2 the fragments would be read once per pixel row and more often than the activations.  The tile's
 // input halo is staged in LDS as hi and lo halves, split once per value.  Two blocks per CU (two waves per
 // SIMD at 256 VGPRs): one block's staging and barriers overlap the other's products.
 constexpr int kConvTW = 16, kConvPW = kConvTW + 2;
+constexpr int kConvPix = 144;                        // LDS bytes per halo pixel: 32 channels hi, lo, pad
 constexpr int kConvThreads = 256;
 
 __device__ __forceinline__ void conv_weights(h8 (&A)[9][2][2], const h8* __restrict__ frag, int role, int lane) {
@@ -264,15 +214,14 @@ __device__ __forceinline__ void conv_weights(h8 (&A)[9][2][2], const h8* __restr
 }
 
 // One row of 16 pixels: acc[T] = sum over the 9 taps of the wave's two row tiles.  p: the lane's operand of
-// the top left tap (hi; lo is `lo` bytes further), rows `row` bytes apart, pixels `pix`.
-__device__ __forceinline__ void conv_row(const unsigned char* p, int lo, int row, int pix, const h8 (&A)[9][2][2],
-                                         f4 (&acc)[2]) {
+// the top left tap.
+__device__ __forceinline__ void conv_row(const unsigned char* p, const h8 (&A)[9][2][2], f4 (&acc)[2]) {
   f4 small[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
   acc[0] = acc[1] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int tap = 0; tap < 9; ++tap) {
-    const unsigned char* q = p + (tap / 3) * row + (tap % 3) * pix;
-    const h8 bh = *reinterpret_cast<const h8*>(q), bl = *reinterpret_cast<const h8*>(q + lo);
+    const unsigned char* q = p + ((tap / 3) * kConvPW + tap % 3) * kConvPix;
+    const h8 bh = *reinterpret_cast<const h8*>(q), bl = *reinterpret_cast<const h8*>(q + 64);
 #pragma unroll
     for (int T = 0; T < 2; ++T) acc[T] = mfma_f16(A[tap][T][0], bh, acc[T]);
 #pragma unroll
@@ -295,16 +244,17 @@ __device__ __forceinline__ float block_max(float m, float* red, int wave, int la
 }
 
 template <int TH>
-struct RefineLayout {
-  static constexpr int Rows = TH + 2, Pix = 144, Chunks = Rows * kConvPW * 8;   // float4 chunks of the halo
+struct ConvLayout {
+  static constexpr int Rows = TH + 2, Chunks = Rows * kConvPW * 8;   // float4 chunks of the halo
   static constexpr int Per = (Chunks + kConvThreads - 1) / kConvThreads;
+  static constexpr int SizeHalo = Rows * kConvPW * kConvPix;
   static constexpr int RPix = 272;                   // refine outputs: 64 channels hi, 64 lo, pad
-  static constexpr int OffR = Rows * kConvPW * Pix, OffRed = OffR + TH * kConvTW * RPix;
-  static constexpr int Lds = OffRed + 16;
+  static constexpr int LdsRefine = SizeHalo + TH * kConvTW * RPix;
 };
 struct F32ConvTiles {
   int H, W, tiles_x, tiles_y, num;
 };
+// The tile's halo, 32 of the CH channels of a pixel (in: the first of them), zero outside the grid.
 template <int PER, int CH>
 __device__ __forceinline__ void conv_fetch(float4 (&v)[PER], const float* __restrict__ in, const F32ConvTiles& G, int tidx,
                                            int th, int chunks, int tid) {
@@ -313,7 +263,7 @@ __device__ __forceinline__ void conv_fetch(float4 (&v)[PER], const float* __rest
   const float* f = in + (size_t)b * G.H * G.W * CH;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int i = tid + k * kConvThreads, pix = i / (CH / 4), c = i % (CH / 4);
+    const int i = tid + k * kConvThreads, pix = i >> 3, c = i & 7;
     const int py = pix / kConvPW, y = y0 + py, x = x0 + pix - py * kConvPW;
     const bool in_grid = (unsigned)y < (unsigned)G.H && (unsigned)x < (unsigned)G.W && i < chunks;
     v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -333,19 +283,67 @@ __device__ __forceinline__ float chunk_max(const float4 (&v)[PER]) {
   }
   return m;
 }
-// Splits the staged chunks into LDS: pixel stride `pix`, hi halves of the CH channels first, lo halves after.
-template <int PER, int CH>
-__device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char* lds, int pix_bytes, float s, int chunks,
-                                           int tid) {
+// Splits the staged chunks into LDS: hi halves of a pixel's 32 channels first, lo halves after.
+template <int PER>
+__device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char* lds, float s, int chunks, int tid) {
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int i = tid + k * kConvThreads, pix = i / (CH / 4), c = i % (CH / 4);
+    const int i = tid + k * kConvThreads, pix = i >> 3, c = i & 7;
     if (i < chunks) {
       u2 hi, lo;
       split4(v[k].x * s, v[k].y * s, v[k].z * s, v[k].w * s, hi, lo);
-      unsigned char* d = lds + pix * pix_bytes + 8 * c;
+      unsigned char* d = lds + pix * kConvPix + 8 * c;
       *reinterpret_cast<u2*>(d) = hi;
-      *reinterpret_cast<u2*>(d + 2 * CH) = lo;
+      *reinterpret_cast<u2*>(d + 64) = lo;
+    }
+  }
+}
+
+// A grouped 3x3 layer (2 groups of 32 -> 32, zero padding) + LeakyReLU: blockIdx.y is the conv group, so the
+// block's waves share its weights and split the tile's rows.  One thread per pixel and group with FP32 FMAs:
+// 147 us at 1080p, 50 us for 256 x 256.
+template <int TH>
+__global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const float* __restrict__ in, const h8* __restrict__ frag,
+                                                                      const float* __restrict__ bias, float* __restrict__ out,
+                                                                      F32ConvTiles G, F32SplitScale sc) {
+  typedef ConvLayout<TH> LY;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[LY::SizeHalo];
+  __shared__ __attribute__((aligned(16))) float red[4];
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, grp = blockIdx.y;
+  const int n = lane & 15, g = lane >> 4;
+  float4 v[LY::Per];
+  int tidx = tile_of(0, G.num);
+  if (tidx < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, tidx, TH, LY::Chunks, tid);
+  h8 A[9][2][2];
+  conv_weights(A, frag, grp, lane);
+  f4 bs[2];
+#pragma unroll
+  for (int T = 0; T < 2; ++T) bs[T] = *reinterpret_cast<const f4*>(bias + 32 * grp + 16 * T + 4 * g);
+  const int iters = tile_iters(G.num);
+  for (int it = 0; it < iters; ++it) {
+    if (tidx >= G.num) break;                        // block-uniform
+    const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per;
+    const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
+    const int ex = scale_exponent(block_max(chunk_max(v), red, wave, lane));
+    conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
+    tidx = tile_of(it + 1, G.num);
+    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, tidx, TH, LY::Chunks, fresh(tid));
+    lds_barrier();
+    const float inv = inverse_scale(ex + sc.exponent);
+    for (int row = wave; row < TH; row += 4) {
+      f4 acc[2];
+      conv_row(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
+      const int y = y0 + row, x = x0 + n;
+      if (y < G.H && x < G.W) {
+        float* d = out + (((size_t)b * G.H + y) * G.W + x) * 64 + 32 * grp + 4 * g;
+#pragma unroll
+        for (int T = 0; T < 2; ++T) {
+          f4 r;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[T][i], inv, bs[T][i]), 0.1f);
+          *reinterpret_cast<f4*>(d + 16 * T) = r;
+        }
+      }
     }
   }
 }
@@ -355,7 +353,7 @@ __device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char
 // of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (416 KB per tile), which
 // two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
 // (scaled by a bound of their magnitude from the tile's input maximum and the weights) and wave w computes
-// tail channels 16 w .. + 15 from them.
+// tail channels 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
 template <int TH>
 __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const float* __restrict__ work,
                                                                           const h8* __restrict__ rfrag,
@@ -364,20 +362,16 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
                                                                           const float* __restrict__ tbias,
                                                                           float* __restrict__ meta, F32ConvTiles G,
                                                                           F32SplitScale rs, F32SplitScale ts) {
-  typedef RefineLayout<TH> LY;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  float* red = reinterpret_cast<float*>(smem + LY::OffRed);
+  typedef ConvLayout<TH> LY;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[LY::LdsRefine];
+  __shared__ __attribute__((aligned(16))) float red[4];
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, role = wave & 1, half = wave >> 1;
   const int n = lane & 15, g = lane >> 4;
   float4 v[LY::Per];
   int tidx = tile_of(0, G.num);
   if (tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
-  h8 A[9][2][2], At[2][2];
+  h8 A[9][2][2];
   conv_weights(A, rfrag, role, lane);
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int part = 0; part < 2; ++part) At[k][part] = tfrag[((wave * 2 + k) * 2 + part) * 64 + lane];
   f4 rb[2];
 #pragma unroll
   for (int T = 0; T < 2; ++T) rb[T] = *reinterpret_cast<const f4*>(rbias + 32 * role + 16 * T + 4 * g);
@@ -389,17 +383,17 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
     const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
     const float m = block_max(chunk_max(v), red, wave, lane);
     const int ex = scale_exponent(m);
-    conv_stage<LY::Per, 32>(v, smem, LY::Pix, pow2f(ex), LY::Chunks, tid);
+    conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
     tidx = tile_of(it + 1, G.num);
-    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
+    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, fresh(tid));
     lds_barrier();
     // |refine output| <= gain m + offset
     const int er = scale_exponent(fminf(fmaf(rs.gain, m, rs.offset), 0x1p126f));
     const float inv = inverse_scale(ex + rs.exponent), sr = pow2f(er);
     for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); ++row) {
       f4 acc[2];
-      conv_row(smem + (row * kConvPW + n) * LY::Pix + 16 * g, 64, kConvPW * LY::Pix, LY::Pix, A, acc);
-      unsigned char* d = smem + LY::OffR + (row * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
+      conv_row(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
+      unsigned char* d = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
 #pragma unroll
       for (int T = 0; T < 2; ++T) {
         float r[4];
@@ -411,11 +405,18 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
         *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
       }
     }
+    // the tail fragments are read for every tile: kept, they do not fit the 256 VGPRs
+    h8 At[2][2];
+    const h8* tf = tfrag + wave * 4 * 64 + fresh(lane);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int part = 0; part < 2; ++part) At[k][part] = tf[(k * 2 + part) * 64];
     lds_barrier();
     const float tinv = inverse_scale(er + ts.exponent);
 #pragma unroll 2
     for (int row = 0; row < TH; ++row) {
-      const unsigned char* p = smem + LY::OffR + (row * kConvTW + n) * LY::RPix + 16 * g;
+      const unsigned char* p = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix + 16 * g;
       f4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
@@ -517,14 +518,36 @@ __global__ __launch_bounds__(kF32Threads) void f32_head_kernel(const Tin* __rest
 // ---- launchers ---------------------------------------------------------------------------------------
 static int f32_grid(long n) { return (int)((n + kF32Threads - 1) / kF32Threads); }
 
+static F32ConvTiles conv_tiles(int H, int W, int th, int batch) {
+  F32ConvTiles G{H, W, (W + kConvTW - 1) / kConvTW, (H + th - 1) / th, 0};
+  G.num = batch * G.tiles_x * G.tiles_y;
+  return G;
+}
+// Persistent blocks for `tiles` tiles with `most` resident at once, a multiple of 8 (the XCDs) where possible.
+static int conv_grid(int tiles, int most) {
+  const int g = std::min(tiles, most);
+  return g >= 8 ? g - g % 8 : g;
+}
+template <int TH>
+static hipError_t launch_grouped_t(const float* in, const F32Weights& W, int l, float* out, int Hl, int Wl, int batch, int cus,
+                                   hipStream_t stream) {
+  const F32ConvTiles G = conv_tiles(Hl, Wl, TH, batch);
+  hipLaunchKernelGGL(f32_grouped_kernel<TH>, dim3(conv_grid(G.num, cus), 2), dim3(kConvThreads), 0, stream, in,
+                     (const h8*)W.grouped[l], W.image + kF32Grouped + l * kF32GroupedStride + 18432, out, G,
+                     W.grouped_scale[l]);
+  return hipGetLastError();
+}
+static hipError_t launch_f32_grouped(const float* in, const F32Weights& W, int l, float* out, int Hl, int Wl, int batch,
+                                     int cus, hipStream_t stream) {
+  // tiles of 8 rows where they fill the resident blocks (cus per conv group), else of 4 (one row per wave)
+  return conv_tiles(Hl, Wl, 8, batch).num >= cus ? launch_grouped_t<8>(in, W, l, out, Hl, Wl, batch, cus, stream)
+                                                 : launch_grouped_t<4>(in, W, l, out, Hl, Wl, batch, cus, stream);
+}
 template <int TH>
 static hipError_t launch_refine_t(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch, int cus,
                                   hipStream_t stream) {
-  F32ConvTiles G{Hq, Wq, (Wq + kConvTW - 1) / kConvTW, (Hq + TH - 1) / TH, 0};
-  G.num = batch * G.tiles_x * G.tiles_y;
-  int grid = std::min(G.num, 2 * cus);
-  if (grid >= 8) grid -= grid % 8;
-  hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(grid), dim3(kConvThreads), RefineLayout<TH>::Lds, stream, work,
+  const F32ConvTiles G = conv_tiles(Hq, Wq, TH, batch);
+  hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(conv_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
                      (const h8*)W.refine, (const h8*)W.tail, W.image + kF32Refine + 18432, W.image + kF32Tail + 4096, meta,
                      G, W.refine_scale, W.tail_scale);
   return hipGetLastError();
@@ -532,9 +555,8 @@ static hipError_t launch_refine_t(const float* work, const F32Weights& W, float*
 static hipError_t launch_f32_refine_tail(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch,
                                          int cus, hipStream_t stream) {
   // tiles of 8 rows where they fill the 2 x cus resident blocks, else of 2 rows (more blocks, less work each)
-  const long tiles8 = (long)batch * ((Wq + kConvTW - 1) / kConvTW) * ((Hq + 7) / 8);
-  return tiles8 >= 2 * cus ? launch_refine_t<8>(work, W, meta, Hq, Wq, batch, cus, stream)
-                           : launch_refine_t<2>(work, W, meta, Hq, Wq, batch, cus, stream);
+  return conv_tiles(Hq, Wq, 8, batch).num >= 2 * cus ? launch_refine_t<8>(work, W, meta, Hq, Wq, batch, cus, stream)
+                                                     : launch_refine_t<2>(work, W, meta, Hq, Wq, batch, cus, stream);
 }
 
 hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights& wts, float* skip, float* low0, float* low1,
@@ -559,12 +581,8 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
                      dst[0], Hl, Wl, batch);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[2], stream)) != hipSuccess) return e;
-  for (int l = 0; l < 4; ++l) {
-    const int gtiles = batch * ((Hl + kF32GT - 1) / kF32GT) * ((Wl + kF32GT - 1) / kF32GT);
-    hipLaunchKernelGGL(f32_grouped_kernel, dim3(gtiles, 2), dim3(kF32Threads), 0, stream, (const float*)dst[l],
-                       wimg + kF32Grouped + l * kF32GroupedStride, dst[l + 1], Hl, Wl, batch);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  for (int l = 0; l < 4; ++l)
+    if ((e = launch_f32_grouped(dst[l], wts, l, dst[l + 1], Hl, Wl, batch, cus, stream)) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[3], stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(f32_expand_kernel, dim3(f32_grid(lowpx)), dim3(kF32Threads), 0, stream, (const float*)dst[4],
                      (const float*)skip, wimg, work, Hl, Wl, batch);

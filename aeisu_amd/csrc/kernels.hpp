@@ -133,8 +133,8 @@ struct F32SplitScale {
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
   const float* image;
-  const void *refine, *tail;               // [T][tap][part], [T][k][part]
-  F32SplitScale refine_scale, tail_scale;
+  const void *grouped[4], *refine, *tail;  // [T][tap][part] (T = 2 group + t), [T][k][part] for the tail
+  F32SplitScale grouped_scale[4], refine_scale, tail_scale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong
