@@ -314,8 +314,8 @@ struct ModeWeights {
   DeviceBuffer body_consts;        // epilogue constants of the fused body (kBodyConsts floats)
   DeviceBuffer fp32;               // FP32 policy: the whole weight image (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
-  DeviceBuffer f32_grouped[4], f32_refine, f32_tail;
-  F32SplitScale f32_grouped_scale[4] = {}, f32_refine_scale{}, f32_tail_scale{};
+  DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail;
+  F32SplitScale f32_compress_scale{}, f32_grouped_scale[4] = {}, f32_expand_scale{}, f32_refine_scale{}, f32_tail_scale{};
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -330,7 +330,9 @@ struct ModeWeights {
     fn(tail_bias);
     fn(body_consts);
     fn(fp32);
+    fn(f32_compress);
     for (DeviceBuffer& b : f32_grouped) fn(b);
+    fn(f32_expand);
     fn(f32_refine);
     fn(f32_tail);
   }
@@ -341,6 +343,10 @@ struct ModeWeights {
       W.grouped[l] = f32_grouped[l].ptr;
       W.grouped_scale[l] = f32_grouped_scale[l];
     }
+    W.compress = f32_compress.ptr;
+    W.compress_scale = f32_compress_scale;
+    W.expand = f32_expand.ptr;
+    W.expand_scale = f32_expand_scale;
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
     W.refine_scale = f32_refine_scale;
@@ -550,6 +556,12 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   layer("expand", 128, 64, 1, kF32Expand, 0.1f);
   layer("refine", 64, 32, 3, kF32Refine, 0.1f);
   layer("tail", 64, 64, 1, kF32Tail, 1.0f);
+  rt.f32_compress_scale = split("compress", 64, 128, 1, 16,
+                                [](int f, int m, int s) { return (16 * (f / 4) + m) * 128 + s * 4 + f % 4; }, rt.f32_compress);
+  rt.f32_expand_scale = split("expand", 128, 64, 1, 16, [](int f, int m, int s) {
+    const int T = f / 2;
+    return ((16 * (T >> 2) + m) * 4 + (T & 3)) * 64 + 32 * (f % 2) + s;
+  }, rt.f32_expand);
   auto conv3 = [](int f, int m, int s) { return ((16 * (f / 9) + m) * 32 + s) * 9 + f % 9; };
   for (int l = 0; l < 4; ++l)
     rt.f32_grouped_scale[l] = split("bottleneck" + std::to_string(l), 64, 32, 3, 36, conv3, rt.f32_grouped[l]);

@@ -74,84 +74,6 @@ __global__ __launch_bounds__(kF32Threads) void f32_project_kernel(const Tin* __r
                                                        leaky01(acc[co + 2] + wp[1026 + co]), leaky01(acc[co + 3] + wp[1027 + co]));
 }
 
-// ---- pixel_unshuffle + compress 1x1 (128 -> 64) + LeakyReLU: one low pixel per thread ---------------
-__global__ __launch_bounds__(kF32Threads) void f32_compress_kernel(const float* __restrict__ skip, const float* __restrict__ wimg,
-                                                                   float* __restrict__ low, int Hl, int Wl, int batch) {
-  const long idx = (long)blockIdx.x * kF32Threads + threadIdx.x;
-  if (idx >= (long)batch * Hl * Wl) return;
-  const int b = (int)(idx / ((long)Hl * Wl));
-  const int rem = (int)(idx - (long)b * Hl * Wl);
-  const int ly = rem / Wl, lx = rem - ly * Wl;
-  const int Hq = 2 * Hl, Wq = 2 * Wl;
-  const float* wc = wimg + kF32Compress;
-  float acc[64];
-#pragma unroll
-  for (int co = 0; co < 64; ++co) acc[co] = 0.f;
-  for (int ph = 0; ph < 4; ++ph) {                 // unshuffled input channel = skip channel * 4 + phase
-    const float* in = skip + (((size_t)b * Hq + 2 * ly + (ph >> 1)) * Wq + 2 * lx + (ph & 1)) * 32;
-    for (int c0 = 0; c0 < 32; c0 += 4) {
-      const float4 x4 = *reinterpret_cast<const float4*>(in + c0);
-      const float xs[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float* wr = wc + ((c0 + e) * 4 + ph) * 64;
-#pragma unroll
-        for (int co = 0; co < 64; ++co) acc[co] = fmaf(xs[e], wr[co], acc[co]);
-      }
-    }
-  }
-  float* out = low + (size_t)idx * 64;
-#pragma unroll
-  for (int co = 0; co < 64; co += 4)
-    *reinterpret_cast<float4*>(out + co) =
-        make_float4(leaky01(acc[co] + wc[8192 + co]), leaky01(acc[co + 1] + wc[8193 + co]),
-                    leaky01(acc[co + 2] + wc[8194 + co]), leaky01(acc[co + 3] + wc[8195 + co]));
-}
-
-// ---- expand 1x1 (64 -> 128) + LeakyReLU, pixel_shuffle, + skip: one low pixel per thread ----------
-// Expand output channel c * 4 + 2i + j goes to channel c of packed pixel (2ly + i, 2lx + j).
-__global__ __launch_bounds__(kF32Threads) void f32_expand_kernel(const float* __restrict__ low, const float* __restrict__ skip,
-                                                                 const float* __restrict__ wimg, float* __restrict__ work,
-                                                                 int Hl, int Wl, int batch) {
-  const long idx = (long)blockIdx.x * kF32Threads + threadIdx.x;
-  if (idx >= (long)batch * Hl * Wl) return;
-  const int b = (int)(idx / ((long)Hl * Wl));
-  const int rem = (int)(idx - (long)b * Hl * Wl);
-  const int ly = rem / Wl, lx = rem - ly * Wl;
-  const int Hq = 2 * Hl, Wq = 2 * Wl;
-  const float* we = wimg + kF32Expand;
-  const float* in = low + (size_t)idx * 64;
-  for (int half = 0; half < 2; ++half) {           // output channels 64 half .. 64 half + 63
-    float acc[64];
-#pragma unroll
-    for (int co = 0; co < 64; ++co) acc[co] = 0.f;
-    for (int c0 = 0; c0 < 64; c0 += 4) {
-      const float4 x4 = *reinterpret_cast<const float4*>(in + c0);
-      const float xs[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float* wr = we + (c0 + e) * 128 + 64 * half;
-#pragma unroll
-        for (int co = 0; co < 64; ++co) acc[co] = fmaf(xs[e], wr[co], acc[co]);
-      }
-    }
-#pragma unroll
-    for (int ph = 0; ph < 4; ++ph) {
-      const size_t o = (((size_t)b * Hq + 2 * ly + (ph >> 1)) * Wq + 2 * lx + (ph & 1)) * 32 + 16 * half;
-#pragma unroll
-      for (int c = 0; c < 16; c += 4) {
-        const float4 sk = *reinterpret_cast<const float4*>(skip + o + c);
-        const int e0 = 4 * c + ph;                 // acc index of output channel (16 half + c) * 4 + ph
-        *reinterpret_cast<float4*>(work + o + c) =
-            make_float4(leaky01(acc[e0] + we[8192 + 64 * half + e0]) + sk.x,
-                        leaky01(acc[e0 + 4] + we[8192 + 64 * half + e0 + 4]) + sk.y,
-                        leaky01(acc[e0 + 8] + we[8192 + 64 * half + e0 + 8]) + sk.z,
-                        leaky01(acc[e0 + 12] + we[8192 + 64 * half + e0 + 12]) + sk.w);
-      }
-    }
-  }
-}
-
 // ---- split products on the FP16 MFMA ----------------------------------------------------------------
 // An FP32 operand x is scaled by a power of two and written as hi + lo, hi = fp16(x), lo = fp16(x - hi),
 // and a product is hi hi' + (hi lo' + lo hi'): three FP16 MFMAs in place of the FP32 FMAs, at 5 times the
@@ -436,6 +358,154 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
   }
 }
 
+// ---- 1x1 layers of the low grid ---------------------------------------------------------------------
+// A wave takes 16 low pixels at a time: a lane reads the 8 channels of its MFMA K slots straight from memory
+// (32 contiguous bytes), splits them in registers, and the pixel's scale comes from the four lanes that hold
+// its channels.  All 32 weight fragments stay in registers (128 VGPRs).  The next group's loads are in flight
+// during the products.
+__device__ __forceinline__ float pixel_max(float m) {    // over the lanes n, n + 16, n + 32, n + 48
+  m = fmaxf(m, __shfl_xor(m, 16));
+  return fmaxf(m, __shfl_xor(m, 32));
+}
+__device__ __forceinline__ void split8(float4 a, float4 b, float s, h8& hi, h8& lo) {
+  u2 h0, l0, h1, l1;
+  split4(a.x * s, a.y * s, a.z * s, a.w * s, h0, l0);
+  split4(b.x * s, b.y * s, b.z * s, b.w * s, h1, l1);
+  hi = __builtin_bit_cast(h8, u4{h0[0], h0[1], h1[0], h1[1]});
+  lo = __builtin_bit_cast(h8, u4{l0[0], l0[1], l1[0], l1[1]});
+}
+struct LowPixel {
+  int b, y, x;
+};
+__device__ __forceinline__ LowPixel low_pixel(int idx, int Hl, int Wl) {
+  const int per = Hl * Wl, b = idx / per, rem = idx - b * per, y = rem / Wl;
+  return {b, y, rem - y * Wl};
+}
+
+// pixel_unshuffle + compress 1x1 (128 -> 64) + LeakyReLU: K chunk k is phase k's 32 skip channels.  At 1080p
+// 103 us with one thread per pixel and FP32 FMAs.
+__global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const float* __restrict__ skip,
+                                                                      const h8* __restrict__ frag,
+                                                                      const float* __restrict__ bias,
+                                                                      float* __restrict__ low, int Hl, int Wl, int pixels,
+                                                                      F32SplitScale sc) {
+  const int lane = lane_id(), n = lane & 15, g = lane >> 4, waves = gridDim.x * (kF32Threads / 64);
+  const int groups = (pixels + 15) >> 4;
+  int grp = blockIdx.x * (kF32Threads / 64) + (threadIdx.x >> 6);
+  auto fetch = [&](int gi, float4 (&v)[8]) {
+    const LowPixel p = low_pixel(min(gi * 16 + n, pixels - 1), Hl, Wl);
+    const float* s = skip + (((size_t)p.b * 2 * Hl + 2 * p.y) * 2 * Wl + 2 * p.x) * 32 + 8 * g;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float* q = s + (size_t)(k >> 1) * 2 * Wl * 32 + (k & 1) * 32;
+      v[2 * k] = *reinterpret_cast<const float4*>(q);
+      v[2 * k + 1] = *reinterpret_cast<const float4*>(q + 4);
+    }
+  };
+  float4 v[8];
+  if (grp < groups) fetch(grp, v);
+  h8 A[4][4][2];
+  f4 bs[4];
+#pragma unroll
+  for (int T = 0; T < 4; ++T) {
+    bs[T] = *reinterpret_cast<const f4*>(bias + 16 * T + 4 * g);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int part = 0; part < 2; ++part) A[T][k][part] = frag[((T * 4 + k) * 2 + part) * 64 + lane];
+  }
+  for (; grp < groups; grp += waves) {
+    const int ex = scale_exponent(pixel_max(chunk_max(v)));
+    const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
+    h8 bh[4], bl[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) split8(v[2 * k], v[2 * k + 1], s, bh[k], bl[k]);
+    if (grp + waves < groups) fetch(grp + waves, v);
+    const int idx = grp * 16 + n;
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+      f4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc = mfma_f16(A[T][k][0], bh[k], acc);
+        small = mfma_f16(A[T][k][0], bl[k], small);
+        small = mfma_f16(A[T][k][1], bh[k], small);
+      }
+      f4 r;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[i] + small[i], inv, bs[T][i]), 0.1f);
+      if (idx < pixels) *reinterpret_cast<f4*>(low + (size_t)idx * 64 + 16 * T + 4 * g) = r;
+    }
+  }
+}
+
+// expand 1x1 (64 -> 128) + LeakyReLU, pixel_shuffle, + skip: row tile T holds channels 16 (T >> 2) .. + 15 of
+// phase T & 3 (expand output channel c * 4 + 2i + j goes to channel c of packed pixel (2ly + i, 2lx + j)).  At
+// 1080p 118 us with one thread per pixel and FP32 FMAs.
+__global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float* __restrict__ low,
+                                                                    const float* __restrict__ skip,
+                                                                    const h8* __restrict__ frag,
+                                                                    const float* __restrict__ bias,
+                                                                    float* __restrict__ work, int Hl, int Wl, int pixels,
+                                                                    F32SplitScale sc) {
+  const int lane = lane_id(), n = lane & 15, g = lane >> 4, waves = gridDim.x * (kF32Threads / 64);
+  const int groups = (pixels + 15) >> 4;
+  int grp = blockIdx.x * (kF32Threads / 64) + (threadIdx.x >> 6);
+  auto fetch = [&](int gi, float4 (&v)[4]) {
+    const float* s = low + (size_t)min(gi * 16 + n, pixels - 1) * 64 + 8 * g;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      v[2 * k] = *reinterpret_cast<const float4*>(s + 32 * k);
+      v[2 * k + 1] = *reinterpret_cast<const float4*>(s + 32 * k + 4);
+    }
+  };
+  float4 v[4];
+  if (grp < groups) fetch(grp, v);
+  __shared__ __attribute__((aligned(16))) float sb[128];   // bias by row tile and row
+  if (threadIdx.x < 128) {
+    const int T = threadIdx.x >> 4, m = threadIdx.x & 15;
+    sb[threadIdx.x] = bias[(16 * (T >> 2) + m) * 4 + (T & 3)];
+  }
+  lds_barrier();
+  h8 A[8][2][2];
+#pragma unroll
+  for (int T = 0; T < 8; ++T)
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int part = 0; part < 2; ++part) A[T][k][part] = frag[((T * 2 + k) * 2 + part) * 64 + lane];
+  for (; grp < groups; grp += waves) {
+    const int idx = grp * 16 + n;
+    const LowPixel p = low_pixel(min(idx, pixels - 1), Hl, Wl);
+    const size_t o = (((size_t)p.b * 2 * Hl + 2 * p.y) * 2 * Wl + 2 * p.x) * 32 + 4 * g;
+    auto at = [&](int T) { return o + (size_t)((T & 3) >> 1) * 2 * Wl * 32 + (T & 1) * 32 + 16 * (T >> 2); };
+    f4 sk[8];
+#pragma unroll
+    for (int T = 0; T < 8; ++T) sk[T] = *reinterpret_cast<const f4*>(skip + at(T));
+    const int ex = scale_exponent(pixel_max(chunk_max(v)));
+    const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
+    h8 bh[2], bl[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) split8(v[2 * k], v[2 * k + 1], s, bh[k], bl[k]);
+    if (grp + waves < groups) fetch(grp + waves, v);
+#pragma unroll
+    for (int T = 0; T < 8; ++T) {
+      f4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        acc = mfma_f16(A[T][k][0], bh[k], acc);
+        small = mfma_f16(A[T][k][0], bl[k], small);
+        small = mfma_f16(A[T][k][1], bh[k], small);
+      }
+      const f4 bs = *reinterpret_cast<const f4*>(sb + 16 * T + 4 * g);
+      f4 r;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[i] + small[i], inv, bs[i]), 0.1f) + sk[T][i];
+      if (idx < pixels) *reinterpret_cast<f4*>(work + at(T)) = r;
+    }
+  }
+}
+
 // ---- head: clamp, polyphase filter synthesis, 5x5 application, clip: one LR pixel per thread -------
 // coefficient_clamp (aeisu/reconstruction.py:15-17) in FP32 with the reference's separate multiply
 // and add; a NaN coefficient stays NaN (so does the output, which raises the non-finite flag).
@@ -577,15 +647,17 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
   // layer outputs: lows[i] when every layer is kept, else ping-pong between low0 and low1
   float* dst[5];
   for (int i = 0; i < 5; ++i) dst[i] = lows ? lows[i] : (i % 2 ? low1 : low0);
-  hipLaunchKernelGGL(f32_compress_kernel, dim3(f32_grid(lowpx)), dim3(kF32Threads), 0, stream, (const float*)skip, wimg,
-                     dst[0], Hl, Wl, batch);
+  const int low_blocks = (int)std::min((lowpx + 63) / 64, 2L * cus);     // four groups of 16 pixels a block, persistent
+  hipLaunchKernelGGL(f32_compress_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)skip,
+                     (const h8*)wts.compress, wimg + kF32Compress + 8192, dst[0], Hl, Wl, (int)lowpx, wts.compress_scale);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[2], stream)) != hipSuccess) return e;
   for (int l = 0; l < 4; ++l)
     if ((e = launch_f32_grouped(dst[l], wts, l, dst[l + 1], Hl, Wl, batch, cus, stream)) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[3], stream)) != hipSuccess) return e;
-  hipLaunchKernelGGL(f32_expand_kernel, dim3(f32_grid(lowpx)), dim3(kF32Threads), 0, stream, (const float*)dst[4],
-                     (const float*)skip, wimg, work, Hl, Wl, batch);
+  hipLaunchKernelGGL(f32_expand_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)dst[4],
+                     (const float*)skip, (const h8*)wts.expand, wimg + kF32Expand + 8192, work, Hl, Wl, (int)lowpx,
+                     wts.expand_scale);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[4], stream)) != hipSuccess) return e;
   if ((e = launch_f32_refine_tail(work, wts, meta, Hq, Wq, batch, cus, stream)) != hipSuccess) return e;

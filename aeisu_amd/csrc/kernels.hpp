@@ -133,8 +133,9 @@ struct F32SplitScale {
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
   const float* image;
-  const void *grouped[4], *refine, *tail;  // [T][tap][part] (T = 2 group + t), [T][k][part] for the tail
-  F32SplitScale grouped_scale[4], refine_scale, tail_scale;
+  const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
+  const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
+  F32SplitScale compress_scale, grouped_scale[4], expand_scale, refine_scale, tail_scale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong
