@@ -314,7 +314,8 @@ struct ModeWeights {
   DeviceBuffer body_consts;        // epilogue constants of the fused body (kBodyConsts floats)
   DeviceBuffer fp32;               // FP32 policy: the whole weight image (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
-  DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail;
+  DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail, f32_head;
+  float f32_head_unscale = 1.f;
   F32SplitScale f32_compress_scale{}, f32_grouped_scale[4] = {}, f32_expand_scale{}, f32_refine_scale{}, f32_tail_scale{};
 
   // every device buffer, for commit() and byte accounting
@@ -335,6 +336,7 @@ struct ModeWeights {
     fn(f32_expand);
     fn(f32_refine);
     fn(f32_tail);
+    fn(f32_head);
   }
   F32Weights f32_weights() const {
     F32Weights W;
@@ -347,6 +349,8 @@ struct ModeWeights {
     W.compress_scale = f32_compress_scale;
     W.expand = f32_expand.ptr;
     W.expand_scale = f32_expand_scale;
+    W.head = f32_head.ptr;
+    W.head_unscale = f32_head_unscale;
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
     W.refine_scale = f32_refine_scale;
@@ -568,8 +572,26 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   rt.f32_refine_scale = split("refine", 64, 32, 3, 36, conv3, rt.f32_refine);
   rt.f32_tail_scale = split("tail", 64, 64, 1, 8,
                             [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; }, rt.f32_tail);
-  for (int i = 0; i < 100; ++i) img[kF32Base + i] = base[i];
-  for (int i = 0; i < 1600; ++i) img[kF32Basis + i] = basis[i];
+  // head bank, scaled so that the largest weight lies in [2^13, 2^14): row 4g + i of tile t is phase g of tap
+  // 4t + i (taps past 24 are zero), slots 0..15 the hi halves of the coefficients' weights, 16..31 the lo halves
+  float top = 0.f;
+  for (int i = 0; i < 1600; ++i) top = std::max(top, std::fabs(basis[i]));
+  const int e = top > 0.f ? std::min(13 - std::ilogb(top), 30) : 0;
+  auto bank = pack_frags<uint16_t>(7, 8, [&](int t, int m, int s) -> uint16_t {
+    const int tap = 4 * t + m % 4;
+    if (tap > 24) return 0;
+    const float v = std::ldexp(basis[(tap * 16 + s % 16) * 4 + m / 4], e);
+    const uint16_t hi = f32_to_f16_bits(v);
+    return s < 16 ? hi : f32_to_f16_bits(v - f16_bits_to_f32(hi));
+  });
+  std::vector<float> rows(4 * 7 * 4, 0.f);
+  for (int g = 0; g < 4; ++g)
+    for (int tap = 0; tap < 25; ++tap) rows[g * 28 + tap] = std::ldexp(base[tap * 4 + g], e);
+  const size_t halves = bank.size();
+  bank.resize(halves + 2 * rows.size());
+  std::memcpy(bank.data() + halves, rows.data(), rows.size() * sizeof(float));
+  rt.f32_head.upload(bank);
+  rt.f32_head_unscale = std::ldexp(1.f, -e);
   for (int i = 0; i < 24; ++i) img[kF32Analysis + i] = rt.analysis[i];
   rt.fp32.upload(img);
 }
@@ -1094,8 +1116,8 @@ static void enqueue_fp32(const ModeWeights& w, const Geometry& g, const Scratch&
                                      g.nlow == 5 ? lows : nullptr, static_cast<float*>(sc.work), static_cast<float*>(sc.meta),
                                      g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, g.cus, s, ev),
                "FP32 controller launch", s);
-  check_launch(launch_f32_head(g.in_fp32, g.out_fp32, d_in, static_cast<const float*>(sc.meta), w.fp32.as<float>(), d_out,
-                               g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, sc.nonfinite, s),
+  check_launch(launch_f32_head(g.in_fp32, g.out_fp32, d_in, static_cast<const float*>(sc.meta), w.f32_weights(), d_out,
+                               g.H, g.W, g.Hq, g.Wq, g.py, g.px, g.batch, g.cus, sc.nonfinite, s),
                "FP32 head launch", s);
   if (ev) check_hip(hipEventRecord(ev[6], s), "hipEventRecord");
 }

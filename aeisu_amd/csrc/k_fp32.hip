@@ -506,7 +506,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
   }
 }
 
-// ---- head: clamp, polyphase filter synthesis, 5x5 application, clip: one LR pixel per thread -------
+// ---- head: clamp, polyphase filter synthesis, 5x5 application, clip ----------------------------------
 // coefficient_clamp (aeisu/reconstruction.py:15-17) in FP32 with the reference's separate multiply
 // and add; a NaN coefficient stays NaN (so does the output, which raises the non-finite flag).
 __device__ __forceinline__ float clamp_coef(float a) {
@@ -517,72 +517,165 @@ __device__ __forceinline__ float clamp_coef(float a) {
   v = v > 2.5f ? 2.5f : v;
   return copysignf(v, a);
 }
-template <typename Tout>
-__device__ __forceinline__ Tout from_f32(float v);
-template <>
-__device__ __forceinline__ float from_f32<float>(float v) { return v; }
-template <>
-__device__ __forceinline__ _Float16 from_f32<_Float16>(float v) { return (_Float16)v; }
+
+// Persistent blocks over tiles of 64 x 4 LR pixels, one row per wave, in two chunks of 32 pixels.  The filter
+// weights of a chunk's even and odd pixels are two MFMA products of 16 columns, as in k_head.hip: row 4g + i of
+// row tile t is (phase g, tap 4t + i), so accumulator lane (n, g) holds all 25 taps of phase g of pixels 2n and
+// 2n + 1, and [K_hi | K_lo] . [c ; c] runs once with the coefficients' lo and once with their hi halves on top
+// of the FP32 base (bank and base scaled by a power of two, the RGB tile by its inverse).
+// The lane applies them with FP32 FMAs in tap order.  Two neighbouring pixels share 20 of their 25 window
+// positions: 30 LDS reads of 16 bytes instead of 50, which would take 46 us of LDS time at 1080p; the tile
+// holds even and odd columns apart, so that the lanes' reads are contiguous.  One thread per pixel took 168 us
+// at 1080p (1,600 FMAs of synthesis and strided coefficient reads).
+constexpr int kF32HW = 64, kF32HH = 4;                       // LR pixels of a tile
+constexpr int kF32HLW = kF32HW + 4, kF32HLH = kF32HH + 4;    // with the 2-pixel halo
+constexpr int kF32HPos = kF32HLW * kF32HLH, kF32HPer = (kF32HPos + kF32Threads - 1) / kF32Threads;
+constexpr int kF32HPlane = kF32HPos / 2;
+struct F32HeadGeom {
+  int H, W, Hq, Wq, py, px, tiles_x, tiles_y, num;
+  float unscale;                                             // of the bank's power of two
+};
+template <typename Tin>
+struct F32HeadFetch {
+  Tin rgb[kF32HPer][3];
+  float4 coef[2][2][2];                                      // [chunk][pixel parity][half of the lane's eight]
+};
+struct F32HeadTile {
+  int b, y0, x0;
+};
+__device__ __forceinline__ F32HeadTile f32_head_tile(int tidx, const F32HeadGeom& G) {
+  const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per, ty = rem / G.tiles_x;
+  return {b, ty * kF32HH, (rem - ty * G.tiles_x) * kF32HW};
+}
+template <typename Tin>
+__device__ __forceinline__ void f32_head_fetch(F32HeadFetch<Tin>& f, const Tin* __restrict__ src,
+                                               const float* __restrict__ meta, F32HeadTile t, const F32HeadGeom& G, int tid,
+                                               int wave, int n, int g) {
+  const size_t plane = (size_t)G.H * G.W;
+  const Tin* s = src + (size_t)t.b * 3 * plane;
+#pragma unroll
+  for (int k = 0; k < kF32HPer; ++k) {
+    const int q = min(tid + kF32Threads * k, kF32HPos - 1), ly = q / kF32HLW, lx = q - ly * kF32HLW;
+    const size_t o = (size_t)min(max(t.y0 + ly - 2, 0), G.H - 1) * G.W + min(max(t.x0 + lx - 2, 0), G.W - 1);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f.rgb[k][c] = s[c * plane + o];
+  }
+  // pixels past the frame edge take the edge's coefficients (inside the tensor) and are not stored
+  const int Y = min(t.y0 + wave, G.H - 1) + G.py;
+  const float* row = meta + ((size_t)t.b * G.Hq + (Y >> 1)) * G.Wq * 64 + 32 * (Y & 1) + 8 * (g & 1);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int X = min(t.x0 + 32 * j + 2 * n + p, G.W - 1) + G.px;
+      const float* c = row + (size_t)(X >> 1) * 64 + 16 * (X & 1);
+      f.coef[j][p][0] = *reinterpret_cast<const float4*>(c);
+      f.coef[j][p][1] = *reinterpret_cast<const float4*>(c + 4);
+    }
+}
+// Output columns 4n .. 4n + 3 of a chunk row and channel: pixels 2n and 2n + 1, left and right.
+__device__ __forceinline__ void store_quad(float* p, float a, float b, float c, float d, bool second) {
+  if (second) *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
+  else *reinterpret_cast<float2*>(p) = make_float2(a, b);
+}
+__device__ __forceinline__ void store_quad(_Float16* p, float a, float b, float c, float d, bool second) {
+  if (second) *reinterpret_cast<u2*>(p) = u2{pack_h2(a, b), pack_h2(c, d)};
+  else *reinterpret_cast<unsigned*>(p) = pack_h2(a, b);
+}
 
 template <typename Tin, typename Tout>
-__global__ __launch_bounds__(kF32Threads) void f32_head_kernel(const Tin* __restrict__ src, const float* __restrict__ meta,
-                                                               const float* __restrict__ wimg, Tout* __restrict__ out, int H,
-                                                               int W, int Hq, int Wq, int py, int px, int batch,
-                                                               unsigned* __restrict__ nonfinite) {
-  const long idx = (long)blockIdx.x * kF32Threads + threadIdx.x;
-  const bool live = idx < (long)batch * H * W;
-  const long id = live ? idx : 0;
-  const int b = (int)(id / ((long)H * W));
-  const int rem = (int)(id - (long)b * H * W);
-  const int y = rem / W, x = rem - y * W;
-  const size_t plane = (size_t)H * W;
-  const Tin* s = src + (size_t)b * 3 * plane;
-  // coefficients of this LR pixel: channel 16 rho + k of its packed pixel on the padded grid
-  const int Y = y + py, X = x + px, rho = ((Y & 1) << 1) | (X & 1);
-  const float* mp = meta + (((size_t)b * Hq + (Y >> 1)) * Wq + (X >> 1)) * 64 + 16 * rho;
-  float a[16];
+__global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __restrict__ src, const float* __restrict__ meta,
+                                                                  const h8* __restrict__ bank, Tout* __restrict__ out,
+                                                                  F32HeadGeom G, unsigned* __restrict__ nonfinite) {
+  __shared__ float4 tiles[2][2][kF32HPlane];                 // [buffer][column parity]
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, n = lane & 15, g = lane >> 4;
+  h8 A[7];
+  f4 base[7];
+  const f4* bf = reinterpret_cast<const f4*>(bank + 7 * 64);
 #pragma unroll
-  for (int k = 0; k < 16; k += 4) {
-    const float4 v = *reinterpret_cast<const float4*>(mp + k);
-    a[k] = clamp_coef(v.x);
-    a[k + 1] = clamp_coef(v.y);
-    a[k + 2] = clamp_coef(v.z);
-    a[k + 3] = clamp_coef(v.w);
+  for (int t = 0; t < 7; ++t) {
+    A[t] = bank[t * 64 + lane];
+    base[t] = bf[g * 7 + t];
   }
-  // 5x5 RGB window, replicate-clamped
-  float L[25][3];
+  const size_t oplane = (size_t)4 * G.H * G.W;
+  float chk = 0.f;                                           // NaN once an output was not finite
+  const int iters = tile_iters(G.num);
+  int tidx = tile_of(0, G.num);
+  F32HeadFetch<Tin> f;
+  if (tidx < G.num) f32_head_fetch(f, src, meta, f32_head_tile(tidx, G), G, tid, wave, n, g);
+  for (int it = 0; it < iters; ++it) {
+    if (tidx >= G.num) break;                                // block-uniform
+    const F32HeadTile t = f32_head_tile(tidx, G);
+    float4(*buf)[kF32HPlane] = tiles[it & 1];
 #pragma unroll
-  for (int t = 0; t < 25; ++t) {
-    const int sy = min(max(y + t / 5 - 2, 0), H - 1), sx = min(max(x + t % 5 - 2, 0), W - 1);
-    const size_t o = (size_t)sy * W + sx;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) L[t][c] = to_f32(s[c * plane + o]);
-  }
-  const float* base = wimg + kF32Base;     // [25][4]
-  const float* basis = wimg + kF32Basis;   // [25][16][4]
-  const size_t oplane = (size_t)4 * H * W;
-  Tout* o = out + (size_t)b * 3 * oplane;
-  float chk = 0.f;
-#pragma unroll
-  for (int ph = 0; ph < 4; ++ph) {
-    float u[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < 25; ++t) {
-      float wt = 0.f;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) wt = fmaf(a[k], basis[(t * 16 + k) * 4 + ph], wt);
-      wt += base[t * 4 + ph];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) u[c] = fmaf(wt, L[t][c], u[c]);
+    for (int k = 0; k < kF32HPer; ++k) {
+      const int q = tid + kF32Threads * k;                   // positions of a row alternate between the planes
+      if (q < kF32HPos) buf[q & 1][q >> 1] = make_float4((float)f.rgb[k][0] * G.unscale, (float)f.rgb[k][1] * G.unscale, (float)f.rgb[k][2] * G.unscale, 0.f);
     }
-    chk = fmaf(u[0] + u[1] + u[2], 0.f, chk);
-    if (live) {
-      const size_t op = (size_t)(2 * y + (ph >> 1)) * (2 * W) + 2 * x + (ph & 1);
+    float4 coef[2][2][2];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) o[c * oplane + op] = from_f32<Tout>(__builtin_amdgcn_fmed3f(u[c], 0.f, 1.f));
+    for (int i = 0; i < 8; ++i) coef[i >> 2][(i >> 1) & 1][i & 1] = f.coef[i >> 2][(i >> 1) & 1][i & 1];
+    tidx = tile_of(it + 1, G.num);
+    if (it + 1 < iters && tidx < G.num) f32_head_fetch(f, src, meta, f32_head_tile(tidx, G), G, fresh(tid), wave, n, g);
+    lds_barrier();                                           // buf complete; the other buffer is free again
+    const int y = t.y0 + wave;
+    if (y >= G.H) continue;                                  // wave-uniform; the barriers are above
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (t.x0 + 32 * j >= G.W) break;                       // wave-uniform
+      f4 w[2][7];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const float4 c0 = coef[j][p][0], c1 = coef[j][p][1];
+        h8 hi, lo;
+        split8(make_float4(clamp_coef(c0.x), clamp_coef(c0.y), clamp_coef(c0.z), clamp_coef(c0.w)),
+               make_float4(clamp_coef(c1.x), clamp_coef(c1.y), clamp_coef(c1.z), clamp_coef(c1.w)), 1.f, hi, lo);
+#pragma unroll
+        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], lo, base[q]);
+#pragma unroll
+        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], hi, w[p][q]);
+      }
+      float u[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int dy = 0; dy < 5; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 6; ++dx) {
+          const float4 L = buf[dx & 1][(wave + dy) * (kF32HLW / 2) + 16 * j + n + (dx >> 1)];
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            if (dx - p < 0 || dx - p > 4) continue;
+            const int tap = dy * 5 + dx - p;
+            const float wt = w[p][tap >> 2][tap & 3];
+            u[p][0] = fmaf(wt, L.x, u[p][0]);
+            u[p][1] = fmaf(wt, L.y, u[p][1]);
+            u[p][2] = fmaf(wt, L.z, u[p][2]);
+          }
+        }
+      // pair phases (TL, TR) in lane groups 0 and 1 and (BL, BR) in 2 and 3: even groups then store channel 0
+      // and channel 2, odd groups channel 1
+      const int x = t.x0 + 32 * j + 2 * n;
+      float left[2][3], right[2][3];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const bool inside = x + p < G.W;
+        chk = fmaf(inside ? u[p][0] + u[p][1] + u[p][2] : 0.f, 0.f, chk);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          left[p][c] = __builtin_amdgcn_fmed3f(u[p][c], 0.f, 1.f);
+          right[p][c] = left[p][c];
+          permlane16_swap(left[p][c], right[p][c]);
+        }
+      }
+      if (x < G.W) {
+        const bool second = x + 1 < G.W, odd = g & 1;
+        Tout* o = out + (size_t)t.b * 3 * oplane + (size_t)(2 * y + (g >> 1)) * (2 * G.W) + 2 * x;
+        store_quad(o + (odd ? oplane : 0), odd ? left[0][1] : left[0][0], odd ? right[0][1] : right[0][0],
+                   odd ? left[1][1] : left[1][0], odd ? right[1][1] : right[1][0], second);
+        if (!odd) store_quad(o + 2 * oplane, left[0][2], right[0][2], left[1][2], right[1][2], second);
+      }
     }
   }
-  if (nonfinite && __ballot(live && chk != chk) != 0ull && (threadIdx.x & 63) == 0) atomicOr(nonfinite, 1u);
+  if (nonfinite && __ballot(chk != chk) != 0ull && lane == 0) atomicOr(nonfinite, 1u);
 }
 
 // ---- launchers ---------------------------------------------------------------------------------------
@@ -666,13 +759,15 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
   return hipSuccess;
 }
 
-hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const float* wimg, void* out,
-                           int H, int W, int Hq, int Wq, int py, int px, int batch, unsigned* nonfinite,
+hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const F32Weights& wts, void* out,
+                           int H, int W, int Hq, int Wq, int py, int px, int batch, int cus, unsigned* nonfinite,
                            hipStream_t stream) {
-  const int grid = f32_grid((long)batch * H * W);
-#define AEISU_F32_HEAD(TI, TO)                                                                                     \
-  hipLaunchKernelGGL((f32_head_kernel<TI, TO>), dim3(grid), dim3(kF32Threads), 0, stream, (const TI*)src, meta, wimg, \
-                     (TO*)out, H, W, Hq, Wq, py, px, batch, nonfinite)
+  F32HeadGeom G{H, W, Hq, Wq, py, px, (W + kF32HW - 1) / kF32HW, (H + kF32HH - 1) / kF32HH, 0, wts.head_unscale};
+  G.num = batch * G.tiles_x * G.tiles_y;
+  const int grid = conv_grid(G.num, 2 * cus);
+#define AEISU_F32_HEAD(TI, TO)                                                                                        \
+  hipLaunchKernelGGL((f32_head_kernel<TI, TO>), dim3(grid), dim3(kF32Threads), 0, stream, (const TI*)src, meta,       \
+                     (const h8*)wts.head, (TO*)out, G, nonfinite)
   if (in_fp32 && out_fp32) AEISU_F32_HEAD(float, float);
   else if (in_fp32) AEISU_F32_HEAD(float, _Float16);
   else if (out_fp32) AEISU_F32_HEAD(_Float16, float);

@@ -112,7 +112,7 @@ hipError_t launch_fused_tail_head(int in_fp32, int out_fp32, int qclamp, const v
 //   project  W[32 feature channel f*4+phase][32] b[32]; compress W[128 skip channel c*4+phase][64] b[64];
 //   bottleneck l: W[9][32 group input][64] b[64] (output 32g+o reads group g's inputs);
 //   expand W[64][128] b[128] (output c*4+phase); refine W[9][32][64] b[64]; tail W[64][64] b[64];
-//   then adaptive_base [25][4], adaptive_basis [25][16][4], the 24 analysis constants.
+//   then the 24 analysis constants.
 constexpr int kF32Project = 0;
 constexpr int kF32Compress = kF32Project + 32 * 32 + 32;
 constexpr int kF32GroupedStride = 9 * 32 * 64 + 64;
@@ -120,9 +120,7 @@ constexpr int kF32Grouped = kF32Compress + 128 * 64 + 64;
 constexpr int kF32Expand = kF32Grouped + 4 * kF32GroupedStride;
 constexpr int kF32Refine = kF32Expand + 64 * 128 + 128;
 constexpr int kF32Tail = kF32Refine + 9 * 32 * 64 + 64;
-constexpr int kF32Base = kF32Tail + 64 * 64 + 64;
-constexpr int kF32Basis = kF32Base + 25 * 4;
-constexpr int kF32Analysis = kF32Basis + 25 * 16 * 4;
+constexpr int kF32Analysis = kF32Tail + 64 * 64 + 64;
 constexpr int kF32Floats = kF32Analysis + 24;
 // A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent, and an output's
 // magnitude is at most gain * (largest input magnitude) + offset.
@@ -135,6 +133,9 @@ struct F32Weights {
   const float* image;
   const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
+  const void* head;                        // 7 fragments [K_hi | K_lo] (row 4g + i of tile t: phase g, tap 4t + i), then
+                                           // the FP32 base float4 [g][t], both divided by head_unscale
+  float head_unscale;
   F32SplitScale compress_scale, grouped_scale[4], expand_scale, refine_scale, tail_scale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
@@ -143,8 +144,8 @@ struct F32Weights {
 hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights& wts, float* skip, float* low0, float* low1,
                                  float* const* lows, float* work, float* meta, int H, int W, int Hq, int Wq, int py, int px,
                                  int batch, int cus, hipStream_t stream, hipEvent_t* ev);
-hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const float* wimg, void* out,
-                           int H, int W, int Hq, int Wq, int py, int px, int batch, unsigned* nonfinite,
+hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const F32Weights& wts, void* out,
+                           int H, int W, int Hq, int Wq, int py, int px, int batch, int cus, unsigned* nonfinite,
                            hipStream_t stream);
 
 // Resident blocks per CU (occupancy), used to size the persistent grids.

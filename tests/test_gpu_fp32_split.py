@@ -14,7 +14,7 @@ import torch
 from torch.nn import functional as F
 
 from oracle import model as M
-from tests._util import WEIGHTS
+from tests._util import WEIGHTS, crop_output, pad_frame
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,32 @@ def test_nonfinite_input_stays_local(model, bad):
     far = torch.ones(160, 300, dtype=torch.bool)
     far[2 * (40 - 32):2 * (40 + 33), 2 * (70 - 32):2 * (70 + 33)] = False
     assert (got - clean).abs()[..., far].max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("dtypes", [("f32", "f32"), ("f16", "f32"), ("f32", "f16"), ("f16", "f16")], ids="-".join)
+@pytest.mark.parametrize("size", [(1, 1, 1), (1, 4, 64), (2, 5, 65), (1, 7, 31), (1, 33, 130), (3, 250, 331)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_head_against_64_bits(model, size, dtypes):
+    """The head on the GPU's own coefficients, at ragged widths and heights, in every pair of layouts.  An
+    output is 25 filter weights (each 16 products and a base) applied to the window: 2^-22 (3 + 4 * 16 / 8) of
+    the weights' terms and 25 FP32 roundings of the sums, and the output's rounding."""
+    from aeisu_amd import _lib as L
+    kind = {"f16": torch.float16, "f32": torch.float32}
+    m, state = model
+    b, h, w = size
+    print(f"case: FP32 head {size} {dtypes}", flush=True)
+    frames = (1.4 * torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(h + w)) - 0.2).to(kind[dtypes[0]])
+    flags = L.FLAG_KEEP_INTERMEDIATES
+    got = m.run(frames.cuda(), out_dtype=kind[dtypes[1]], flags=flags).cpu().double()
+    hd = m.handle(b, h, w, kind[dtypes[0]], kind[dtypes[1]], flags)
+    _, _, _, _, hq, wq = m.geometry(hd)
+    meta = m.intermediate(hd, L.BUF_META).cpu().view(torch.float32).reshape(b, hq, wq, 64).permute(0, 3, 1, 2).double()
+    padded = pad_frame(frames).double()
+    base, basis = state["base"].double(), state["basis"].double()
+    ref = crop_output(M.reconstruct(padded, meta, base, basis), h, w)
+    size_ = crop_output(M.reconstruct(padded.abs(), meta.abs(), base.abs(), basis.abs()), h, w)
+    bound = (2.0 ** -22 * 11 + 25 * 2.0 ** -24) * size_ + 1e-12
+    if dtypes[1] == "f16":
+        bound = bound + 2.0 ** -11 * ref.abs() + 2.0 ** -25
+    over = (got - ref.clamp(0, 1)).abs() - bound
+    assert over.max().item() <= 0, f"{over.max().item():.3g} over the bound"
