@@ -35,7 +35,8 @@
 //    per LDS pixel; the Mixed policy widens codes to FP16 operands with
 //    v_cvt_scalef32_pk_f16_fp8 as it reads them.  The frame-input variants also come with
 //    T = 16 for frames whose 24x24 tiles would leave CUs idle (body_fused_plan picks the tiles
-//    per shape: trailing frames or right-hand columns on 16x16 tiles, in the same launch).
+//    per shape: trailing frames or right-hand columns on 16x16 tiles, in the same launch), and with
+//    the compress exchange T = 12 and 8 for the smallest frames (body_fused_xc_small_tile).
 //  * FP16 activations: T = 16, 144 bytes per LDS pixel.
 // Compress exchange (body_fused_xc_kernel, frame input): when a whole-frame launch has no more tiles
 // than the device has CUs, every tile is resident at once, so a tile computes compress on its T x T
@@ -355,8 +356,9 @@ __device__ __forceinline__ void fb_compress(const BodyFusedArgs& P, BodyTileF t,
 }
 
 // ---- frame input: RGB staging, analysis features and project per 16-pixel group -----------------
-// A group of a flattened region (side S >= 16, low-grid origin (oy, ox)) covers at most two row
-// segments: m pixels of region row r from column c, then 16 - m pixels of row r + 1 from column 0.
+// A group of a flattened region (side S >= 16, or 8 or 12, whose groups start at columns 0, or 0, 4 and 8;
+// low-grid origin (oy, ox)) covers at most two row segments: m pixels of region row r from column c, then
+// 16 - m pixels of row r + 1 from column 0.
 // Its stage covers the 6 padded-LR rows 4 ly - 1 .. 4 ly + 4 of each segment's low row ly, side by
 // side: segment 1 in stage columns 0 .. 4m + 1, segment 2 after it (68 columns in all).  The stage
 // holds the luma of every stage pixel (kSR rows of kSW floats), computed once per LR pixel, and the

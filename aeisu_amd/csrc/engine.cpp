@@ -950,7 +950,7 @@ static Geometry make_geometry(int mode, bool project_precise, int cus, int batch
   // once (one block per CU), else launches of whole frames where they beat the plan without it
   if (g.fused_rgb && !(flags & AEISU_FLAG_BODY_NO_EXCHANGE)) {
     if (plan.cols24 == 0 && (plan.frames24 == batch || plan.frames24 == 0)) {
-      const int tile = plan.frames24 == batch ? 24 : 16;
+      const int tile = plan.frames24 == batch ? 24 : body_fused_xc_small_tile(mode, batch, g.Hl, g.Wl, cus);
       if (body_fused_num_tiles(mode, batch, g.Hl, g.Wl, tile) <= cus) {
         g.body_xc_tile = tile;
         g.body_xc_frames = batch;

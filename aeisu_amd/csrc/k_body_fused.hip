@@ -83,6 +83,20 @@ BodyXcPlan body_fused_xc_plan(int mode, int batch, int Hl, int Wl, int cus, bool
   return launches * kGain < 0.99 * base ? BodyXcPlan{24, frames} : none;
 }
 
+// Side of the exchange's tiles for launches that would leave CUs idle with 24x24 tiles: such a launch takes one
+// tile's latency, so the smallest tiles that are all resident at once are taken.  With the exchange a tile's
+// compress costs only its core, so smaller tiles add no compress work, only the grouped layers' halos, which
+// idle CUs take.  Whole call, Mixed: 48 x 64 38.7 us on 16x16 tiles, 26.9 on 8x8; 270 x 480 40.2 and 28.3;
+// 360 x 640 45.7 on 16x16, 39.4 on 12x12; 480 x 854 50.3 and 44.6 (INT8: 33.8 and 24.0, 35.7 and 25.4, 41.0 and
+// 34.9, 45.7 and 40.3).  12x12 tiles serve launches whose 16x16 tiles would leave half of the CUs idle: 540p has
+// 144 of those and keeps them (its plan is fixed by test_body_exchange_selection; 12x12 tiles measured 44.5
+// against 50.8 us).
+int body_fused_xc_small_tile(int mode, int batch, int Hl, int Wl, int cus) {
+  if (body_fused_num_tiles(mode, batch, Hl, Wl, 8) <= cus) return 8;
+  if (body_fused_num_tiles(mode, batch, Hl, Wl, 12) <= cus && 2 * body_fused_num_tiles(mode, batch, Hl, Wl, 16) <= cus) return 12;
+  return 16;
+}
+
 // FP16 policy: the same trade between 16x16 tiles and 8x8 tiles (compress region 16^2 against
 // 24^2 pixels plus the fixed per-tile prologue: about half the cost), split by low rows since the
 // batch is usually one frame: rows [0, R) on 16x16 tiles, the rest on 8x8 tiles, in one launch.
@@ -124,7 +138,13 @@ hipError_t body_fused_prepare() {
       {body_xc_ptr<3, 1, 24>(), BodyFusedCfg<3, 24>::LdsRgb}, {body_xc_ptr<3, 2, 24>(), BodyFusedCfg<3, 24>::LdsRgb},
       {body_xc_ptr<1, 1, 16>(), BodyFusedCfg<1, 16>::LdsRgb}, {body_xc_ptr<1, 2, 16>(), BodyFusedCfg<1, 16>::LdsRgb},
       {body_xc_ptr<2, 1, 16>(), BodyFusedCfg<2, 16>::LdsRgb}, {body_xc_ptr<2, 2, 16>(), BodyFusedCfg<2, 16>::LdsRgb},
-      {body_xc_ptr<3, 1, 16>(), BodyFusedCfg<3, 16>::LdsRgb}, {body_xc_ptr<3, 2, 16>(), BodyFusedCfg<3, 16>::LdsRgb}};
+      {body_xc_ptr<3, 1, 16>(), BodyFusedCfg<3, 16>::LdsRgb}, {body_xc_ptr<3, 2, 16>(), BodyFusedCfg<3, 16>::LdsRgb},
+      {body_xc_ptr<1, 1, 8>(), BodyFusedCfg<1, 8>::LdsRgb},   {body_xc_ptr<1, 2, 8>(), BodyFusedCfg<1, 8>::LdsRgb},
+      {body_xc_ptr<2, 1, 8>(), BodyFusedCfg<2, 8>::LdsRgb},   {body_xc_ptr<2, 2, 8>(), BodyFusedCfg<2, 8>::LdsRgb},
+      {body_xc_ptr<3, 1, 8>(), BodyFusedCfg<3, 8>::LdsRgb},   {body_xc_ptr<3, 2, 8>(), BodyFusedCfg<3, 8>::LdsRgb},
+      {body_xc_ptr<1, 1, 12>(), BodyFusedCfg<1, 12>::LdsRgb}, {body_xc_ptr<1, 2, 12>(), BodyFusedCfg<1, 12>::LdsRgb},
+      {body_xc_ptr<2, 1, 12>(), BodyFusedCfg<2, 12>::LdsRgb}, {body_xc_ptr<2, 2, 12>(), BodyFusedCfg<2, 12>::LdsRgb},
+      {body_xc_ptr<3, 1, 12>(), BodyFusedCfg<3, 12>::LdsRgb}, {body_xc_ptr<3, 2, 12>(), BodyFusedCfg<3, 12>::LdsRgb}};
   for (const K& e : k) {
     const hipError_t r = hipFuncSetAttribute(e.fn, hipFuncAttributeMaxDynamicSharedMemorySize, e.lds);
     if (r != hipSuccess) return r;
@@ -179,10 +199,14 @@ static void launch_xc_t(const BodyFusedArgs& args, int tiles, hipStream_t stream
 template <int MODE>
 static void launch_xc_m(BodySrc src, const BodyFusedArgs& args, int tile, int tiles, hipStream_t stream) {
   if (src == BodySrc::Frames16) {
-    if (tile == 16) launch_xc_t<MODE, 1, 16>(args, tiles, stream);
+    if (tile == 8) launch_xc_t<MODE, 1, 8>(args, tiles, stream);
+    else if (tile == 12) launch_xc_t<MODE, 1, 12>(args, tiles, stream);
+    else if (tile == 16) launch_xc_t<MODE, 1, 16>(args, tiles, stream);
     else launch_xc_t<MODE, 1, 24>(args, tiles, stream);
   } else {
-    if (tile == 16) launch_xc_t<MODE, 2, 16>(args, tiles, stream);
+    if (tile == 8) launch_xc_t<MODE, 2, 8>(args, tiles, stream);
+    else if (tile == 12) launch_xc_t<MODE, 2, 12>(args, tiles, stream);
+    else if (tile == 16) launch_xc_t<MODE, 2, 16>(args, tiles, stream);
     else launch_xc_t<MODE, 2, 24>(args, tiles, stream);
   }
 }
@@ -190,7 +214,7 @@ static void launch_xc_m(BodySrc src, const BodyFusedArgs& args, int tile, int ti
 hipError_t launch_body_fused_xc(int mode, BodySrc src, const BodyFusedArgs& args, int batch, int tile, int cus,
                                 hipStream_t stream) {
   // whole frames only, every tile resident at once (the LDS admits one block per CU)
-  if (mode == 0 || src == BodySrc::Skip || (tile != 24 && tile != 16)) return hipErrorInvalidValue;
+  if (mode == 0 || src == BodySrc::Skip || (tile != 24 && tile != 16 && tile != 12 && tile != 8)) return hipErrorInvalidValue;
   if (args.row0 || args.rows || args.col0 || args.cols || !args.xbuf || !args.xflags)
     return hipErrorInvalidValue;
   const int tiles = body_fused_num_tiles(mode, batch, args.Hl, args.Wl, tile);

@@ -83,12 +83,14 @@ struct BodyXcPlan {
   int tile, frames;
 };
 BodyXcPlan body_fused_xc_plan(int mode, int batch, int Hl, int Wl, int cus, bool tile24_only);
+// side of the tiles (8, 12 or 16) of a whole-batch launch with the exchange where 24x24 tiles leave CUs idle
+int body_fused_xc_small_tile(int mode, int batch, int Hl, int Wl, int cus);
 // FP16 policy (skip input): low rows [0, R) on 16x16 tiles, the rest on 8x8 tiles; returns R
 int body_fused_row_split(int mode, int batch, int Hl, int Wl, int cus);
 hipError_t body_fused_prepare();
 hipError_t launch_body_fused(int mode, BodySrc src, const BodyFusedArgs& args, int batch, int tile,
                              hipStream_t stream);
-// Frame-input body with the compress exchange (quantized policies, whole frames, tile 24 or 16): one
+// Frame-input body with the compress exchange (quantized policies, whole frames, tile 24, 16, 12 or 8): one
 // block per tile, every block resident at once (tiles <= CUs, one block per CU), neighbouring tiles
 // synchronised through args.xflags.
 hipError_t launch_body_fused_xc(int mode, BodySrc src, const BodyFusedArgs& args, int batch, int tile, int cus,

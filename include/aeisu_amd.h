@@ -62,7 +62,7 @@ extern "C" {
                                             engine's structure); default: one fused kernel, the
                                             coefficients stay on chip.  KEEP_INTERMEDIATES implies it */
 #define AEISU_FLAG_BODY_TILE24 16u       /* frame-input body: always 24x24-low-pixel tiles (by default small
-                                            frames take 16x16 tiles; parity tests run both) */
+                                            frames take 16x16 or smaller tiles; parity tests run both) */
 #define AEISU_FLAG_BODY_NO_EXCHANGE 32u  /* frame-input body: every tile computes its whole compress halo (by
                                             default, when a launch's tiles all fit on the device at once,
                                             tiles take the halo ring from their neighbours; parity tests run
