@@ -877,11 +877,7 @@ const ModeWeights& Model::weights(int mode) {
   return *modes[mode];
 }
 
-static int clamp_grid(int tiles, int per_cu, int cus) {
-  int g = std::min(tiles, std::max(1, per_cu) * cus);
-  if (g >= 8) g -= g % 8;
-  return std::max(g, 1);
-}
+static int clamp_grid(int tiles, int per_cu, int cus) { return persistent_grid(tiles, std::max(1, per_cu) * cus); }
 
 static Geometry make_geometry(int mode, bool project_precise, int cus, int batch, int height, int width, int in_layout,
                               int out_layout, unsigned flags) {

@@ -686,16 +686,11 @@ static F32ConvTiles conv_tiles(int H, int W, int th, int batch) {
   G.num = batch * G.tiles_x * G.tiles_y;
   return G;
 }
-// Persistent blocks for `tiles` tiles with `most` resident at once, a multiple of 8 (the XCDs) where possible.
-static int conv_grid(int tiles, int most) {
-  const int g = std::min(tiles, most);
-  return g >= 8 ? g - g % 8 : g;
-}
 template <int TH>
 static hipError_t launch_grouped_t(const float* in, const F32Weights& W, int l, float* out, int Hl, int Wl, int batch, int cus,
                                    hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hl, Wl, TH, batch);
-  hipLaunchKernelGGL(f32_grouped_kernel<TH>, dim3(conv_grid(G.num, cus), 2), dim3(kConvThreads), 0, stream, in,
+  hipLaunchKernelGGL(f32_grouped_kernel<TH>, dim3(persistent_grid(G.num, cus), 2), dim3(kConvThreads), 0, stream, in,
                      (const h8*)W.grouped[l], W.image + kF32Grouped + l * kF32GroupedStride + 18432, out, G,
                      W.grouped_scale[l]);
   return hipGetLastError();
@@ -710,7 +705,7 @@ template <int TH>
 static hipError_t launch_refine_t(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch, int cus,
                                   hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hq, Wq, TH, batch);
-  hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(conv_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
+  hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(persistent_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
                      (const h8*)W.refine, (const h8*)W.tail, W.image + kF32Refine + 18432, W.image + kF32Tail + 4096, meta,
                      G, W.refine_scale, W.tail_scale);
   return hipGetLastError();
@@ -764,7 +759,7 @@ hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const flo
                            hipStream_t stream) {
   F32HeadGeom G{H, W, Hq, Wq, py, px, (W + kF32HW - 1) / kF32HW, (H + kF32HH - 1) / kF32HH, 0, wts.head_unscale};
   G.num = batch * G.tiles_x * G.tiles_y;
-  const int grid = conv_grid(G.num, 2 * cus);
+  const int grid = persistent_grid(G.num, 2 * cus);
 #define AEISU_F32_HEAD(TI, TO)                                                                                        \
   hipLaunchKernelGGL((f32_head_kernel<TI, TO>), dim3(grid), dim3(kF32Threads), 0, stream, (const TI*)src, meta,       \
                      (const h8*)wts.head, (TO*)out, G, nonfinite)
