@@ -312,7 +312,7 @@ struct ModeWeights {
   DeviceBuffer compress_rgb;       // INT8 compress weights in the frame-input fused body's K order
   DeviceBuffer tail_bias;
   DeviceBuffer body_consts;        // epilogue constants of the fused body (kBodyConsts floats)
-  DeviceBuffer fp32;               // FP32 policy: the whole weight image (kernels.hpp kF32*)
+  DeviceBuffer fp32;               // FP32 policy: project weights and every bias (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
   DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail, f32_head;
   float f32_head_unscale = 1.f;
@@ -505,7 +505,7 @@ static void require_prelu(const Artifact& a, const std::string& layer, uint32_t 
 static std::vector<float> as_f32_vector(const TensorView& t) { return std::vector<float>(t.f32(), t.f32() + t.count()); }
 
 // FP32 policy: every layer's FP32 weights (<layer>.weight_fp32, written by the folded-checkpoint
-// converter) re-laid [tap][ci][co] into one image (kernels.hpp kF32*).
+// converter): the FP32 image (kernels.hpp kF32*), and the split layers' MFMA fragments and scales.
 static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, const float* basis) {
   std::vector<float> img(kF32Floats, 0.f);
   auto w32 = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks) {
@@ -513,19 +513,16 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
       fail(AEISU_ERR_ARTIFACT, "the FP32 policy needs " + l + ".weight_fp32 (convert a folded FP32 checkpoint)");
     return a.need(l + ".weight_fp32", kF32, {cout, cin, ks, ks}).f32();
   };
-  auto layer = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, int off, float slope) {
+  auto check = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, float slope) {
     const float* w = w32(l, cout, cin, ks);
     require_prelu(a, l, cout, slope);
+    for (size_t i = 0; i < size_t(cout) * cin * ks * ks; ++i)
+      if (!std::isfinite(w[i])) fail(AEISU_ERR_ARTIFACT, "nonfinite weight in " + l);
+    return w;
+  };
+  auto bias = [&](const std::string& l, uint32_t cout, int off) {
     const float* b = a.need(l + ".bias", kF32, {cout}).f32();
-    for (uint32_t o = 0; o < cout; ++o) {
-      for (uint32_t i = 0; i < cin; ++i)
-        for (uint32_t t = 0; t < ks * ks; ++t) {
-          const float v = w[(size_t(o) * cin + i) * ks * ks + t];
-          if (!std::isfinite(v)) fail(AEISU_ERR_ARTIFACT, "nonfinite weight in " + l);
-          img[off + (size_t(t) * cin + i) * cout + o] = v;         // [tap][ci][co]
-        }
-      img[off + size_t(ks * ks) * cin * cout + o] = b[o];
-    }
+    std::copy(b, b + cout, img.begin() + off);
   };
   // hi / lo FP16 fragments of a layer's weights, scaled so that the largest lies in [2^14, 2^15): chunk f of
   // `chunks`, row m, slot s is the weight at(f, m, s); the fragment order is chunk, then hi and lo
@@ -554,12 +551,22 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
     }));
     return sc;
   };
-  layer("project", 32, 32, 1, kF32Project, 0.1f);
-  layer("compress", 64, 128, 1, kF32Compress, 0.1f);
-  for (int l = 0; l < 4; ++l) layer("bottleneck" + std::to_string(l), 64, 32, 3, kF32Grouped + l * kF32GroupedStride, 0.1f);
-  layer("expand", 128, 64, 1, kF32Expand, 0.1f);
-  layer("refine", 64, 32, 3, kF32Refine, 0.1f);
-  layer("tail", 64, 64, 1, kF32Tail, 1.0f);
+  const float* wp = check("project", 32, 32, 1, 0.1f);
+  for (int o = 0; o < 32; ++o)
+    for (int i = 0; i < 32; ++i) img[kF32Project + i * 32 + o] = wp[o * 32 + i];
+  bias("project", 32, kF32Project + 1024);
+  check("compress", 64, 128, 1, 0.1f);
+  bias("compress", 64, kF32BiasCompress);
+  for (int l = 0; l < 4; ++l) {
+    check("bottleneck" + std::to_string(l), 64, 32, 3, 0.1f);
+    bias("bottleneck" + std::to_string(l), 64, kF32BiasGrouped + 64 * l);
+  }
+  check("expand", 128, 64, 1, 0.1f);
+  bias("expand", 128, kF32BiasExpand);
+  check("refine", 64, 32, 3, 0.1f);
+  bias("refine", 64, kF32BiasRefine);
+  check("tail", 64, 64, 1, 1.0f);
+  bias("tail", 64, kF32BiasTail);
   rt.f32_compress_scale = split("compress", 64, 128, 1, 16,
                                 [](int f, int m, int s) { return (16 * (f / 4) + m) * 128 + s * 4 + f % 4; }, rt.f32_compress);
   rt.f32_expand_scale = split("expand", 128, 64, 1, 16, [](int f, int m, int s) {
@@ -573,16 +580,20 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   rt.f32_tail_scale = split("tail", 64, 64, 1, 8,
                             [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; }, rt.f32_tail);
   // head bank, scaled so that the largest weight lies in [2^13, 2^14): row 4g + i of tile t is phase g of tap
-  // 4t + i (taps past 24 are zero), slots 0..15 the hi halves of the coefficients' weights, 16..31 the lo halves
+  // 4t + i (taps past 24 are zero); slots 0..15 the lo parts of the coefficients' weights and 16..31 the hi
+  // parts, or (fragments 7..13) the third and the hi parts
   float top = 0.f;
   for (int i = 0; i < 1600; ++i) top = std::max(top, std::fabs(basis[i]));
   const int e = top > 0.f ? std::min(13 - std::ilogb(top), 30) : 0;
-  auto bank = pack_frags<uint16_t>(7, 8, [&](int t, int m, int s) -> uint16_t {
-    const int tap = 4 * t + m % 4;
+  auto bank = pack_frags<uint16_t>(14, 8, [&](int f, int m, int s) -> uint16_t {
+    const int tap = 4 * (f % 7) + m % 4;
     if (tap > 24) return 0;
     const float v = std::ldexp(basis[(tap * 16 + s % 16) * 4 + m / 4], e);
     const uint16_t hi = f32_to_f16_bits(v);
-    return s < 16 ? hi : f32_to_f16_bits(v - f16_bits_to_f32(hi));
+    const float rest = v - f16_bits_to_f32(hi);
+    const uint16_t lo = f32_to_f16_bits(rest);
+    if (f < 7) return s < 16 ? lo : hi;
+    return s < 16 ? f32_to_f16_bits(rest - f16_bits_to_f32(lo)) : hi;
   });
   std::vector<float> rows(4 * 7 * 4, 0.f);
   for (int g = 0; g < 4; ++g)

@@ -7,12 +7,8 @@
 //   meta  [B][Hq][Wq][64]   refine 3x3 + LeakyReLU -> tail 1x1 (the packed coefficients)
 // and the head writes the clipped 2x frame.
 //
-// Two forms of kernel:
-//  * one thread per output pixel holds all its output channels in registers and walks the input
-//    channels; the weights, laid out [tap][ci][co] (kernels.hpp kF32*), are read at wave-uniform
-//    addresses, so they come through the scalar cache and feed the FP32 FMAs as scalar operands;
-//  * products of hi / lo FP16 splits on the MFMA (below), FP32 sums.
-// The sums run in a fixed order, which differs from the reference's convolution order only by FP32
+// The project runs as FP32 MFMAs, every other product as hi / lo FP16 splits on the FP16 MFMA (below);
+// all sums are FP32, in a fixed order that differs from the reference's convolution order only by FP32
 // rounding.
 #include <algorithm>
 
@@ -24,18 +20,25 @@ namespace aeisu {
 
 constexpr int kF32Threads = 256;
 
-__device__ __forceinline__ float leaky01(float v) { return v < 0.f ? v * 0.1f : v; }
-
 template <typename T>
 __device__ __forceinline__ float to_f32(T v) { return (float)v; }
 
-// ---- analysis features + project 1x1 + LeakyReLU: one packed pixel per thread ---------------------
+// ---- analysis features + project 1x1 + LeakyReLU ----------------------------------------------------
+// One wave per block takes 64 packed pixels: each lane computes one pixel's 32 features, hands them over
+// through LDS, and the wave runs the product as FP32 MFMAs (FP32 operands: the project weights reach 31 with
+// heavy cancellation, and split operands would double the layer's error).  K step j takes feature j of the four
+// phases (input channels 4j .. 4j + 3); features lie in LDS by phase, so that a lane's operands are 32
+// contiguous bytes.  With the product as 1,024 FMAs per
+// thread each wave waited for 1,024 weights from the scalar cache and stored 128 bytes per lane: 46 us at
+// 1080p, 11 to 15 us for 256 x 256.
+constexpr int kF32FeatRow = 36;                              // floats of a pixel's features in LDS (32 + 4 pad)
 template <typename Tin>
-__global__ __launch_bounds__(kF32Threads) void f32_project_kernel(const Tin* __restrict__ src, const float* __restrict__ wimg,
-                                                                  float* __restrict__ skip, int H, int W, int Hq, int Wq,
-                                                                  int py, int px, int batch) {
-  const long idx = (long)blockIdx.x * kF32Threads + threadIdx.x;
-  if (idx >= (long)batch * Hq * Wq) return;
+__global__ __launch_bounds__(64) void f32_project_kernel(const Tin* __restrict__ src, const float* __restrict__ wimg,
+                                                         float* __restrict__ skip, int H, int W, int Hq, int Wq, int py,
+                                                         int px, long pixels) {
+  __shared__ __attribute__((aligned(16))) float feat[64 * kF32FeatRow];
+  const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
+  const long first = (long)blockIdx.x * 64, idx = min(first + lane, pixels - 1);
   const int b = (int)(idx / ((long)Hq * Wq));
   const int rem = (int)(idx - (long)b * Hq * Wq);
   const int qy = rem / Wq, qx = rem - qy * Wq;
@@ -54,24 +57,43 @@ __global__ __launch_bounds__(kF32Threads) void f32_project_kernel(const Tin* __r
       for (int c = 0; c < 3; ++c) w[c][a][c4] = to_f32(s[c * plane + o]);
     }
   }
+  float A[2][8];
+  f4 bs[2];
+#pragma unroll
+  for (int T = 0; T < 2; ++T) {
+    bs[T] = *reinterpret_cast<const f4*>(wimg + kF32Project + 1024 + 16 * T + 4 * g);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) A[T][j] = wimg[kF32Project + (4 * j + g) * 32 + 16 * T + n];
+  }
   const Analysis an = analysis_from(wimg + kF32Analysis);
   float f[8][4];
   window_features(w, an, f);
-  const float* wp = wimg + kF32Project;
-  float acc[32];
 #pragma unroll
-  for (int co = 0; co < 32; ++co) acc[co] = 0.f;
+  for (int q = 0; q < 8; ++q)                                // phase q >> 1, features 4 (q & 1) .. + 3
+    *reinterpret_cast<float4*>(feat + lane * kF32FeatRow + 4 * q) =
+        make_float4(f[4 * (q & 1)][q >> 1], f[4 * (q & 1) + 1][q >> 1], f[4 * (q & 1) + 2][q >> 1], f[4 * (q & 1) + 3][q >> 1]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // one wave: its LDS stores are done
 #pragma unroll
-  for (int ci = 0; ci < 32; ++ci) {                // input channel = feature * 4 + phase (pixel_unshuffle)
-    const float x = f[ci >> 2][ci & 3];
+  for (int p = 0; p < 4; ++p) {
+    const float* row = feat + (16 * p + n) * kF32FeatRow + 8 * g;
+    const f4 lo = *reinterpret_cast<const f4*>(row), hi = *reinterpret_cast<const f4*>(row + 4);
+    f4 acc[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int co = 0; co < 32; ++co) acc[co] = fmaf(x, wp[ci * 32 + co], acc[co]);
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int T = 0; T < 2; ++T)
+        acc[T] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[T][j], j < 4 ? lo[j] : hi[j - 4], acc[T], 0, 0, 0);
+    const long o = first + 16 * p + n;
+    if (o < pixels) {
+#pragma unroll
+      for (int T = 0; T < 2; ++T) {
+        f4 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = leaky(acc[T][i] + bs[T][i], 0.1f);
+        *reinterpret_cast<f4*>(skip + o * 32 + 16 * T + 4 * g) = r;
+      }
+    }
   }
-  float* out = skip + (size_t)idx * 32;
-#pragma unroll
-  for (int co = 0; co < 32; co += 4)
-    *reinterpret_cast<float4*>(out + co) = make_float4(leaky01(acc[co] + wp[1024 + co]), leaky01(acc[co + 1] + wp[1025 + co]),
-                                                       leaky01(acc[co + 2] + wp[1026 + co]), leaky01(acc[co + 3] + wp[1027 + co]));
 }
 
 // ---- split products on the FP16 MFMA ----------------------------------------------------------------
@@ -521,8 +543,13 @@ __device__ __forceinline__ float clamp_coef(float a) {
 // Persistent blocks over tiles of 64 x 4 LR pixels, one row per wave, in two chunks of 32 pixels.  The filter
 // weights of a chunk's even and odd pixels are two MFMA products of 16 columns, as in k_head.hip: row 4g + i of
 // row tile t is (phase g, tap 4t + i), so accumulator lane (n, g) holds all 25 taps of phase g of pixels 2n and
-// 2n + 1, and [K_hi | K_lo] . [c ; c] runs once with the coefficients' lo and once with their hi halves on top
-// of the FP32 base (bank and base scaled by a power of two, the RGB tile by its inverse).
+// 2n + 1, with bank and coefficients in three FP16 parts each (exact),
+// [K_3 | K_hi] . [c_hi ; c_3] + [K_lo | K_hi] . [c_lo ; c_lo] + [K_lo | K_hi] . [c_hi ; c_hi], small terms
+// first, since the MFMA cuts off the bits of all terms below the largest of a pass; the FP32 base is added to
+// the sum, not taken as its first addend.  Against 64 bits (frames of 33 x 65 to 1080p) the output's error is
+// 1.21e-7 (area) and 1.20e-7 (DIV2K) where one FP32 FMA chain per weight gave 1.17e-7 and 1.26e-7; two parts
+// each gave 1.15e-7 and 1.36e-7, the base as first addend 1.22e-7 and 1.61e-7.  Bank and base are scaled by a
+// power of two, the RGB tile by its inverse.
 // The lane applies them with FP32 FMAs in tap order.  Two neighbouring pixels share 20 of their 25 window
 // positions: 30 LDS reads of 16 bytes instead of 50, which would take 46 us of LDS time at 1080p; the tile
 // holds even and odd columns apart, so that the lanes' reads are contiguous.  One thread per pixel took 168 us
@@ -589,12 +616,13 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __r
                                                                   F32HeadGeom G, unsigned* __restrict__ nonfinite) {
   __shared__ float4 tiles[2][2][kF32HPlane];                 // [buffer][column parity]
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, n = lane & 15, g = lane >> 4;
-  h8 A[7];
+  h8 A[7], A2[7];
   f4 base[7];
-  const f4* bf = reinterpret_cast<const f4*>(bank + 7 * 64);
+  const f4* bf = reinterpret_cast<const f4*>(bank + 14 * 64);
 #pragma unroll
   for (int t = 0; t < 7; ++t) {
     A[t] = bank[t * 64 + lane];
+    A2[t] = bank[(7 + t) * 64 + lane];
     base[t] = bf[g * 7 + t];
   }
   const size_t oplane = (size_t)4 * G.H * G.W;
@@ -627,13 +655,26 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __r
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const float4 c0 = coef[j][p][0], c1 = coef[j][p][1];
-        h8 hi, lo;
-        split8(make_float4(clamp_coef(c0.x), clamp_coef(c0.y), clamp_coef(c0.z), clamp_coef(c0.w)),
-               make_float4(clamp_coef(c1.x), clamp_coef(c1.y), clamp_coef(c1.z), clamp_coef(c1.w)), 1.f, hi, lo);
+        const float c[8] = {clamp_coef(c0.x), clamp_coef(c0.y), clamp_coef(c0.z), clamp_coef(c0.w),
+                            clamp_coef(c1.x), clamp_coef(c1.y), clamp_coef(c1.z), clamp_coef(c1.w)};
+        u4 hi, lo, third;
 #pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], lo, base[q]);
+        for (int e = 0; e < 4; ++e) {
+          hi[e] = pack_h2(c[2 * e], c[2 * e + 1]);
+          const float r0 = residual_lo(c[2 * e], hi[e]), r1 = residual_hi(c[2 * e + 1], hi[e]);
+          lo[e] = pack_h2(r0, r1);
+          const unsigned t = pack_h2(residual_lo(r0, lo[e]), residual_hi(r1, lo[e]));
+          third[e] = g < 2 ? hi[e] : t;
+        }
+        const h8 bh = __builtin_bit_cast(h8, hi), bl = __builtin_bit_cast(h8, lo), bt = __builtin_bit_cast(h8, third);
 #pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], hi, w[p][q]);
+        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A2[q], bt, f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], bl, w[p][q]);
+#pragma unroll
+        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], bh, w[p][q]);
+#pragma unroll
+        for (int q = 0; q < 7; ++q) w[p][q] += base[q];
       }
       float u[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
 #pragma unroll
@@ -679,8 +720,6 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __r
 }
 
 // ---- launchers ---------------------------------------------------------------------------------------
-static int f32_grid(long n) { return (int)((n + kF32Threads - 1) / kF32Threads); }
-
 static F32ConvTiles conv_tiles(int H, int W, int th, int batch) {
   F32ConvTiles G{H, W, (W + kConvTW - 1) / kConvTW, (H + th - 1) / th, 0};
   G.num = batch * G.tiles_x * G.tiles_y;
@@ -691,7 +730,7 @@ static hipError_t launch_grouped_t(const float* in, const F32Weights& W, int l, 
                                    hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hl, Wl, TH, batch);
   hipLaunchKernelGGL(f32_grouped_kernel<TH>, dim3(persistent_grid(G.num, cus), 2), dim3(kConvThreads), 0, stream, in,
-                     (const h8*)W.grouped[l], W.image + kF32Grouped + l * kF32GroupedStride + 18432, out, G,
+                     (const h8*)W.grouped[l], W.image + kF32BiasGrouped + 64 * l, out, G,
                      W.grouped_scale[l]);
   return hipGetLastError();
 }
@@ -706,7 +745,7 @@ static hipError_t launch_refine_t(const float* work, const F32Weights& W, float*
                                   hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hq, Wq, TH, batch);
   hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(persistent_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
-                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32Refine + 18432, W.image + kF32Tail + 4096, meta,
+                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32BiasRefine, W.image + kF32BiasTail, meta,
                      G, W.refine_scale, W.tail_scale);
   return hipGetLastError();
 }
@@ -724,11 +763,11 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
   const float* wimg = wts.image;
   const long packed = (long)batch * Hq * Wq, lowpx = (long)batch * Hl * Wl;
   if (in_fp32)
-    hipLaunchKernelGGL(f32_project_kernel<float>, dim3(f32_grid(packed)), dim3(kF32Threads), 0, stream,
-                       (const float*)src, wimg, skip, H, W, Hq, Wq, py, px, batch);
+    hipLaunchKernelGGL(f32_project_kernel<float>, dim3((unsigned)((packed + 63) / 64)), dim3(64), 0, stream,
+                       (const float*)src, wimg, skip, H, W, Hq, Wq, py, px, packed);
   else
-    hipLaunchKernelGGL(f32_project_kernel<_Float16>, dim3(f32_grid(packed)), dim3(kF32Threads), 0, stream,
-                       (const _Float16*)src, wimg, skip, H, W, Hq, Wq, py, px, batch);
+    hipLaunchKernelGGL(f32_project_kernel<_Float16>, dim3((unsigned)((packed + 63) / 64)), dim3(64), 0, stream,
+                       (const _Float16*)src, wimg, skip, H, W, Hq, Wq, py, px, packed);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[1], stream)) != hipSuccess) return e;
@@ -737,14 +776,14 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
   for (int i = 0; i < 5; ++i) dst[i] = lows ? lows[i] : (i % 2 ? low1 : low0);
   const int low_blocks = (int)std::min((lowpx + 63) / 64, 2L * cus);     // four groups of 16 pixels a block, persistent
   hipLaunchKernelGGL(f32_compress_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)skip,
-                     (const h8*)wts.compress, wimg + kF32Compress + 8192, dst[0], Hl, Wl, (int)lowpx, wts.compress_scale);
+                     (const h8*)wts.compress, wimg + kF32BiasCompress, dst[0], Hl, Wl, (int)lowpx, wts.compress_scale);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[2], stream)) != hipSuccess) return e;
   for (int l = 0; l < 4; ++l)
     if ((e = launch_f32_grouped(dst[l], wts, l, dst[l + 1], Hl, Wl, batch, cus, stream)) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[3], stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(f32_expand_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)dst[4],
-                     (const float*)skip, (const h8*)wts.expand, wimg + kF32Expand + 8192, work, Hl, Wl, (int)lowpx,
+                     (const float*)skip, (const h8*)wts.expand, wimg + kF32BiasExpand, work, Hl, Wl, (int)lowpx,
                      wts.expand_scale);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[4], stream)) != hipSuccess) return e;

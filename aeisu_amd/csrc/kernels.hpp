@@ -120,20 +120,15 @@ hipError_t launch_fused_tail_head(int in_fp32, int out_fp32, int qclamp, const v
                                   void* out, int H, int W, int Hq, int Wq, int py, int px, int batch,
                                   unsigned* nonfinite, int grid, hipStream_t stream);
 
-// FP32 policy (k_fp32.hip): per-layer kernels on FP32 NHWC activations.  Weight image (floats),
-// every layer [tap][ci][co] (co fastest) followed by its bias:
-//   project  W[32 feature channel f*4+phase][32] b[32]; compress W[128 skip channel c*4+phase][64] b[64];
-//   bottleneck l: W[9][32 group input][64] b[64] (output 32g+o reads group g's inputs);
-//   expand W[64][128] b[128] (output c*4+phase); refine W[9][32][64] b[64]; tail W[64][64] b[64];
-//   then the 24 analysis constants.
+// FP32 policy (k_fp32.hip): per-layer kernels on FP32 NHWC activations.  FP32 image (floats): the project's
+// W[32 feature channel f*4+phase][32 outputs] and b[32], the other layers' biases, the 24 analysis constants.
 constexpr int kF32Project = 0;
-constexpr int kF32Compress = kF32Project + 32 * 32 + 32;
-constexpr int kF32GroupedStride = 9 * 32 * 64 + 64;
-constexpr int kF32Grouped = kF32Compress + 128 * 64 + 64;
-constexpr int kF32Expand = kF32Grouped + 4 * kF32GroupedStride;
-constexpr int kF32Refine = kF32Expand + 64 * 128 + 128;
-constexpr int kF32Tail = kF32Refine + 9 * 32 * 64 + 64;
-constexpr int kF32Analysis = kF32Tail + 64 * 64 + 64;
+constexpr int kF32BiasCompress = kF32Project + 32 * 32 + 32;
+constexpr int kF32BiasGrouped = kF32BiasCompress + 64;
+constexpr int kF32BiasExpand = kF32BiasGrouped + 4 * 64;
+constexpr int kF32BiasRefine = kF32BiasExpand + 128;
+constexpr int kF32BiasTail = kF32BiasRefine + 64;
+constexpr int kF32Analysis = kF32BiasTail + 64;
 constexpr int kF32Floats = kF32Analysis + 24;
 // A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent, and an output's
 // magnitude is at most gain * (largest input magnitude) + offset.
@@ -146,8 +141,8 @@ struct F32Weights {
   const float* image;
   const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
-  const void* head;                        // 7 fragments [K_hi | K_lo] (row 4g + i of tile t: phase g, tap 4t + i), then
-                                           // the FP32 base float4 [g][t], both divided by head_unscale
+  const void* head;                        // fragments [K_lo | K_hi] x 7 (row 4g + i of tile t: phase g, tap 4t + i) and
+                                           // [K_3 | K_hi] x 7, the FP32 base float4 [g][t], all divided by head_unscale
   float head_unscale;
   F32SplitScale compress_scale, grouped_scale[4], expand_scale, refine_scale, tail_scale;
 };
