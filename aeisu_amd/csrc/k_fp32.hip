@@ -530,14 +530,15 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
 
 // ---- head: clamp, polyphase filter synthesis, 5x5 application, clip ----------------------------------
 // coefficient_clamp (aeisu/reconstruction.py:15-17) in FP32 with the reference's separate multiply
-// and add; a NaN coefficient stays NaN (so does the output, which raises the non-finite flag).
+// and add: sign(a) min(|a|, 2 + 0.05 (|a| - 2), 2.5), since the line lies above |a| up to 2 and below it
+// after.  gfx950's v_minimum3_f32 propagates NaN: a NaN coefficient stays NaN (so does the output, which raises
+// the non-finite flag).
 __device__ __forceinline__ float clamp_coef(float a) {
 #pragma clang fp contract(off)
-  const float m = fabsf(a);
-  if (m <= 2.f) return a;
-  float v = 2.f + 0.05f * (m - 2.f);
-  v = v > 2.5f ? 2.5f : v;
-  return copysignf(v, a);
+  const float v = 2.f + 0.05f * (fabsf(a) - 2.f);
+  float c;
+  asm("v_minimum3_f32 %0, |%1|, %2, %3" : "=v"(c) : "v"(a), "v"(v), "s"(2.5f));
+  return __builtin_copysignf(c, a);
 }
 
 // Persistent blocks over tiles of 64 x 4 LR pixels, one row per wave, in two chunks of 32 pixels.  The filter
@@ -562,11 +563,6 @@ struct F32HeadGeom {
   int H, W, Hq, Wq, py, px, tiles_x, tiles_y, num;
   float unscale;                                             // of the bank's power of two
 };
-template <typename Tin>
-struct F32HeadFetch {
-  Tin rgb[kF32HPer][3];
-  float4 coef[2][2][2];                                      // [chunk][pixel parity][half of the lane's eight]
-};
 struct F32HeadTile {
   int b, y0, x0;
 };
@@ -575,9 +571,8 @@ __device__ __forceinline__ F32HeadTile f32_head_tile(int tidx, const F32HeadGeom
   return {b, ty * kF32HH, (rem - ty * G.tiles_x) * kF32HW};
 }
 template <typename Tin>
-__device__ __forceinline__ void f32_head_fetch(F32HeadFetch<Tin>& f, const Tin* __restrict__ src,
-                                               const float* __restrict__ meta, F32HeadTile t, const F32HeadGeom& G, int tid,
-                                               int wave, int n, int g) {
+__device__ __forceinline__ void f32_head_rgb(Tin (&v)[kF32HPer][3], const Tin* __restrict__ src, F32HeadTile t,
+                                             const F32HeadGeom& G, int tid) {
   const size_t plane = (size_t)G.H * G.W;
   const Tin* s = src + (size_t)t.b * 3 * plane;
 #pragma unroll
@@ -585,20 +580,22 @@ __device__ __forceinline__ void f32_head_fetch(F32HeadFetch<Tin>& f, const Tin* 
     const int q = min(tid + kF32Threads * k, kF32HPos - 1), ly = q / kF32HLW, lx = q - ly * kF32HLW;
     const size_t o = (size_t)min(max(t.y0 + ly - 2, 0), G.H - 1) * G.W + min(max(t.x0 + lx - 2, 0), G.W - 1);
 #pragma unroll
-    for (int c = 0; c < 3; ++c) f.rgb[k][c] = s[c * plane + o];
+    for (int c = 0; c < 3; ++c) v[k][c] = s[c * plane + o];
   }
-  // pixels past the frame edge take the edge's coefficients (inside the tensor) and are not stored
-  const int Y = min(t.y0 + wave, G.H - 1) + G.py;
-  const float* row = meta + ((size_t)t.b * G.Hq + (Y >> 1)) * G.Wq * 64 + 32 * (Y & 1) + 8 * (g & 1);
+}
+// The lane's eight coefficients of pixels 2n and 2n + 1 of chunk j of the wave's row.  Pixels past the frame edge
+// take the edge's (inside the tensor) and are not stored.
+__device__ __forceinline__ void f32_head_coef(float4 (&c)[2][2], const float* __restrict__ meta, F32HeadTile t,
+                                              const F32HeadGeom& G, int j, int wave, int lane) {
+  const int n = lane & 15, Y = min(t.y0 + wave, G.H - 1) + G.py;
+  const float* row = meta + ((size_t)t.b * G.Hq + (Y >> 1)) * G.Wq * 64 + 32 * (Y & 1) + 8 * ((lane >> 4) & 1);
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int X = min(t.x0 + 32 * j + 2 * n + p, G.W - 1) + G.px;
-      const float* c = row + (size_t)(X >> 1) * 64 + 16 * (X & 1);
-      f.coef[j][p][0] = *reinterpret_cast<const float4*>(c);
-      f.coef[j][p][1] = *reinterpret_cast<const float4*>(c + 4);
-    }
+  for (int p = 0; p < 2; ++p) {
+    const int X = min(t.x0 + 32 * j + 2 * n + p, G.W - 1) + G.px;
+    const float* q = row + (size_t)(X >> 1) * 64 + 16 * (X & 1);
+    c[p][0] = *reinterpret_cast<const float4*>(q);
+    c[p][1] = *reinterpret_cast<const float4*>(q + 4);
+  }
 }
 // Output columns 4n .. 4n + 3 of a chunk row and channel: pixels 2n and 2n + 1, left and right.
 __device__ __forceinline__ void store_quad(float* p, float a, float b, float c, float d, bool second) {
@@ -611,26 +608,30 @@ __device__ __forceinline__ void store_quad(_Float16* p, float a, float b, float 
 }
 
 template <typename Tin, typename Tout>
-__global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __restrict__ src, const float* __restrict__ meta,
+__global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __restrict__ src, const float* __restrict__ meta,
                                                                   const h8* __restrict__ bank, Tout* __restrict__ out,
                                                                   F32HeadGeom G, unsigned* __restrict__ nonfinite) {
   __shared__ float4 tiles[2][2][kF32HPlane];                 // [buffer][column parity]
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, n = lane & 15, g = lane >> 4;
-  h8 A[7], A2[7];
-  f4 base[7];
-  const f4* bf = reinterpret_cast<const f4*>(bank + 14 * 64);
+  __shared__ h8 bank3[7 * 64];                               // the third parts' fragments and the base: kept in
+  __shared__ f4 base[4 * 7];                                 // registers they cost the third wave per SIMD
+  h8 A[7];
 #pragma unroll
-  for (int t = 0; t < 7; ++t) {
-    A[t] = bank[t * 64 + lane];
-    A2[t] = bank[(7 + t) * 64 + lane];
-    base[t] = bf[g * 7 + t];
-  }
+  for (int t = 0; t < 7; ++t) A[t] = bank[t * 64 + lane];
+  for (int i = tid; i < 7 * 64; i += kF32Threads) bank3[i] = bank[7 * 64 + i];
+  if (tid < 28) base[tid] = reinterpret_cast<const f4*>(bank + 14 * 64)[tid];
   const size_t oplane = (size_t)4 * G.H * G.W;
   float chk = 0.f;                                           // NaN once an output was not finite
   const int iters = tile_iters(G.num);
   int tidx = tile_of(0, G.num);
-  F32HeadFetch<Tin> f;
-  if (tidx < G.num) f32_head_fetch(f, src, meta, f32_head_tile(tidx, G), G, tid, wave, n, g);
+  // in flight: the next tile's RGB and the next chunk's coefficients (read as soon as the last ones are used)
+  Tin rgb[kF32HPer][3];
+  float4 coef[2][2];                                         // [pixel parity][half of the lane's eight]
+  if (tidx < G.num) {
+    const F32HeadTile t = f32_head_tile(tidx, G);
+    f32_head_rgb(rgb, src, t, G, tid);
+    f32_head_coef(coef, meta, t, G, 0, wave, lane);
+  }
   for (int it = 0; it < iters; ++it) {
     if (tidx >= G.num) break;                                // block-uniform
     const F32HeadTile t = f32_head_tile(tidx, G);
@@ -638,23 +639,26 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __r
 #pragma unroll
     for (int k = 0; k < kF32HPer; ++k) {
       const int q = tid + kF32Threads * k;                   // positions of a row alternate between the planes
-      if (q < kF32HPos) buf[q & 1][q >> 1] = make_float4((float)f.rgb[k][0] * G.unscale, (float)f.rgb[k][1] * G.unscale, (float)f.rgb[k][2] * G.unscale, 0.f);
+      if (q < kF32HPos) buf[q & 1][q >> 1] = make_float4((float)rgb[k][0] * G.unscale, (float)rgb[k][1] * G.unscale, (float)rgb[k][2] * G.unscale, 0.f);
     }
-    float4 coef[2][2][2];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) coef[i >> 2][(i >> 1) & 1][i & 1] = f.coef[i >> 2][(i >> 1) & 1][i & 1];
-    tidx = tile_of(it + 1, G.num);
-    if (it + 1 < iters && tidx < G.num) f32_head_fetch(f, src, meta, f32_head_tile(tidx, G), G, fresh(tid), wave, n, g);
+    const int next = tile_of(it + 1, G.num);
+    const bool more = it + 1 < iters && next < G.num;
+    tidx = more ? next : G.num;
+    const F32HeadTile tn = f32_head_tile(more ? next : 0, G);
+    if (more) f32_head_rgb(rgb, src, tn, G, fresh(tid));
     lds_barrier();                                           // buf complete; the other buffer is free again
     const int y = t.y0 + wave;
-    if (y >= G.H) continue;                                  // wave-uniform; the barriers are above
-#pragma unroll
+    if (y >= G.H) {                                          // wave-uniform; the barriers are above
+      if (more) f32_head_coef(coef, meta, tn, G, 0, wave, fresh(lane));
+      continue;
+    }
     for (int j = 0; j < 2; ++j) {
-      if (t.x0 + 32 * j >= G.W) break;                       // wave-uniform
+      const int lane_j = fresh(lane);
       f4 w[2][7];
+      h8 bh[2], bl[2], bt[2];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const float4 c0 = coef[j][p][0], c1 = coef[j][p][1];
+        const float4 c0 = coef[p][0], c1 = coef[p][1];
         const float c[8] = {clamp_coef(c0.x), clamp_coef(c0.y), clamp_coef(c0.z), clamp_coef(c0.w),
                             clamp_coef(c1.x), clamp_coef(c1.y), clamp_coef(c1.z), clamp_coef(c1.w)};
         u4 hi, lo, third;
@@ -663,19 +667,27 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_head_kernel(const Tin* __r
           hi[e] = pack_h2(c[2 * e], c[2 * e + 1]);
           const float r0 = residual_lo(c[2 * e], hi[e]), r1 = residual_hi(c[2 * e + 1], hi[e]);
           lo[e] = pack_h2(r0, r1);
-          const unsigned t = pack_h2(residual_lo(r0, lo[e]), residual_hi(r1, lo[e]));
-          third[e] = g < 2 ? hi[e] : t;
+          const unsigned t3 = pack_h2(residual_lo(r0, lo[e]), residual_hi(r1, lo[e]));
+          third[e] = (lane_j >> 4) < 2 ? hi[e] : t3;
         }
-        const h8 bh = __builtin_bit_cast(h8, hi), bl = __builtin_bit_cast(h8, lo), bt = __builtin_bit_cast(h8, third);
-#pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A2[q], bt, f4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], bl, w[p][q]);
-#pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] = mfma_f16(A[q], bh, w[p][q]);
-#pragma unroll
-        for (int q = 0; q < 7; ++q) w[p][q] += base[q];
+        bh[p] = __builtin_bit_cast(h8, hi);
+        bl[p] = __builtin_bit_cast(h8, lo);
+        bt[p] = __builtin_bit_cast(h8, third);
       }
+#pragma unroll
+      for (int q = 0; q < 7; ++q) {
+        const h8 a3 = bank3[q * 64 + lane_j];
+        const f4 bs = base[(lane_j >> 4) * 7 + q];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          w[p][q] = mfma_f16(a3, bt[p], f4{0.f, 0.f, 0.f, 0.f});
+          w[p][q] = mfma_f16(A[q], bl[p], w[p][q]);
+          w[p][q] = mfma_f16(A[q], bh[p], w[p][q]);
+          w[p][q] += bs;
+        }
+      }
+      if (j == 0) f32_head_coef(coef, meta, t, G, 1, wave, lane_j);
+      else if (more) f32_head_coef(coef, meta, tn, G, 0, wave, lane_j);
       float u[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
 #pragma unroll
       for (int dy = 0; dy < 5; ++dy)
@@ -798,7 +810,7 @@ hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const flo
                            hipStream_t stream) {
   F32HeadGeom G{H, W, Hq, Wq, py, px, (W + kF32HW - 1) / kF32HW, (H + kF32HH - 1) / kF32HH, 0, wts.head_unscale};
   G.num = batch * G.tiles_x * G.tiles_y;
-  const int grid = persistent_grid(G.num, 2 * cus);
+  const int grid = persistent_grid(G.num, 3 * cus);
 #define AEISU_F32_HEAD(TI, TO)                                                                                        \
   hipLaunchKernelGGL((f32_head_kernel<TI, TO>), dim3(grid), dim3(kF32Threads), 0, stream, (const TI*)src, meta,       \
                      (const h8*)wts.head, (TO*)out, G, nonfinite)
