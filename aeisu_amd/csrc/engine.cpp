@@ -870,6 +870,7 @@ static void prepare_device(int device) {
   if (device < 0 || device >= 64) fail(AEISU_ERR_HIP, "device ordinal out of range");
   if (g_prepared[device]) return;
   check_hip(fused_prepare(), "hipFuncSetAttribute(fused LDS)");
+  check_hip(refine_prepare(), "hipFuncSetAttribute(refine LDS)");
   check_hip(body_fused_prepare(), "hipFuncSetAttribute(fused body LDS)");
   check_hip(noalloc_scratch_init(device), "hipGetSymbolAddress(scratch)");
   g_prepared[device] = true;

@@ -159,6 +159,7 @@ hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const flo
 // Resident blocks per CU (occupancy), used to size the persistent grids.
 int head_blocks_per_cu(int in_fp32, int out_fp32, int qclamp);
 int project_blocks_per_cu(int in_fp32, int precise);
+hipError_t refine_prepare();
 int refine_blocks_per_cu();
 int body_blocks_per_cu(int kind, int mode);   // kind 0 compress, 1 grouped, 2 expand
 
