@@ -157,24 +157,38 @@ __device__ __forceinline__ void conv_weights(h8 (&A)[9][2][2], const h8* __restr
       for (int part = 0; part < 2; ++part) A[tap][T][part] = frag[(((2 * role + T) * 9 + tap) * 2 + part) * 64 + lane];
 }
 
-// One row of 16 pixels: acc[T] = sum over the 9 taps of the wave's two row tiles.  p: the lane's operand of
-// the top left tap.
-__device__ __forceinline__ void conv_row(const unsigned char* p, const h8 (&A)[9][2][2], f4 (&acc)[2]) {
-  f4 small[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
-  acc[0] = acc[1] = f4{0.f, 0.f, 0.f, 0.f};
+// R neighbouring rows of 16 pixels: acc[r][T] = sum over the 9 taps of the wave's two row tiles.  p: the lane's
+// operand of the first row's top left tap.  The rows share the operands of the input rows between them: R = 2
+// reads 24 pairs of operands from LDS instead of 36.
+template <int R>
+__device__ __forceinline__ void conv_rows(const unsigned char* p, const h8 (&A)[9][2][2], f4 (&acc)[R][2]) {
+  f4 small[R][2];
 #pragma unroll
-  for (int tap = 0; tap < 9; ++tap) {
-    const unsigned char* q = p + ((tap / 3) * kConvPW + tap % 3) * kConvPix;
-    const h8 bh = *reinterpret_cast<const h8*>(q), bl = *reinterpret_cast<const h8*>(q + 64);
+  for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int T = 0; T < 2; ++T) acc[T] = mfma_f16(A[tap][T][0], bh, acc[T]);
+    for (int T = 0; T < 2; ++T) acc[r][T] = small[r][T] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int T = 0; T < 2; ++T) small[T] = mfma_f16(A[tap][T][0], bl, small[T]);
+  for (int iy = 0; iy < R + 2; ++iy)
 #pragma unroll
-    for (int T = 0; T < 2; ++T) small[T] = mfma_f16(A[tap][T][1], bh, small[T]);
-  }
+    for (int dx = 0; dx < 3; ++dx) {
+      const unsigned char* q = p + (iy * kConvPW + dx) * kConvPix;
+      const h8 bh = *reinterpret_cast<const h8*>(q), bl = *reinterpret_cast<const h8*>(q + 64);
 #pragma unroll
-  for (int T = 0; T < 2; ++T) acc[T] += small[T];
+      for (int r = 0; r < R; ++r) {
+        if (iy - r < 0 || iy - r > 2) continue;
+        const int tap = 3 * (iy - r) + dx;
+#pragma unroll
+        for (int T = 0; T < 2; ++T) acc[r][T] = mfma_f16(A[tap][T][0], bh, acc[r][T]);
+#pragma unroll
+        for (int T = 0; T < 2; ++T) small[r][T] = mfma_f16(A[tap][T][0], bl, small[r][T]);
+#pragma unroll
+        for (int T = 0; T < 2; ++T) small[r][T] = mfma_f16(A[tap][T][1], bh, small[r][T]);
+      }
+    }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int T = 0; T < 2; ++T) acc[r][T] += small[r][T];
 }
 
 // The tile's largest finite magnitude over all waves, through `red` (one float per wave).  Ends with a
@@ -274,17 +288,19 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
     if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, tidx, TH, LY::Chunks, fresh(tid));
     lds_barrier();
     const float inv = inverse_scale(ex + sc.exponent);
-    for (int row = wave; row < TH; row += 4) {
-      f4 acc[2];
-      conv_row(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
-      const int y = y0 + row, x = x0 + n;
+    constexpr int R = TH / 4;                        // rows R wave .. R wave + R - 1
+    f4 acc[R][2];
+    conv_rows<R>(smem + (R * wave * kConvPW + n) * kConvPix + 16 * g, A, acc);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int y = y0 + R * wave + j, x = x0 + n;
       if (y < G.H && x < G.W) {
         float* d = out + (((size_t)b * G.H + y) * G.W + x) * 64 + 32 * grp + 4 * g;
 #pragma unroll
         for (int T = 0; T < 2; ++T) {
           f4 r;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[T][i], inv, bs[T][i]), 0.1f);
+          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[j][T][i], inv, bs[T][i]), 0.1f);
           *reinterpret_cast<f4*>(d + 16 * T) = r;
         }
       }
@@ -334,19 +350,23 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
     // |refine output| <= gain m + offset
     const int er = scale_exponent(fminf(fmaf(rs.gain, m, rs.offset), 0x1p126f));
     const float inv = inverse_scale(ex + rs.exponent), sr = pow2f(er);
-    for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); ++row) {
-      f4 acc[2];
-      conv_row(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
-      unsigned char* d = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
+    constexpr int R = TH >= 4 ? 2 : 1;
+    for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); row += R) {
+      f4 acc[R][2];
+      conv_rows<R>(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
 #pragma unroll
-      for (int T = 0; T < 2; ++T) {
-        float r[4];
+      for (int j = 0; j < R; ++j) {
+        unsigned char* d = smem + LY::SizeHalo + ((row + j) * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[T][i], inv, rb[T][i]), 0.1f) * sr;
-        u2 hi, lo;
-        split4(r[0], r[1], r[2], r[3], hi, lo);
-        *reinterpret_cast<u2*>(d + 32 * T) = hi;
-        *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
+        for (int T = 0; T < 2; ++T) {
+          float r[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[j][T][i], inv, rb[T][i]), 0.1f) * sr;
+          u2 hi, lo;
+          split4(r[0], r[1], r[2], r[3], hi, lo);
+          *reinterpret_cast<u2*>(d + 32 * T) = hi;
+          *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
+        }
       }
     }
     // the tail fragments are read for every tile: kept, they do not fit the 256 VGPRs
