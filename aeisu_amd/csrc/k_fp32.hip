@@ -617,13 +617,15 @@ __device__ __forceinline__ void f32_head_coef(float4 (&c)[2][2], const float* __
     c[p][1] = *reinterpret_cast<const float4*>(q + 4);
   }
 }
+// The output is written once and not read here: the non-temporal hint keeps it from displacing the coefficients
+// (1080p frame 352 -> 335 us).
 // Output columns 4n .. 4n + 3 of a chunk row and channel: pixels 2n and 2n + 1, left and right.
 __device__ __forceinline__ void store_quad(float* p, float a, float b, float c, float d, bool second) {
-  if (second) *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
+  if (second) __builtin_nontemporal_store(f4{a, b, c, d}, reinterpret_cast<f4*>(p));
   else *reinterpret_cast<float2*>(p) = make_float2(a, b);
 }
 __device__ __forceinline__ void store_quad(_Float16* p, float a, float b, float c, float d, bool second) {
-  if (second) *reinterpret_cast<u2*>(p) = u2{pack_h2(a, b), pack_h2(c, d)};
+  if (second) __builtin_nontemporal_store(u2{pack_h2(a, b), pack_h2(c, d)}, reinterpret_cast<u2*>(p));
   else *reinterpret_cast<unsigned*>(p) = pack_h2(a, b);
 }
 

@@ -109,15 +109,18 @@ __device__ __forceinline__ void head_fetch(HeadPrefetch<QC>& p, const Tin* __res
   }
 }
 
+// The output is written once and not read here: the non-temporal hint keeps it from displacing coefficients and
+// frames (1080p, frames and coefficients changing from call to call: 72.5 -> 60.6 us with FP32 output).
 template <typename Tout>
 __device__ __forceinline__ void store_pair(Tout* p, float left, float right);
 template <>
 __device__ __forceinline__ void store_pair<_Float16>(_Float16* p, float left, float right) {
-  *reinterpret_cast<unsigned*>(p) = pack_h2(left, right);
+  __builtin_nontemporal_store(pack_h2(left, right), reinterpret_cast<unsigned*>(p));
 }
 template <>
 __device__ __forceinline__ void store_pair<float>(float* p, float left, float right) {
-  *reinterpret_cast<float2*>(p) = make_float2(left, right);
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(f2v{left, right}, reinterpret_cast<f2v*>(p));
 }
 
 template <typename Tin, typename Tout, bool QC>
