@@ -159,7 +159,7 @@ __device__ __forceinline__ void conv_weights(h8 (&A)[9][2][2], const h8* __restr
 
 // R neighbouring rows of 16 pixels: acc[r][T] = sum over the 9 taps of the wave's two row tiles.  p: the lane's
 // operand of the first row's top left tap.  The rows share the operands of the input rows between them: R = 2
-// reads 24 pairs of operands from LDS instead of 36.
+// reads 24 operands from LDS instead of 36 (1080p: refine + tail 80 -> 78 us, a grouped layer 27 -> 25).
 template <int R>
 __device__ __forceinline__ void conv_rows(const unsigned char* p, const h8 (&A)[9][2][2], f4 (&acc)[R][2]) {
   f4 small[R][2];
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
 
 // refine 3x3 (32 -> 64) + LeakyReLU + tail 1x1 (64 -> 64).  One thread per pixel with FP32 FMAs was bound by
 // their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 86 and 9.5.  Its 210 MB take 41 us
-// of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (416 KB per tile), which
+// of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (320 KB per tile), which
 // two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
 // (scaled by a bound of their magnitude from the tile's input maximum and the weights) and wave w computes
 // tail channels 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
