@@ -770,9 +770,13 @@ static hipError_t launch_grouped_t(const float* in, const F32Weights& W, int l, 
 }
 static hipError_t launch_f32_grouped(const float* in, const F32Weights& W, int l, float* out, int Hl, int Wl, int batch,
                                      int cus, hipStream_t stream) {
-  // tiles of 8 rows where they fill the resident blocks (cus per conv group), else of 4 (one row per wave)
-  return conv_tiles(Hl, Wl, 8, batch).num >= cus ? launch_grouped_t<8>(in, W, l, out, Hl, Wl, batch, cus, stream)
-                                                 : launch_grouped_t<4>(in, W, l, out, Hl, Wl, batch, cus, stream);
+  // tiles of 8 or of 4 rows (one per wave), whichever takes less: rounds of the resident blocks (cus per conv group)
+  // times a tile's rows and about four for its halo, staging and barriers.  360 x 640: 143 tiles of 8 rows in one
+  // round where tiles of 4 rows take two, frame 87.9 -> 83.3 us; 256 x 256 keeps 90 tiles of 4 rows, 540p 8 rows.
+  auto cost = [&](int th) { return ((long)conv_tiles(Hl, Wl, th, batch).num + cus - 1) / cus * (th + 4); };
+  return cost(8) <= cost(4)
+             ? launch_grouped_t<8>(in, W, l, out, Hl, Wl, batch, cus, stream)
+             : launch_grouped_t<4>(in, W, l, out, Hl, Wl, batch, cus, stream);
 }
 template <int TH>
 static hipError_t launch_refine_t(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch, int cus,

@@ -78,8 +78,9 @@ def compare(model, state, frames):
     check("refine + tail", meta, ref, tb + through)
 
 
-# one tile and less, ragged tiles, tile multiples, many frames (the large-launch variants), one long row
-SIZES = [(1, 1, 1), (1, 33, 65), (2, 96, 128), (1, 97, 31), (40, 70, 90), (3, 150, 1030)]
+# one tile and less, ragged tiles, tile multiples, many frames (the large-launch variants), long rows, the grouped
+# layers' 8-row tiles in one round
+SIZES = [(1, 1, 1), (1, 33, 65), (2, 96, 128), (1, 97, 31), (40, 70, 90), (3, 150, 1030), (1, 350, 640)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
