@@ -930,7 +930,7 @@ static Geometry make_geometry(int mode, bool project_precise, int cus, int batch
   g.flags = flags;
   g.cus = cus;
   if (mode == kModeFp32) {
-    // per-layer FP32 kernels, one thread per pixel (no persistent grids, no fused variants)
+    // per-layer FP32 kernels (grids chosen at the launch, no fused variants)
     g.act_bytes = g.low_bytes = 4;
     g.nlow = (flags & AEISU_FLAG_KEEP_INTERMEDIATES) ? 5 : 2;
     return g;
