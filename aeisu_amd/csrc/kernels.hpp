@@ -136,14 +136,14 @@ struct F32SplitScale {
   int exponent;
   float gain, offset;
 };
+constexpr int kF32HeadBase = 7 * 64 * 4, kF32HeadFloats = kF32HeadBase + 4 * 7 * 4;
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
   const float* image;
   const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
-  const void* head;                        // fragments [K_lo | K_hi] x 7 (row 4g + i of tile t: phase g, tap 4t + i) and
-                                           // [K_3 | K_hi] x 7, the FP32 base float4 [g][t], all divided by head_unscale
-  float head_unscale;
+  const float* head;                       // FP32 bank [t][lane][K step] (row 4g + i of tile t: phase g, tap 4t + i; step j
+                                           // of lane group g: coefficient 4g + j), then the base float4 [g][t]
   F32SplitScale compress_scale, grouped_scale[4], expand_scale, refine_scale, tail_scale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage

@@ -143,3 +143,55 @@ def test_head_against_64_bits(model, size, dtypes):
         bound = bound + 2.0 ** -11 * ref.abs() + 2.0 ** -25
     over = (got - ref.clamp(0, 1)).abs() - bound
     assert over.max().item() <= 0, f"{over.max().item():.3g} over the bound"
+
+
+def chain(acc, pairs):
+    """acc + the products of `pairs`, one FP32 fused multiply-add after the other (a product of two FP32 values is
+    exact in 64 bits, where the sum's own rounding is 2^-29 of the FP32 one)."""
+    for a, b in pairs:
+        acc = (acc.double() + a.double() * b.double()).float()
+    return acc
+
+
+def head_chain(padded, meta, base, basis, y0, x0, h, w):
+    """The head of an h x w frame at (y0, x0) of its padded grid with one FP32 FMA chain per filter weight (the
+    base added last) and per output."""
+    c = F.pixel_shuffle(meta.view(meta.shape[0], 4, 16, *meta.shape[2:]).transpose(1, 2).flatten(1, 2), 2)
+    c = c[..., y0:y0 + h, x0:x0 + w]
+    mag = c.abs()
+    c = torch.where(mag <= 2, c, torch.sign(c) * (2 + 0.05 * (mag - 2)).clamp(max=2.5))
+    src = padded[..., y0 - 2:y0 + h + 2, x0 - 2:x0 + w + 2]
+    phases = []
+    for ph in range(4):
+        u = torch.zeros(c.shape[0], 3, h, w)
+        for tap in range(25):
+            wt = chain(torch.zeros(c.shape[0], 1, h, w), ((c[:, k:k + 1], basis[tap, k, ph]) for k in range(16)))
+            wt = wt + base[tap, ph]
+            u = chain(u, [(wt, src[..., tap // 5:tap // 5 + h, tap % 5:tap % 5 + w])])
+        phases.append(u)
+    return F.pixel_shuffle(torch.stack(phases, 2).flatten(1, 2), 2).clamp(0, 1)
+
+
+def test_head_no_further_from_64_bits_than_fma_chains(model):
+    """The error over a whole frame, not only a bound of every value: its norm is at most that of FP32 FMA chains
+    (0.98 of it on the GPU), and its mean is zero, as rounding to nearest leaves it.  An error of some 5e-8 in each of
+    270,000 outputs, alike over the windows of about 100 of them, has a mean of 1e-9 by chance; sums that cut bits
+    off instead of rounding shift it by 1.3e-8."""
+    from aeisu_amd import _lib as L
+    from aeisu_amd import frames as scenes
+    m, state = model
+    h, w = 150, 150
+    print("case: FP32 head against FMA chains", flush=True)
+    frames = scenes.scene(h, w, 11, texture=True)[None].float()
+    flags = L.FLAG_KEEP_INTERMEDIATES
+    got = m.run(frames.cuda(), flags=flags).cpu()
+    hd = m.handle(1, h, w, torch.float32, torch.float32, flags)
+    _, _, _, _, hq, wq = m.geometry(hd)
+    meta = m.intermediate(hd, L.BUF_META).cpu().view(torch.float32).reshape(1, hq, wq, 64).permute(0, 3, 1, 2)
+    padded = pad_frame(frames)
+    ref = crop_output(M.reconstruct(padded.double(), meta.double(), state["base"].double(), state["basis"].double()), h, w).clamp(0, 1)
+    one = head_chain(padded, meta, state["base"], state["basis"], 16 + -h % 32 // 2, 16 + -w % 32 // 2, h, w)
+    ours, theirs = got.double() - ref, one.double() - ref
+    print(f"  error norm {ours.norm():.4g}, FMA chains {theirs.norm():.4g}; mean {ours.mean():.3g}, {theirs.mean():.3g}", flush=True)
+    assert ours.norm() <= theirs.norm()
+    assert ours.mean().abs() <= 3e-9
