@@ -526,22 +526,11 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   // `chunks`, row m, slot s is the weight at(f, m, s); the fragment order is chunk, then hi and lo
   auto split = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, int chunks, auto at, DeviceBuffer& dst) {
     const float* w = w32(l, cout, cin, ks);
-    const float* b = a.need(l + ".bias", kF32, {cout}).f32();
-    double top = 0, gain = 0, offset = 0;
     const size_t per = size_t(cin) * ks * ks;
-    for (uint32_t o = 0; o < cout; ++o) {
-      double sum = 0;
-      for (size_t i = 0; i < per; ++i) {
-        top = std::max(top, std::fabs((double)w[o * per + i]));
-        sum += std::fabs((double)w[o * per + i]);
-      }
-      gain = std::max(gain, sum);
-      offset = std::max(offset, std::fabs((double)b[o]));
-    }
+    float top = 0.f;
+    for (size_t i = 0; i < cout * per; ++i) top = std::max(top, std::fabs(w[i]));
     F32SplitScale sc;
     sc.exponent = top > 0 ? std::min(std::max(14 - std::ilogb(top), -60), 24) : 0;
-    sc.gain = (float)(1.001 * gain);
-    sc.offset = (float)(1.001 * offset);
     dst.upload(pack_frags<uint16_t>(2 * chunks, 8, [&](int f, int m, int s) {
       const float v = std::ldexp(w[at(f / 2, m, s)], sc.exponent);
       const uint16_t hi = f32_to_f16_bits(v);

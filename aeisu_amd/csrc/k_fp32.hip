@@ -19,6 +19,7 @@
 namespace aeisu {
 
 constexpr int kF32Threads = 256;
+typedef float f2 __attribute__((ext_vector_type(2)));
 
 template <typename T>
 __device__ __forceinline__ float to_f32(T v) { return (float)v; }
@@ -105,8 +106,11 @@ __global__ __launch_bounds__(64) void f32_project_kernel(const Tin* __restrict__
 // against 64 bits: coefficients 0.72 to 0.98 of the chain's error).  The cross terms go to an accumulator
 // of their own: added to the main sum they would be rounded at its magnitude.
 //
-// The scale keeps FP32's range: the largest magnitude of the tile (finite values only) goes to
-// [2^14, 2^15), so nothing overflows FP16, and a value is cut off at 2^-38 of the tile's largest.
+// The scale keeps FP32's range: the largest magnitude that shares it goes to [2^14, 2^15), so nothing overflows
+// FP16, and the lo halves end at 2^-39 of that.  The 1x1 layers and the tail take a scale per pixel.  The 3x3 layers
+// take the tile's largest (finite) pixel, and pixels below 2^-14 of it in a pass of their own with their own
+// scale (bands): a pixel's values are thus held to 2^-22 of themselves or 2^-25 of its largest, whatever lies
+// beside it.
 __device__ __forceinline__ float residual_lo(float v, unsigned w) {   // v - (low half of w), exact
   float r;
   asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
@@ -133,11 +137,30 @@ __device__ __forceinline__ float finite_abs(float v) {
   return a < __builtin_inff() ? a : 0.f;
 }
 __device__ __forceinline__ float inverse_scale(int e) { return pow2f(-min(max(e, -126), 126)); }
-__device__ __forceinline__ float wave_max(float m) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-  return m;
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
 }
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor8 = 0x128;
+// Magnitudes are compared as the bits of non-negative floats.
+__device__ __forceinline__ unsigned max_of_8(unsigned m) {   // over 8 neighbouring lanes
+  m = max(m, dpp<kDppXor1>(m));
+  m = max(m, dpp<kDppXor2>(m));
+  return max(m, dpp<kDppHalfMirror>(m));
+}
+__device__ __forceinline__ unsigned max_of_rows(unsigned m) {   // over the lanes n, n + 16, n + 32, n + 48
+  unsigned a = m, b = m;
+  permlane16_swap_u(a, b);
+  a = b = max(a, b);
+  permlane32_swap_u(a, b);
+  return max(a, b);
+}
+__device__ __forceinline__ unsigned max_of_wave(unsigned m) {
+  m = max_of_8(m);
+  return max_of_rows(max(m, dpp<kDppRor8>(m)));
+}
+__device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ unsigned as_bits(float v) { return __builtin_bit_cast(unsigned, v); }
 
 // ---- 3x3 layers: persistent blocks of four waves over tiles of 16 x TH pixels -----------------------
 // A wave serves 32 output channels (two MFMA row tiles) of some of the tile's pixel rows and keeps their 36
@@ -191,22 +214,12 @@ __device__ __forceinline__ void conv_rows(const unsigned char* p, const h8 (&A)[
     for (int T = 0; T < 2; ++T) acc[r][T] += small[r][T];
 }
 
-// The tile's largest finite magnitude over all waves, through `red` (one float per wave).  Ends with a
-// block barrier, before which every wave has left the previous tile's LDS data.
-__device__ __forceinline__ float block_max(float m, float* red, int wave, int lane) {
-  m = wave_max(m);
-  if (lane == 0) red[wave] = m;
-  lds_barrier();
-  const float4 r = *reinterpret_cast<const float4*>(red);
-  return fmaxf(fmaxf(r.x, r.y), fmaxf(r.z, r.w));
-}
-
 template <int TH>
 struct ConvLayout {
   static constexpr int Rows = TH + 2, Chunks = Rows * kConvPW * 8;   // float4 chunks of the halo
   static constexpr int Per = (Chunks + kConvThreads - 1) / kConvThreads;
   static constexpr int SizeHalo = Rows * kConvPW * kConvPix;
-  static constexpr int RPix = 272;                   // refine outputs: 64 channels hi, 64 lo, pad
+  static constexpr int RPix = 272;                   // refine outputs: 64 channels hi, 64 lo, two inverse scales, pad
   static constexpr int LdsRefine = SizeHalo + TH * kConvTW * RPix;
 };
 struct F32ConvTiles {
@@ -228,19 +241,84 @@ __device__ __forceinline__ void conv_fetch(float4 (&v)[PER], const float* __rest
     if (in_grid) v[k] = *reinterpret_cast<const float4*>(f + ((size_t)y * G.W + x) * CH + 4 * c);
   }
 }
+__device__ __forceinline__ float abs_max(float4 v) {
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+__device__ __forceinline__ float finite_max(float4 v) {
+  return fmaxf(fmaxf(finite_abs(v.x), finite_abs(v.y)), fmaxf(finite_abs(v.z), finite_abs(v.w)));
+}
 template <int PER>
 __device__ __forceinline__ float chunk_max(const float4 (&v)[PER]) {
   float m = 0.f;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) m = fmaxf(m, fmaxf(fmaxf(fabsf(v[k].x), fabsf(v[k].y)), fmaxf(fabsf(v[k].z), fabsf(v[k].w))));
+  for (int k = 0; k < PER; ++k) m = fmaxf(m, abs_max(v[k]));
   if (!(m < __builtin_inff())) {                     // an infinity somewhere: the largest finite value
     m = 0.f;
 #pragma unroll
-    for (int k = 0; k < PER; ++k)
-      m = fmaxf(m, fmaxf(fmaxf(finite_abs(v[k].x), finite_abs(v[k].y)), fmaxf(finite_abs(v[k].z), finite_abs(v[k].w))));
+    for (int k = 0; k < PER; ++k) m = fmaxf(m, finite_max(v[k]));
   }
   return m;
 }
+// Largest magnitude of a set of pixels and smallest that is not zero (infinite if there is none).
+struct PixelRange {
+  float top, bottom;
+};
+// Over the block (uniform); through `red`, 8 words.  Holds a block barrier, before which every wave has left the LDS
+// data of the tile or band before.  bottom: bits - 1, so that zeros count as the largest.
+__device__ __forceinline__ PixelRange block_range(unsigned top, unsigned bottom, unsigned* red, int wave, int lane) {
+  top = max_of_wave(top);
+  bottom = ~max_of_wave(~bottom);
+  if (lane == 0) {
+    red[wave] = top;
+    red[4 + wave] = bottom;
+  }
+  lds_barrier();
+  const u4 t = *reinterpret_cast<const u4*>(red), b = *reinterpret_cast<const u4*>(red + 4);
+  top = __builtin_amdgcn_readfirstlane(max(max(t[0], t[1]), max(t[2], t[3])));
+  bottom = __builtin_amdgcn_readfirstlane(min(min(b[0], b[1]), min(b[2], b[3])));
+  return {as_float(top), bottom == 0xffffffffu ? __builtin_inff() : as_float(bottom + 1u)};
+}
+// A tile's pixels are staged in bands, magnitudes from a band's largest down to kBand of it: a band's pixels share a
+// scale, the others are staged as zeros, and each band's products are added to the sums.  A pixel's magnitude is
+// its largest finite value (8 lanes hold a pixel); it is zero for zeros, infinities and NaN alone.
+constexpr float kBand = 0x1p-14f;
+template <int PER>
+__device__ __forceinline__ PixelRange range_below(const float4 (&v)[PER], float cap, unsigned* red, int wave, int lane) {
+  unsigned top = 0u, bottom = 0xffffffffu;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const unsigned p = max_of_8(as_bits(finite_max(v[k])));
+    if (as_float(p) < cap) {
+      top = max(top, p);
+      bottom = min(bottom, p - 1u);
+    }
+  }
+  return block_range(top, bottom, red, wave, lane);
+}
+template <int PER>
+__device__ __forceinline__ void keep_band(float4 (&v)[PER], float low, float cap) {
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const float p = as_float(max_of_8(as_bits(finite_max(v[k]))));
+    if (p > 0.f && (p < low || p >= cap)) v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+}
+// The whole tile's range; of its chunks of four channels where they all lie in one band, as nearly always, since that
+// takes no exchange between the lanes of a pixel.  red: 16 words.
+template <int PER>
+__device__ __forceinline__ PixelRange tile_range(const float4 (&v)[PER], unsigned* red, int wave, int lane) {
+  unsigned top = 0u, bottom = 0xffffffffu;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const unsigned m = as_bits(abs_max(v[k]));
+    top = max(top, m);
+    bottom = min(bottom, m - 1u);
+  }
+  const PixelRange r = block_range(top, bottom, red, wave, lane);
+  if (r.top < __builtin_inff() && r.bottom >= r.top * kBand) return r;
+  return range_below<PER>(v, __builtin_inff(), red + 8, wave, lane);
+}
+
 // Splits the staged chunks into LDS: hi halves of a pixel's 32 channels first, lo halves after.
 template <int PER>
 __device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char* lds, float s, int chunks, int tid) {
@@ -266,7 +344,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
                                                                       F32ConvTiles G, F32SplitScale sc) {
   typedef ConvLayout<TH> LY;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LY::SizeHalo];
-  __shared__ __attribute__((aligned(16))) float red[4];
+  __shared__ __attribute__((aligned(16))) unsigned red[16];
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, grp = blockIdx.y;
   const int n = lane & 15, g = lane >> 4;
   float4 v[LY::Per];
@@ -282,29 +360,44 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
     if (tidx >= G.num) break;                        // block-uniform
     const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per;
     const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
-    const int ex = scale_exponent(block_max(chunk_max(v), red, wave, lane));
-    conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
-    tidx = tile_of(it + 1, G.num);
-    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, tidx, TH, LY::Chunks, fresh(tid));
-    lds_barrier();
-    const float inv = inverse_scale(ex + sc.exponent);
-    constexpr int R = TH / 4;                        // rows R wave .. R wave + R - 1
-    f4 acc[R][2];
-    conv_rows<R>(smem + (R * wave * kConvPW + n) * kConvPix + 16 * g, A, acc);
+    const int next = tile_of(it + 1, G.num);
+    PixelRange rg = tile_range(v, red, wave, lane);
+    for (float cap = __builtin_inff();;) {           // over the tile's bands: one but for tiles with outliers
+      const float low = rg.top * kBand;
+      const bool first = cap == __builtin_inff(), last = rg.bottom >= low;
+      const int ex = scale_exponent(rg.top);
+      if (!(first && last)) keep_band<LY::Per>(v, low, cap);
+      conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
+      if (last && it + 1 < iters && next < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, next, TH, LY::Chunks, fresh(tid));
+      lds_barrier();
+      const float inv = inverse_scale(ex + sc.exponent);
+      constexpr int R = TH / 4;                      // rows R wave .. R wave + R - 1
+      f4 acc[R][2];
+      conv_rows<R>(smem + (R * wave * kConvPW + n) * kConvPix + 16 * g, A, acc);
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const int y = y0 + R * wave + j, x = x0 + n;
-      if (y < G.H && x < G.W) {
-        float* d = out + (((size_t)b * G.H + y) * G.W + x) * 64 + 32 * grp + 4 * g;
+      for (int j = 0; j < R; ++j) {
+        const int y = y0 + R * wave + j, x = x0 + n;
+        if (y < G.H && x < G.W) {
+          float* d = out + (((size_t)b * G.H + y) * G.W + x) * 64 + 32 * grp + 4 * g;
 #pragma unroll
-        for (int T = 0; T < 2; ++T) {
-          f4 r;
+          for (int T = 0; T < 2; ++T) {
+            f4 r = bs[T];
+            if (!first) r = *reinterpret_cast<const f4*>(d + 16 * T);   // the sum so far
 #pragma unroll
-          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[j][T][i], inv, bs[T][i]), 0.1f);
-          *reinterpret_cast<f4*>(d + 16 * T) = r;
+            for (int i = 0; i < 4; ++i) {
+              r[i] = fmaf(acc[j][T][i], inv, r[i]);
+              if (last) r[i] = leaky(r[i], 0.1f);
+            }
+            *reinterpret_cast<f4*>(d + 16 * T) = r;
+          }
         }
       }
+      if (last) break;
+      cap = low;
+      conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, tidx, TH, LY::Chunks, fresh(tid));
+      rg = range_below<LY::Per>(v, cap, red + 8, wave, lane);
     }
+    tidx = next;
   }
 }
 
@@ -312,8 +405,8 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
 // their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 86 and 9.5.  Its 210 MB take 41 us
 // of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (320 KB per tile), which
 // two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
-// (scaled by a bound of their magnitude from the tile's input maximum and the weights) and wave w computes
-// tail channels 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
+// (a scale for each pixel's 32 channels of a wave, kept beside them) and wave w computes tail channels
+// 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
 template <int TH>
 __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const float* __restrict__ work,
                                                                           const h8* __restrict__ rfrag,
@@ -324,50 +417,81 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
                                                                           F32SplitScale rs, F32SplitScale ts) {
   typedef ConvLayout<TH> LY;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LY::LdsRefine];
-  __shared__ __attribute__((aligned(16))) float red[4];
+  __shared__ __attribute__((aligned(16))) unsigned red[16];
+  __shared__ __attribute__((aligned(16))) float rb[64], tb[64];   // biases: in registers the kernel spills
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, role = wave & 1, half = wave >> 1;
-  const int n = lane & 15, g = lane >> 4;
   float4 v[LY::Per];
+  if (tid < 64) rb[tid] = rbias[tid];
+  else if (tid < 128) tb[tid - 64] = tbias[tid - 64];
   int tidx = tile_of(0, G.num);
   if (tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
   h8 A[9][2][2];
   conv_weights(A, rfrag, role, lane);
-  f4 rb[2];
-#pragma unroll
-  for (int T = 0; T < 2; ++T) rb[T] = *reinterpret_cast<const f4*>(rbias + 32 * role + 16 * T + 4 * g);
-  const f4 tb = *reinterpret_cast<const f4*>(tbias + 16 * wave + 4 * g);
   const int iters = tile_iters(G.num);
   for (int it = 0; it < iters; ++it) {
     if (tidx >= G.num) break;                        // block-uniform
     const int per = G.tiles_x * G.tiles_y, b = tidx / per, rem = tidx - b * per;
     const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
-    const float m = block_max(chunk_max(v), red, wave, lane);
-    const int ex = scale_exponent(m);
-    conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
-    tidx = tile_of(it + 1, G.num);
-    if (it + 1 < iters && tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, fresh(tid));
-    lds_barrier();
-    // |refine output| <= gain m + offset
-    const int er = scale_exponent(fminf(fmaf(rs.gain, m, rs.offset), 0x1p126f));
-    const float inv = inverse_scale(ex + rs.exponent), sr = pow2f(er);
-    constexpr int R = TH >= 4 ? 2 : 1;
-    for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); row += R) {
-      f4 acc[R][2];
-      conv_rows<R>(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
+    const int next = tile_of(it + 1, G.num);
+    PixelRange rg = tile_range(v, red, wave, lane);
+    for (float cap = __builtin_inff();;) {           // over the tile's bands
+      const float low = rg.top * kBand;
+      const bool first = cap == __builtin_inff(), last = rg.bottom >= low;
+      const int ex = scale_exponent(rg.top);
+      if (!(first && last)) keep_band<LY::Per>(v, low, cap);
+      conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
+      if (last && it + 1 < iters && next < G.num) conv_fetch<LY::Per, 32>(v, work, G, next, TH, LY::Chunks, fresh(tid));
+      lds_barrier();
+      const float inv = inverse_scale(ex + rs.exponent);
+      constexpr int R = TH >= 4 ? 2 : 1;
+      for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); row += R) {
+        const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
+        f4 acc[R][2];
+        conv_rows<R>(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        unsigned char* d = smem + LY::SizeHalo + ((row + j) * kConvTW + n) * LY::RPix + 64 * role + 8 * g;
+        for (int j = 0; j < R; ++j) {
+          unsigned char* pix = smem + LY::SizeHalo + ((row + j) * kConvTW + n) * LY::RPix;
+          unsigned char* d = pix + 64 * role + 8 * g;
+          f4 r[2];
+          float m = 0.f;
 #pragma unroll
-        for (int T = 0; T < 2; ++T) {
-          float r[4];
+          for (int T = 0; T < 2; ++T) {
+            r[T] = *reinterpret_cast<const f4*>(rb + 32 * role + 16 * T + 4 * g);
+            if (!first) {                            // the sum so far
+              const f2 a = *reinterpret_cast<const f2*>(d + 32 * T), c = *reinterpret_cast<const f2*>(d + 32 * T + 128);
+              r[T] = f4{a[0], a[1], c[0], c[1]};
+            }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[j][T][i], inv, rb[T][i]), 0.1f) * sr;
-          u2 hi, lo;
-          split4(r[0], r[1], r[2], r[3], hi, lo);
-          *reinterpret_cast<u2*>(d + 32 * T) = hi;
-          *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
+            for (int i = 0; i < 4; ++i) {
+              r[T][i] = fmaf(acc[j][T][i], inv, r[T][i]);
+              if (last) r[T][i] = leaky(r[T][i], 0.1f);
+              m = fmaxf(m, fabsf(r[T][i]));
+            }
+          }
+          if (last) {
+            const int er = scale_exponent(as_float(max_of_rows(as_bits(m))));   // of the pixel's 32 channels in this wave
+            const float s = pow2f(er);
+#pragma unroll
+            for (int T = 0; T < 2; ++T) {
+              u2 hi, lo;
+              split4(r[T][0] * s, r[T][1] * s, r[T][2] * s, r[T][3] * s, hi, lo);
+              *reinterpret_cast<u2*>(d + 32 * T) = hi;
+              *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
+            }
+            if (g == 0) *reinterpret_cast<float*>(pix + 256 + 4 * role) = inverse_scale(er + ts.exponent);
+          } else {
+#pragma unroll
+            for (int T = 0; T < 2; ++T) {
+              *reinterpret_cast<f2*>(d + 32 * T) = f2{r[T][0], r[T][1]};
+              *reinterpret_cast<f2*>(d + 32 * T + 128) = f2{r[T][2], r[T][3]};
+            }
+          }
         }
       }
+      if (last) break;
+      cap = low;
+      conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, fresh(tid));
+      rg = range_below<LY::Per>(v, cap, red + 8, wave, lane);
     }
     // the tail fragments are read for every tile: kept, they do not fit the 256 VGPRs
     h8 At[2][2];
@@ -377,26 +501,29 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
 #pragma unroll
       for (int part = 0; part < 2; ++part) At[k][part] = tf[(k * 2 + part) * 64];
     lds_barrier();
-    const float tinv = inverse_scale(er + ts.exponent);
 #pragma unroll 2
     for (int row = 0; row < TH; ++row) {
-      const unsigned char* p = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix + 16 * g;
-      f4 acc = {0.f, 0.f, 0.f, 0.f}, small = {0.f, 0.f, 0.f, 0.f};
+      const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
+      const unsigned char* pix = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix;
+      f4 acc[2];                                     // K chunk k: channels 32 k .. + 31, which share a scale
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        const h8 bh = *reinterpret_cast<const h8*>(p + 64 * k), bl = *reinterpret_cast<const h8*>(p + 64 * k + 128);
-        acc = mfma_f16(At[k][0], bh, acc);
-        small = mfma_f16(At[k][0], bl, small);
-        small = mfma_f16(At[k][1], bh, small);
+        const h8 bh = *reinterpret_cast<const h8*>(pix + 16 * g + 64 * k), bl = *reinterpret_cast<const h8*>(pix + 16 * g + 64 * k + 128);
+        f4 small = mfma_f16(At[k][0], bl, f4{0.f, 0.f, 0.f, 0.f});
+        acc[k] = mfma_f16(At[k][0], bh, f4{0.f, 0.f, 0.f, 0.f});
+        acc[k] += mfma_f16(At[k][1], bh, small);
       }
+      const float2 inv = *reinterpret_cast<const float2*>(pix + 256);
+      const f4 bias = *reinterpret_cast<const f4*>(tb + 16 * wave + 4 * g);
       const int qy = y0 + row, qx = x0 + n;
       if (qy < G.H && qx < G.W) {
         f4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = fmaf(acc[i] + small[i], tinv, tb[i]);
+        for (int i = 0; i < 4; ++i) o[i] = fmaf(acc[0][i], inv.x, fmaf(acc[1][i], inv.y, bias[i]));
         *reinterpret_cast<f4*>(meta + (((size_t)b * G.H + qy) * G.W + qx) * 64 + 16 * wave + 4 * g) = o;
       }
     }
+    tidx = next;
   }
 }
 
@@ -405,10 +532,6 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
 // (32 contiguous bytes), splits them in registers, and the pixel's scale comes from the four lanes that hold
 // its channels.  All 32 weight fragments stay in registers (128 VGPRs).  The next group's loads are in flight
 // during the products.
-__device__ __forceinline__ float pixel_max(float m) {    // over the lanes n, n + 16, n + 32, n + 48
-  m = fmaxf(m, __shfl_xor(m, 16));
-  return fmaxf(m, __shfl_xor(m, 32));
-}
 __device__ __forceinline__ void split8(float4 a, float4 b, float s, h8& hi, h8& lo) {
   u2 h0, l0, h1, l1;
   split4(a.x * s, a.y * s, a.z * s, a.w * s, h0, l0);
@@ -457,7 +580,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
       for (int part = 0; part < 2; ++part) A[T][k][part] = frag[((T * 4 + k) * 2 + part) * 64 + lane];
   }
   for (; grp < groups; grp += waves) {
-    const int ex = scale_exponent(pixel_max(chunk_max(v)));
+    const int ex = scale_exponent(as_float(max_of_rows(as_bits(chunk_max(v)))));
     const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
     h8 bh[4], bl[4];
 #pragma unroll
@@ -524,7 +647,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
     f4 sk[8];
 #pragma unroll
     for (int T = 0; T < 8; ++T) sk[T] = *reinterpret_cast<const f4*>(skip + at(T));
-    const int ex = scale_exponent(pixel_max(chunk_max(v)));
+    const int ex = scale_exponent(as_float(max_of_rows(as_bits(chunk_max(v)))));
     const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
     h8 bh[2], bl[2];
 #pragma unroll

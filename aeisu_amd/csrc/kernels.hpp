@@ -130,11 +130,9 @@ constexpr int kF32BiasRefine = kF32BiasExpand + 128;
 constexpr int kF32BiasTail = kF32BiasRefine + 64;
 constexpr int kF32Analysis = kF32BiasTail + 64;
 constexpr int kF32Floats = kF32Analysis + 24;
-// A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent, and an output's
-// magnitude is at most gain * (largest input magnitude) + offset.
+// A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent.
 struct F32SplitScale {
   int exponent;
-  float gain, offset;
 };
 constexpr int kF32HeadBase = 7 * 64 * 4, kF32HeadFloats = kF32HeadBase + 4 * 7 * 4;
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).

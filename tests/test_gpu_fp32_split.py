@@ -116,6 +116,37 @@ def test_nonfinite_input_stays_local(model, bad):
     assert (got - clean).abs()[..., far].max().item() <= 2e-5
 
 
+# the second size takes the large-launch variants
+@pytest.mark.parametrize("size", [(1, 80, 150), (3, 150, 1030)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("value", [1e4, 1e6, 1e8, -1e12, 1e30])
+def test_finite_outlier_stays_local(model, size, value):
+    """A large finite pixel leaves the pixels that it cannot reach (32 or more away) at their values but for the
+    rounding of splits with another scale (2^-22 or so, as between regions of upscale())."""
+    m, _ = model
+    print(f"case: FP32 frames {size} with one pixel at {value:g}", flush=True)
+    b, h, w = size
+    frames = torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(7))
+    clean = m.run(frames.cuda(), check_finite=False).cpu()
+    y, x = h // 2, w // 2
+    frames[b // 2, 1, y, x] = value
+    got = m.run(frames.cuda(), check_finite=False).cpu()
+    far = torch.ones(b, 1, 2 * h, 2 * w, dtype=torch.bool)
+    far[b // 2, :, max(0, 2 * (y - 32)):2 * (y + 33), 2 * (x - 32):2 * (x + 33)] = False
+    assert ((got - clean).abs() * far).max().item() <= 4e-6
+
+
+@pytest.mark.parametrize("size", [(1, 45, 70), (3, 150, 1030)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("values", [(1e8,), (-1e12, 3e5), (1e30, 1e-30, 1e10)], ids=str)
+def test_stages_with_outliers(model, size, values):
+    """Pixels far apart in magnitude within a tile: every stage within the bound of each pixel's own window."""
+    print(f"case: FP32 stages {size} with pixels at {values}", flush=True)
+    b, h, w = size
+    frames = torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(9))
+    for i, v in enumerate(values):
+        frames[0, :, h // 2 + 9 * i, w // 2 - 13 * i] = v
+    compare(*model, frames)
+
+
 @pytest.mark.parametrize("dtypes", [("f32", "f32"), ("f16", "f32"), ("f32", "f16"), ("f16", "f16")], ids="-".join)
 @pytest.mark.parametrize("size", [(1, 1, 1), (1, 4, 64), (2, 5, 65), (1, 7, 31), (1, 33, 130), (3, 250, 331)],
                          ids=lambda s: "x".join(map(str, s)))
