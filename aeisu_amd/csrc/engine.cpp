@@ -315,7 +315,6 @@ struct ModeWeights {
   DeviceBuffer fp32;               // FP32 policy: project weights and every bias (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
   DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail, f32_head;
-  F32SplitScale f32_compress_scale{}, f32_grouped_scale[4] = {}, f32_expand_scale{}, f32_refine_scale{}, f32_tail_scale{};
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -340,19 +339,12 @@ struct ModeWeights {
   F32Weights f32_weights() const {
     F32Weights W;
     W.image = fp32.as<float>();
-    for (int l = 0; l < 4; ++l) {
-      W.grouped[l] = f32_grouped[l].ptr;
-      W.grouped_scale[l] = f32_grouped_scale[l];
-    }
+    for (int l = 0; l < 4; ++l) W.grouped[l] = f32_grouped[l].ptr;
     W.compress = f32_compress.ptr;
-    W.compress_scale = f32_compress_scale;
     W.expand = f32_expand.ptr;
-    W.expand_scale = f32_expand_scale;
     W.head = f32_head.as<float>();
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
-    W.refine_scale = f32_refine_scale;
-    W.tail_scale = f32_tail_scale;
     return W;
   }
   size_t bytes() const {
@@ -522,21 +514,25 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
     const float* b = a.need(l + ".bias", kF32, {cout}).f32();
     std::copy(b, b + cout, img.begin() + off);
   };
-  // hi / lo FP16 fragments of a layer's weights, scaled so that the largest lies in [2^14, 2^15): chunk f of
-  // `chunks`, row m, slot s is the weight at(f, m, s); the fragment order is chunk, then hi and lo
-  auto split = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, int chunks, auto at, DeviceBuffer& dst) {
+  // hi / lo FP16 fragments of a layer's weights, each output's scaled so that its largest lies in [2^14, 2^15) (its
+  // bias lies at `off`): chunk f of `chunks`, row m, slot s is the weight at(f, m, s); the fragment order is chunk,
+  // then hi and lo
+  auto split = [&](const std::string& l, uint32_t cout, uint32_t cin, uint32_t ks, int off, int chunks, auto at, DeviceBuffer& dst) {
     const float* w = w32(l, cout, cin, ks);
     const size_t per = size_t(cin) * ks * ks;
-    float top = 0.f;
-    for (size_t i = 0; i < cout * per; ++i) top = std::max(top, std::fabs(w[i]));
-    F32SplitScale sc;
-    sc.exponent = top > 0 ? std::min(std::max(14 - std::ilogb(top), -60), 24) : 0;
+    std::vector<int> exponent(cout);
+    for (uint32_t o = 0; o < cout; ++o) {
+      float top = 0.f;
+      for (size_t i = 0; i < per; ++i) top = std::max(top, std::fabs(w[o * per + i]));
+      exponent[o] = top > 0.f ? std::min(std::max(14 - std::ilogb(top), kF32Unscale - 127), kF32Unscale + 126) : 0;
+      img[off + kF32Rows + o] = std::ldexp(1.f, kF32Unscale - exponent[o]);
+    }
     dst.upload(pack_frags<uint16_t>(2 * chunks, 8, [&](int f, int m, int s) {
-      const float v = std::ldexp(w[at(f / 2, m, s)], sc.exponent);
+      const size_t i = at(f / 2, m, s);
+      const float v = std::ldexp(w[i], exponent[i / per]);
       const uint16_t hi = f32_to_f16_bits(v);
       return f % 2 ? f32_to_f16_bits(v - f16_bits_to_f32(hi)) : hi;
     }));
-    return sc;
   };
   const float* wp = check("project", 32, 32, 1, 0.1f);
   for (int o = 0; o < 32; ++o)
@@ -554,18 +550,18 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   bias("refine", 64, kF32BiasRefine);
   check("tail", 64, 64, 1, 1.0f);
   bias("tail", 64, kF32BiasTail);
-  rt.f32_compress_scale = split("compress", 64, 128, 1, 16,
-                                [](int f, int m, int s) { return (16 * (f / 4) + m) * 128 + s * 4 + f % 4; }, rt.f32_compress);
-  rt.f32_expand_scale = split("expand", 128, 64, 1, 16, [](int f, int m, int s) {
+  split("compress", 64, 128, 1, kF32BiasCompress, 16,
+        [](int f, int m, int s) { return (16 * (f / 4) + m) * 128 + s * 4 + f % 4; }, rt.f32_compress);
+  split("expand", 128, 64, 1, kF32BiasExpand, 16, [](int f, int m, int s) {
     const int T = f / 2;
     return ((16 * (T >> 2) + m) * 4 + (T & 3)) * 64 + 32 * (f % 2) + s;
   }, rt.f32_expand);
   auto conv3 = [](int f, int m, int s) { return ((16 * (f / 9) + m) * 32 + s) * 9 + f % 9; };
   for (int l = 0; l < 4; ++l)
-    rt.f32_grouped_scale[l] = split("bottleneck" + std::to_string(l), 64, 32, 3, 36, conv3, rt.f32_grouped[l]);
-  rt.f32_refine_scale = split("refine", 64, 32, 3, 36, conv3, rt.f32_refine);
-  rt.f32_tail_scale = split("tail", 64, 64, 1, 8,
-                            [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; }, rt.f32_tail);
+    split("bottleneck" + std::to_string(l), 64, 32, 3, kF32BiasGrouped + 64 * l, 36, conv3, rt.f32_grouped[l]);
+  split("refine", 64, 32, 3, kF32BiasRefine, 36, conv3, rt.f32_refine);
+  split("tail", 64, 64, 1, kF32BiasTail, 8, [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; },
+        rt.f32_tail);
   // head: FP32 MFMA operands of the bank (taps past 24 are zero) and the base
   std::vector<float> head(kF32HeadFloats, 0.f);
   for (int tap = 0; tap < 25; ++tap)

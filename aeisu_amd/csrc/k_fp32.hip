@@ -110,7 +110,9 @@ __global__ __launch_bounds__(64) void f32_project_kernel(const Tin* __restrict__
 // FP16, and the lo halves end at 2^-39 of that.  The 1x1 layers and the tail take a scale per pixel.  The 3x3 layers
 // take the tile's largest (finite) pixel, and pixels below 2^-14 of it in a pass of their own with their own
 // scale (bands): a pixel's values are thus held to 2^-22 of themselves or 2^-25 of its largest, whatever lies
-// beside it.
+// beside it.  Weights are scaled by output (row): 2^e with the row's largest in [2^14, 2^15).  A sum is brought back
+// by 2^(-x - kF32Unscale) for an operand scale 2^x and then by the row's 2^(kF32Unscale - e), which no sum of FP32 operands
+// (weights below 2^118) leaves FP32's range between.
 __device__ __forceinline__ float residual_lo(float v, unsigned w) {   // v - (low half of w), exact
   float r;
   asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(v));
@@ -136,7 +138,7 @@ __device__ __forceinline__ float finite_abs(float v) {
   const float a = fabsf(v);
   return a < __builtin_inff() ? a : 0.f;
 }
-__device__ __forceinline__ float inverse_scale(int e) { return pow2f(-min(max(e, -126), 126)); }
+__device__ __forceinline__ float inverse_scale(int e) { return pow2f(-e - kF32Unscale); }   // e in [-113, 100]
 template <int CTRL>
 __device__ __forceinline__ unsigned dpp(unsigned v) {
   return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
@@ -341,11 +343,13 @@ __device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char
 template <int TH>
 __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const float* __restrict__ in, const h8* __restrict__ frag,
                                                                       const float* __restrict__ bias, float* __restrict__ out,
-                                                                      F32ConvTiles G, F32SplitScale sc) {
+                                                                      F32ConvTiles G) {
   typedef ConvLayout<TH> LY;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LY::SizeHalo];
   __shared__ __attribute__((aligned(16))) unsigned red[16];
+  __shared__ __attribute__((aligned(16))) float rows[32];
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, grp = blockIdx.y;
+  if (tid < 32) rows[tid] = bias[kF32Rows + 32 * grp + tid];
   const int n = lane & 15, g = lane >> 4;
   float4 v[LY::Per];
   int tidx = tile_of(0, G.num);
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
       conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
       if (last && it + 1 < iters && next < G.num) conv_fetch<LY::Per, 64>(v, in + 32 * grp, G, next, TH, LY::Chunks, fresh(tid));
       lds_barrier();
-      const float inv = inverse_scale(ex + sc.exponent);
+      const float inv = inverse_scale(ex);
       constexpr int R = TH / 4;                      // rows R wave .. R wave + R - 1
       f4 acc[R][2];
       conv_rows<R>(smem + (R * wave * kConvPW + n) * kConvPix + 16 * g, A, acc);
@@ -381,11 +385,12 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
           float* d = out + (((size_t)b * G.H + y) * G.W + x) * 64 + 32 * grp + 4 * g;
 #pragma unroll
           for (int T = 0; T < 2; ++T) {
+            const f4 sc = *reinterpret_cast<const f4*>(rows + 16 * T + 4 * g);
             f4 r = bs[T];
             if (!first) r = *reinterpret_cast<const f4*>(d + 16 * T);   // the sum so far
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              r[i] = fmaf(acc[j][T][i], inv, r[i]);
+              r[i] = fmaf(acc[j][T][i] * inv, sc[i], r[i]);
               if (last) r[i] = leaky(r[i], 0.1f);
             }
             *reinterpret_cast<f4*>(d + 16 * T) = r;
@@ -413,16 +418,18 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
                                                                           const h8* __restrict__ tfrag,
                                                                           const float* __restrict__ rbias,
                                                                           const float* __restrict__ tbias,
-                                                                          float* __restrict__ meta, F32ConvTiles G,
-                                                                          F32SplitScale rs, F32SplitScale ts) {
+                                                                          float* __restrict__ meta, F32ConvTiles G) {
   typedef ConvLayout<TH> LY;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LY::LdsRefine];
   __shared__ __attribute__((aligned(16))) unsigned red[16];
-  __shared__ __attribute__((aligned(16))) float rb[64], tb[64];   // biases: in registers the kernel spills
+  __shared__ __attribute__((aligned(16))) float rb[128], tb[128];   // biases and row scales: in registers the kernel spills
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, role = wave & 1, half = wave >> 1;
   float4 v[LY::Per];
-  if (tid < 64) rb[tid] = rbias[tid];
-  else if (tid < 128) tb[tid - 64] = tbias[tid - 64];
+  {
+    const int i = (tid & 63) + (tid & 64 ? kF32Rows : 0);
+    if (tid < 128) rb[tid] = rbias[i];
+    else tb[tid - 128] = tbias[i];
+  }
   int tidx = tile_of(0, G.num);
   if (tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
   h8 A[9][2][2];
@@ -442,7 +449,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
       conv_stage<LY::Per>(v, smem, pow2f(ex), LY::Chunks, fresh(tid));
       if (last && it + 1 < iters && next < G.num) conv_fetch<LY::Per, 32>(v, work, G, next, TH, LY::Chunks, fresh(tid));
       lds_barrier();
-      const float inv = inverse_scale(ex + rs.exponent);
+      const float inv = inverse_scale(ex);
       constexpr int R = TH >= 4 ? 2 : 1;
       for (int row = half * (TH / 2); row < (half + 1) * (TH / 2); row += R) {
         const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
@@ -457,13 +464,14 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
 #pragma unroll
           for (int T = 0; T < 2; ++T) {
             r[T] = *reinterpret_cast<const f4*>(rb + 32 * role + 16 * T + 4 * g);
+            const f4 sc = *reinterpret_cast<const f4*>(rb + 64 + 32 * role + 16 * T + 4 * g);
             if (!first) {                            // the sum so far
               const f2 a = *reinterpret_cast<const f2*>(d + 32 * T), c = *reinterpret_cast<const f2*>(d + 32 * T + 128);
               r[T] = f4{a[0], a[1], c[0], c[1]};
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              r[T][i] = fmaf(acc[j][T][i], inv, r[T][i]);
+              r[T][i] = fmaf(acc[j][T][i] * inv, sc[i], r[T][i]);
               if (last) r[T][i] = leaky(r[T][i], 0.1f);
               m = fmaxf(m, fabsf(r[T][i]));
             }
@@ -478,7 +486,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
               *reinterpret_cast<u2*>(d + 32 * T) = hi;
               *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
             }
-            if (g == 0) *reinterpret_cast<float*>(pix + 256 + 4 * role) = inverse_scale(er + ts.exponent);
+            if (g == 0) *reinterpret_cast<float*>(pix + 256 + 4 * role) = inverse_scale(er);
           } else {
 #pragma unroll
             for (int T = 0; T < 2; ++T) {
@@ -515,11 +523,12 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
       }
       const float2 inv = *reinterpret_cast<const float2*>(pix + 256);
       const f4 bias = *reinterpret_cast<const f4*>(tb + 16 * wave + 4 * g);
+      const f4 sc = *reinterpret_cast<const f4*>(tb + 64 + 16 * wave + 4 * g);
       const int qy = y0 + row, qx = x0 + n;
       if (qy < G.H && qx < G.W) {
         f4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = fmaf(acc[0][i], inv.x, fmaf(acc[1][i], inv.y, bias[i]));
+        for (int i = 0; i < 4; ++i) o[i] = fmaf(fmaf(acc[0][i], inv.x, acc[1][i] * inv.y), sc[i], bias[i]);
         *reinterpret_cast<f4*>(meta + (((size_t)b * G.H + qy) * G.W + qx) * 64 + 16 * wave + 4 * g) = o;
       }
     }
@@ -552,8 +561,7 @@ __device__ __forceinline__ LowPixel low_pixel(int idx, int Hl, int Wl) {
 __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const float* __restrict__ skip,
                                                                       const h8* __restrict__ frag,
                                                                       const float* __restrict__ bias,
-                                                                      float* __restrict__ low, int Hl, int Wl, int pixels,
-                                                                      F32SplitScale sc) {
+                                                                      float* __restrict__ low, int Hl, int Wl, int pixels) {
   const int lane = lane_id(), n = lane & 15, g = lane >> 4, waves = gridDim.x * (kF32Threads / 64);
   const int groups = (pixels + 15) >> 4;
   int grp = blockIdx.x * (kF32Threads / 64) + (threadIdx.x >> 6);
@@ -569,6 +577,9 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
   };
   float4 v[8];
   if (grp < groups) fetch(grp, v);
+  __shared__ __attribute__((aligned(16))) float rows[64];
+  if (threadIdx.x < 64) rows[threadIdx.x] = bias[kF32Rows + threadIdx.x];
+  lds_barrier();
   h8 A[4][4][2];
   f4 bs[4];
 #pragma unroll
@@ -581,7 +592,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
   }
   for (; grp < groups; grp += waves) {
     const int ex = scale_exponent(as_float(max_of_rows(as_bits(chunk_max(v)))));
-    const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
+    const float s = pow2f(ex), inv = inverse_scale(ex);
     h8 bh[4], bl[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) split8(v[2 * k], v[2 * k + 1], s, bh[k], bl[k]);
@@ -596,9 +607,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
         small = mfma_f16(A[T][k][0], bl[k], small);
         small = mfma_f16(A[T][k][1], bh[k], small);
       }
+      const f4 sc = *reinterpret_cast<const f4*>(rows + 16 * T + 4 * g);
       f4 r;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[i] + small[i], inv, bs[T][i]), 0.1f);
+      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf((acc[i] + small[i]) * inv, sc[i], bs[T][i]), 0.1f);
       if (idx < pixels) *reinterpret_cast<f4*>(low + (size_t)idx * 64 + 16 * T + 4 * g) = r;
     }
   }
@@ -611,8 +623,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
                                                                     const float* __restrict__ skip,
                                                                     const h8* __restrict__ frag,
                                                                     const float* __restrict__ bias,
-                                                                    float* __restrict__ work, int Hl, int Wl, int pixels,
-                                                                    F32SplitScale sc) {
+                                                                    float* __restrict__ work, int Hl, int Wl, int pixels) {
   const int lane = lane_id(), n = lane & 15, g = lane >> 4, waves = gridDim.x * (kF32Threads / 64);
   const int groups = (pixels + 15) >> 4;
   int grp = blockIdx.x * (kF32Threads / 64) + (threadIdx.x >> 6);
@@ -626,10 +637,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
   };
   float4 v[4];
   if (grp < groups) fetch(grp, v);
-  __shared__ __attribute__((aligned(16))) float sb[128];   // bias by row tile and row
-  if (threadIdx.x < 128) {
-    const int T = threadIdx.x >> 4, m = threadIdx.x & 15;
-    sb[threadIdx.x] = bias[(16 * (T >> 2) + m) * 4 + (T & 3)];
+  __shared__ __attribute__((aligned(16))) float sb[256];   // bias, then row scale, by row tile and row
+  {
+    const int T = threadIdx.x >> 4 & 7, m = threadIdx.x & 15;
+    sb[threadIdx.x] = bias[(threadIdx.x < 128 ? 0 : kF32Rows) + (16 * (T >> 2) + m) * 4 + (T & 3)];
   }
   lds_barrier();
   h8 A[8][2][2];
@@ -648,7 +659,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
 #pragma unroll
     for (int T = 0; T < 8; ++T) sk[T] = *reinterpret_cast<const f4*>(skip + at(T));
     const int ex = scale_exponent(as_float(max_of_rows(as_bits(chunk_max(v)))));
-    const float s = pow2f(ex), inv = inverse_scale(ex + sc.exponent);
+    const float s = pow2f(ex), inv = inverse_scale(ex);
     h8 bh[2], bl[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) split8(v[2 * k], v[2 * k + 1], s, bh[k], bl[k]);
@@ -662,10 +673,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
         small = mfma_f16(A[T][k][0], bl[k], small);
         small = mfma_f16(A[T][k][1], bh[k], small);
       }
-      const f4 bs = *reinterpret_cast<const f4*>(sb + 16 * T + 4 * g);
+      const f4 bs = *reinterpret_cast<const f4*>(sb + 16 * T + 4 * g), sc = *reinterpret_cast<const f4*>(sb + 128 + 16 * T + 4 * g);
       f4 r;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf(acc[i] + small[i], inv, bs[i]), 0.1f) + sk[T][i];
+      for (int i = 0; i < 4; ++i) r[i] = leaky(fmaf((acc[i] + small[i]) * inv, sc[i], bs[i]), 0.1f) + sk[T][i];
       if (idx < pixels) *reinterpret_cast<f4*>(work + at(T)) = r;
     }
   }
@@ -870,8 +881,7 @@ static hipError_t launch_grouped_t(const float* in, const F32Weights& W, int l, 
                                    hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hl, Wl, TH, batch);
   hipLaunchKernelGGL(f32_grouped_kernel<TH>, dim3(persistent_grid(G.num, cus), 2), dim3(kConvThreads), 0, stream, in,
-                     (const h8*)W.grouped[l], W.image + kF32BiasGrouped + 64 * l, out, G,
-                     W.grouped_scale[l]);
+                     (const h8*)W.grouped[l], W.image + kF32BiasGrouped + 64 * l, out, G);
   return hipGetLastError();
 }
 static hipError_t launch_f32_grouped(const float* in, const F32Weights& W, int l, float* out, int Hl, int Wl, int batch,
@@ -889,8 +899,7 @@ static hipError_t launch_refine_t(const float* work, const F32Weights& W, float*
                                   hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hq, Wq, TH, batch);
   hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(persistent_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
-                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32BiasRefine, W.image + kF32BiasTail, meta,
-                     G, W.refine_scale, W.tail_scale);
+                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32BiasRefine, W.image + kF32BiasTail, meta, G);
   return hipGetLastError();
 }
 static hipError_t launch_f32_refine_tail(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch,
@@ -920,15 +929,14 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
   for (int i = 0; i < 5; ++i) dst[i] = lows ? lows[i] : (i % 2 ? low1 : low0);
   const int low_blocks = (int)std::min((lowpx + 63) / 64, 2L * cus);     // four groups of 16 pixels a block, persistent
   hipLaunchKernelGGL(f32_compress_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)skip,
-                     (const h8*)wts.compress, wimg + kF32BiasCompress, dst[0], Hl, Wl, (int)lowpx, wts.compress_scale);
+                     (const h8*)wts.compress, wimg + kF32BiasCompress, dst[0], Hl, Wl, (int)lowpx);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[2], stream)) != hipSuccess) return e;
   for (int l = 0; l < 4; ++l)
     if ((e = launch_f32_grouped(dst[l], wts, l, dst[l + 1], Hl, Wl, batch, cus, stream)) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[3], stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(f32_expand_kernel, dim3(low_blocks), dim3(kF32Threads), 0, stream, (const float*)dst[4],
-                     (const float*)skip, (const h8*)wts.expand, wimg + kF32BiasExpand, work, Hl, Wl, (int)lowpx,
-                     wts.expand_scale);
+                     (const float*)skip, (const h8*)wts.expand, wimg + kF32BiasExpand, work, Hl, Wl, (int)lowpx);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (ev && (e = hipEventRecord(ev[4], stream)) != hipSuccess) return e;
   if ((e = launch_f32_refine_tail(work, wts, meta, Hq, Wq, batch, cus, stream)) != hipSuccess) return e;

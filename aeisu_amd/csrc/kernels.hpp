@@ -121,7 +121,8 @@ hipError_t launch_fused_tail_head(int in_fp32, int out_fp32, int qclamp, const v
                                   unsigned* nonfinite, int grid, hipStream_t stream);
 
 // FP32 policy (k_fp32.hip): per-layer kernels on FP32 NHWC activations.  FP32 image (floats): the project's
-// W[32 feature channel f*4+phase][32 outputs] and b[32], the other layers' biases, the 24 analysis constants.
+// W[32 feature channel f*4+phase][32 outputs] and b[32], the other layers' biases, the 24 analysis constants,
+// the other layers' row scales.
 constexpr int kF32Project = 0;
 constexpr int kF32BiasCompress = kF32Project + 32 * 32 + 32;
 constexpr int kF32BiasGrouped = kF32BiasCompress + 64;
@@ -129,11 +130,11 @@ constexpr int kF32BiasExpand = kF32BiasGrouped + 4 * 64;
 constexpr int kF32BiasRefine = kF32BiasExpand + 128;
 constexpr int kF32BiasTail = kF32BiasRefine + 64;
 constexpr int kF32Analysis = kF32BiasTail + 64;
-constexpr int kF32Floats = kF32Analysis + 24;
-// A layer whose products run as hi / lo FP16 splits: its weights are scaled by 2^exponent.
-struct F32SplitScale {
-  int exponent;
-};
+// A layer whose products run as hi / lo FP16 splits: the weights of the output with its bias at b are scaled by 2^e,
+// and 2^(kF32Unscale - e) lies at b + kF32Rows.
+constexpr int kF32Rows = kF32Analysis + 24 - kF32BiasCompress;
+constexpr int kF32Floats = kF32Rows + kF32Analysis;
+constexpr int kF32Unscale = 24;
 constexpr int kF32HeadBase = 7 * 64 * 4, kF32HeadFloats = kF32HeadBase + 4 * 7 * 4;
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
@@ -142,7 +143,6 @@ struct F32Weights {
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
   const float* head;                       // FP32 bank [t][lane][K step] (row 4g + i of tile t: phase g, tap 4t + i; step j
                                            // of lane group g: coefficient 4g + j), then the base float4 [g][t]
-  F32SplitScale compress_scale, grouped_scale[4], expand_scale, refine_scale, tail_scale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong

@@ -147,6 +147,66 @@ def test_stages_with_outliers(model, size, values):
     compare(*model, frames)
 
 
+def with_weights(R, path, change):
+    """(model, folded state) of area's checkpoint with change(layer, weight, bias) for its layers' FP32 weights."""
+    from aeisu_amd import artifacts as A
+    records, header = A.read_records(A.load_blob(WEIGHTS / "aeisu_area.pt")[0])
+    state, arrays = M.load_folded(WEIGHTS / "aeisu_area.pt"), {r[0]: i for i, r in enumerate(records)}
+    for layer in A.LAYERS:
+        iw, ib = arrays[layer + ".weight_fp32"], arrays[layer + ".bias"]
+        w, b = change(layer, torch.from_numpy(records[iw][3]).clone(), torch.from_numpy(records[ib][3]).clone())
+        for i, t in ((iw, w), (ib, b)):
+            records[i] = (*records[i][:3], t.numpy())
+        names = [f"bottleneck_270_{n}{int(layer[-1]) + 1}" for n in "ab"] if layer.startswith("bottleneck") else [A.FOLDED_NAMES[layer]]
+        for name, pw, pb in zip(names, w.chunk(len(names)), b.chunk(len(names))):
+            state[name + ".weight"], state[name + ".bias"] = pw.contiguous(), pb.contiguous()
+    path.write_bytes(A.write(records, **header))
+    return R.load_model(path, precision="fp32"), state
+
+
+def test_weights_over_the_range(R, tmp_path):
+    """Layers whose weights and activations are scaled by powers of two that the next layer takes back: the FP32
+    policy's arithmetic is the same up to those powers, so the outputs are the same bits."""
+    print("case: FP32 policy, layers scaled by 2^-100 to 2^80", flush=True)
+    scale, last = {"compress": -50, "bottleneck0": 30, "bottleneck1": -70, "bottleneck2": 10, "bottleneck3": -20, "refine": 45}, {}
+
+    def change(layer, w, b):
+        before = {"bottleneck0": "compress", "bottleneck1": "bottleneck0", "bottleneck2": "bottleneck1",
+                  "bottleneck3": "bottleneck2", "expand": "bottleneck3", "tail": "refine"}.get(layer)
+        own = scale.get(layer, 0)
+        return w * 2.0 ** (own - scale.get(before, 0)), b * 2.0 ** own
+
+    m, _ = with_weights(R, tmp_path / "scaled.bin", change)
+    frames = torch.rand(2, 3, 70, 90, generator=torch.Generator().manual_seed(2)).cuda()
+    plain = R.load_model(WEIGHTS / "aeisu_area.pt", precision="fp32")
+    assert torch.equal(m.run(frames), plain.run(frames))
+
+
+def test_rows_of_small_weights(R, tmp_path):
+    """Outputs whose weights are far below their layer's largest: every channel within FP32 error of its own
+    magnitude (the 2-norm of its error below 2e-6 of its own; 64 x 2^-24 per sum would be 4e-6)."""
+    print("case: FP32 policy, every other output's weights at 2^-30", flush=True)
+
+    def change(layer, w, b):
+        if layer not in ("project", "expand"):                # expand is added to skip
+            w[1::2] *= 2.0 ** -30
+            b[1::2] *= 2.0 ** -30
+        return w, b
+
+    m, state = with_weights(R, tmp_path / "rows.bin", change)
+    skip, low, work, meta = stages(m, torch.rand(1, 3, 100, 130, generator=torch.Generator().manual_seed(4)))
+    pairs = {"compress": (low[0], conv64(F.pixel_unshuffle(skip, 2), state, "compress_270")[0])}
+    for i in range(1, 5):
+        pairs[f"bottleneck {i}"] = (low[i], torch.cat([conv64(low[i - 1][:, 32 * j:32 * j + 32], state, f"bottleneck_270_{n}{i}")[0]
+                                                       for j, n in enumerate("ab")], 1))
+    pairs["refine + tail"] = (meta, conv64(conv64(work, state, "refine_540")[0], state, "metadata_head", slope=1.0)[0])
+    for name, (got, ref) in pairs.items():
+        size = lambda x: x.double().square().sum((0, 2, 3)).sqrt()  # noqa: E731
+        worst = (size(got - ref) / size(ref)).max().item()
+        print(f"  {name}: worst channel {worst:.3g}", flush=True)
+        assert worst <= 2e-6, name
+
+
 @pytest.mark.parametrize("dtypes", [("f32", "f32"), ("f16", "f32"), ("f32", "f16"), ("f16", "f16")], ids="-".join)
 @pytest.mark.parametrize("size", [(1, 1, 1), (1, 4, 64), (2, 5, 65), (1, 7, 31), (1, 33, 130), (3, 250, 331)],
                          ids=lambda s: "x".join(map(str, s)))
