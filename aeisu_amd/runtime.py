@@ -240,11 +240,13 @@ def load_model(path, device: str = "cuda", precision: Optional[str] = None) -> U
     return Upscaler(blob, precision, device)
 
 
-# Tiles are joined into regions of at most this many LR pixels a side (or one tile), so that a region is one
-# launch sequence instead of one for each tile.  A pixel of the output depends on input less than 32 pixels
-# away, which every region's halo holds, so the result does not depend on where regions are cut.  2048 bounds
-# the scratch of a region (0.7 GB under the FP32 policy).  678 x 1020 at tile 128: 54 tiles of 3 launches, a
-# synchronisation and 2 copies each took 4.2 of the call's 6.1 ms, one region takes 0.1 ms.
+# Tiles are joined into regions of at most 16 tiles and this many LR pixels a side (or one tile), so that a region is
+# one launch sequence instead of one for each tile.  A pixel of the output depends on input less than 32 pixels
+# away, which every region's halo holds, so the result does not depend on where regions are cut (FP32 policy: but
+# for the rounding of its products).  All regions of an image have one shape, hence one scratch: at most that of
+# 2112 x 2112 pixels (0.7 GB under the FP32 policy) at tiles of 128 and more, 1088 x 1088 at 64, 576 x 576 (0.05 GB)
+# at 32.  678 x 1020 at tile 128: 54 tiles of 3 launches, a synchronisation and 2 copies each took 4.2 of the
+# call's 6.1 ms, one region takes 0.1 ms.
 _REGION = 2048
 # Results above this many bytes go to the host through two pinned buffers of this size: the copy from the
 # device overlaps the copy into the result, which torch splits over threads (its pages are touched for the
@@ -283,7 +285,12 @@ def _to_host(x: torch.Tensor) -> torch.Tensor:
 
 @torch.inference_mode()
 def upscale(model: Upscaler, source: torch.Tensor, tile: int = 128) -> torch.Tensor:
-    """aeisu/runtime.py:70-103 on the GPU runtime: CHW [0,1] -> clipped 2x CHW float32 (CPU)."""
+    """aeisu/runtime.py:70-103 on the GPU runtime: CHW [0,1] -> clipped 2x CHW float32 (CPU).
+
+    ``tile`` 0 runs the image whole; else regions of up to 16 tiles a side run one after the other, so a smaller
+    tile takes less scratch (see ``_REGION``).  Each size of region is one of the model's ``max_handles`` kept
+    geometries.
+    """
     if source.ndim != 3 or source.shape[0] != 3:
         raise ValueError("Expected CHW RGB image")
     if tile < 0 or tile % 32:
@@ -298,20 +305,21 @@ def _upscaled(model: Upscaler, image: torch.Tensor, tile: int) -> torch.Tensor:
     h, w = image.shape[-2:]
     ey, ex = -h % 32, -w % 32
     ph, pw = h + 32 + ey, w + 32 + ex
-    step = max(tile, _REGION // tile * tile) if tile else 0
-    if tile == 0 or (ph <= step and pw <= step):
+    side = max(tile, min(_REGION, 16 * tile) // tile * tile) if tile else max(ph, pw)
+    if ph <= side and pw <= side:
         return model.run(image, out_dtype=torch.float32)[0]
     py, px = 16 + ey // 2, 16 + ex // 2
     padded = F.pad(image, (px, 32 + ex - px, py, 32 + ey - py), mode="replicate")
     result = torch.empty(3, 2 * h, 2 * w, dtype=torch.float32, device=model.device)
-    for y in range(0, ph, step):
-        for x in range(0, pw, step):
-            y1, x1 = min(y + step, ph), min(x + step, pw)
-            sy, sx = max(0, y - 32), max(0, x - 32)
-            pred = model.run(padded[:, :, sy:min(ph, y1 + 32), sx:min(pw, x1 + 32)].contiguous(),
-                             out_dtype=torch.float32, pad=False)[0]
+    # cores of equal sides, multiples of 32; their windows, halo included, are moved inwards at the frame's edges
+    step_y, step_x = (32 * -(-p // (32 * -(-p // side))) for p in (ph, pw))
+    wh, ww = min(ph, step_y + 64), min(pw, step_x + 64)
+    for y in range(0, ph, step_y):
+        for x in range(0, pw, step_x):
+            sy, sx = min(max(0, y - 32), ph - wh), min(max(0, x - 32), pw - ww)
+            pred = model.run(padded[:, :, sy:sy + wh, sx:sx + ww].contiguous(), out_dtype=torch.float32, pad=False)[0]
             # the region's core inside the frame
-            ty, tx, by, bx = max(y, py), max(x, px), min(y1, py + h), min(x1, px + w)
+            ty, tx, by, bx = max(y, py), max(x, px), min(y + step_y, py + h), min(x + step_x, px + w)
             if ty < by and tx < bx:
                 result[:, 2 * (ty - py):2 * (by - py), 2 * (tx - px):2 * (bx - px)] = \
                     pred[:, 2 * (ty - sy):2 * (by - sy), 2 * (tx - sx):2 * (bx - sx)]

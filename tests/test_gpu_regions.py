@@ -38,6 +38,33 @@ def test_regions_equal_whole(R, monkeypatch, precision, size, tile, region):
         R.upscale(model, bad, tile)
 
 
+@pytest.mark.parametrize("size", [(150, 333), (65, 500), (200, 60)])
+def test_one_scratch_for_all_regions(R, monkeypatch, size):
+    """Every region of an image has the same shape, at the edges too: one geometry, and the scratch of one region of
+    at most the region's side and its halo."""
+    print(f"case: regions of {size}", flush=True)
+    monkeypatch.setattr(R, "_REGION", 64)
+    model = R.load_model(WEIGHTS / "aeisu_area.pt", precision="fp32")
+    R.upscale(model, torch.rand(3, *size, generator=torch.Generator().manual_seed(6)), 32)
+    other = R.load_model(WEIGHTS / "aeisu_area.pt", precision="fp32")
+    other.run(torch.rand(1, 3, 128, 128, device="cuda"), pad=False)
+    assert model.persistent_bytes() <= other.persistent_bytes()
+
+
+def test_small_tiles_take_less_scratch(R):
+    """A caller short of memory still has it with a smaller tile."""
+    print("case: scratch of upscale() by tile", flush=True)
+    src = torch.rand(3, 700, 1100, generator=torch.Generator().manual_seed(8))
+    used = {}
+    for tile in (32, 64, 128):
+        model = R.load_model(WEIGHTS / "aeisu_area.pt", precision="fp32")
+        weights = model.persistent_bytes()
+        R.upscale(model, src, tile)
+        used[tile] = model.persistent_bytes() - weights
+    assert used[32] < used[64] < used[128]
+    assert used[32] <= 576 * 576 * 200
+
+
 @pytest.mark.parametrize("numel", [1, 2 << 20, (2 << 20) + 1, (4 << 20) + 3, 9_000_001])
 def test_copy_to_host(R, numel):
     """One chunk and less, chunk boundaries and a short last chunk; results are ordinary pageable tensors."""
