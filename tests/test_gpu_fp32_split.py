@@ -1,11 +1,12 @@
 """FP32 policy: every stage against the same stage in 64 bits on the GPU's own input, at the edges of the
 kernels' tiles and over FP32's range.
 
-The convolutions run as hi / lo FP16 splits on the MFMA (k_fp32.hip).  The bound of an output is
+The layers from compress to the tail run as hi / lo FP16 splits on the MFMA (k_fp32.hip).  The bound of an output is
 2^-22 P sum |w||x| with P = 3 + 4 K / 8 at K products: each operand is held to 2^-22 (two operands and the
 dropped lo lo' product: 3), and the FP32 accumulators round once per 8 products, in three chains of which
 one is at the main sum's magnitude (2^-24 a rounding, taken as 2^-22 for terms that the MFMA cuts off when it
-aligns them).  FP32 FMA chains stay within it too.
+aligns them).  That is the worst case of an output, 100 times and more what is seen, so the error over all outputs is
+also held to that of FP32 FMA chains, which a split that loses bits exceeds.
 """
 from __future__ import annotations
 
@@ -14,6 +15,7 @@ import torch
 from torch.nn import functional as F
 
 from oracle import model as M
+from tests._fp32 import chain, conv_chain, conv_size, leaky, rms
 from tests._util import WEIGHTS, crop_output, pad_frame
 
 pytestmark = pytest.mark.gpu
@@ -53,29 +55,53 @@ def conv64(x, state, name, slope=0.1):
     w, b = state[name + ".weight"].double(), state[name + ".bias"].double()
     pad, k = w.shape[-1] // 2, w[0].numel()
     y = F.conv2d(x.double(), w, b, padding=pad)
-    size = F.conv2d(x.double().abs(), w.abs(), b.abs(), padding=pad)
-    return torch.where(y >= 0, y, slope * y), 2.0 ** -22 * (3 + 4 * k / 8) * size
+    return leaky(y, slope), 2.0 ** -22 * (3 + 4 * k / 8) * conv_size(x, w, b)
 
 
-def check(name, got, ref, bound):
+def no_worse(name, got, ref, chains, size, values):
+    """The error of all outputs, relative to the magnitude of each one's terms, is at most that of FP32 FMA chains
+    (`chains` is what those give), but for chance: 10 % (expand's and the project's largest rounding is the same in
+    both, so that their errors come out alike), a factor of 2 for a frame of one value, whose `values` distinct
+    outputs are few.  Splits have 0.3 to 0.7 of it; with 6 bits in the lo halves they have more than twice it
+    (tests/test_fp32_split_cpu.py)."""
+    ours, theirs = rms(got.double() - ref, size), rms(chains.double() - ref, size)
+    print(f"  {name}: {ours:.3g} of the terms, FMA chains {theirs:.3g}", flush=True)
+    assert ours <= (1.1 if values > 1 else 2) * theirs, name
+
+
+def check(name, got, ref, bound, chains, size, values):
+    """Every output within its bound, and all of them no worse than FMA chains."""
     over = (got.double() - ref).abs() - bound
     assert torch.isfinite(got).all(), name
     assert over.max().item() <= 0, f"{name}: {over.max().item():.3g} over the bound"
+    no_worse(name, got, ref, chains, size, values)
+
+
+def conv_fp32(x, state, name, slope=0.1):
+    """The layer with FP32 FMA chains (on the GPU: 64-bit arithmetic on the CPU takes a minute per size)."""
+    y = conv_chain(x.cuda(), state[name + ".weight"].cuda(), state[name + ".bias"].cuda()).cpu()
+    return torch.where(y >= 0, y, y * slope)
 
 
 def compare(model, state, frames):
     skip, low, work, meta = stages(model, frames)
-    check("compress", low[0], *conv64(F.pixel_unshuffle(skip, 2), state, "compress_270"))
+    values = frames[0, 0].numel()
+
+    def layer(x, name):
+        return (*conv64(x, state, name), conv_fp32(x, state, name), conv_size(x, state[name + ".weight"], state[name + ".bias"]))
+
+    check("compress", low[0], *layer(F.pixel_unshuffle(skip, 2), "compress_270"), values)
     for i in range(1, 5):
         for n, part in (("a", slice(0, 32)), ("b", slice(32, 64))):
-            check(f"bottleneck {i}{n}", low[i][:, part], *conv64(low[i - 1][:, part], state, f"bottleneck_270_{n}{i}"))
-    up, bound = conv64(low[4], state, "expand_270")
-    ref = skip.double() + F.pixel_shuffle(up, 2)
-    check("expand", work, ref, F.pixel_shuffle(bound, 2) + 2.0 ** -23 * ref.abs())
-    r, rb = conv64(work, state, "refine_540")
+            check(f"bottleneck {i}{n}", low[i][:, part], *layer(low[i - 1][:, part], f"bottleneck_270_{n}{i}"), values)
+    up, bound, one, size = (F.pixel_shuffle(t, 2) for t in layer(low[4], "expand_270"))
+    ref = skip.double() + up
+    check("expand", work, ref, bound + 2.0 ** -23 * ref.abs(), skip + one, size + skip.double().abs(), values)
+    r, rb, one, size = layer(work, "refine_540")
+    w = state["metadata_head.weight"].double()
     ref, tb = conv64(r, state, "metadata_head", slope=1.0)
-    through = F.conv2d(rb, state["metadata_head.weight"].double().abs())
-    check("refine + tail", meta, ref, tb + through)
+    check("refine + tail", meta, ref, tb + F.conv2d(rb, w.abs()), conv_fp32(one, state, "metadata_head", slope=1.0),
+          conv_size(size, w, state["metadata_head.bias"]), values)
 
 
 # one tile and less, ragged tiles, tile multiples, many frames (the large-launch variants), long rows, the grouped
@@ -88,6 +114,23 @@ def test_stages_against_64_bits(model, size):
     b, h, w = size
     print(f"case: FP32 stages {size}", flush=True)
     compare(*model, torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(h * w)))
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_project_against_64_bits(model, size):
+    """Analysis features and project, against the oracle's FP32 features and FMA chains."""
+    b, h, w = size
+    m, state = model
+    print(f"case: FP32 project {size}", flush=True)
+    frames = torch.rand(b, 3, h, w, generator=torch.Generator().manual_seed(h * w))
+    skip = stages(m, frames)[0]
+    wide = {k: v.double() if torch.is_tensor(v) else v for k, v in state.items()}
+    features = lambda x, st: F.pixel_unshuffle(M.rgb_to_feature8(x, st), 2)  # noqa: E731
+    exact = features(pad_frame(frames).double(), wide)
+    ref = conv64(exact, state, "project_540")[0]
+    one = conv_fp32(features(pad_frame(frames), state), state, "project_540")
+    size_ = conv_size(exact, state["project_540.weight"], state["project_540.bias"])
+    no_worse("project", skip, ref, one, size_, h * w)
 
 
 @pytest.mark.parametrize("gain", [0.0, 1e-30, 1e-6, 3e5, 1e12])
@@ -212,8 +255,8 @@ def test_rows_of_small_weights(R, tmp_path):
                          ids=lambda s: "x".join(map(str, s)))
 def test_head_against_64_bits(model, size, dtypes):
     """The head on the GPU's own coefficients, at ragged widths and heights, in every pair of layouts.  An
-    output is 25 filter weights (each 16 products and a base) applied to the window: 2^-22 (3 + 4 * 16 / 8) of
-    the weights' terms and 25 FP32 roundings of the sums, and the output's rounding."""
+    output is 25 filter weights (16 products and a base, 17 FP32 roundings, of coefficients that the clamp rounds
+    twice) applied to the window (25 roundings): 44 x 2^-24 of the terms, and the output's rounding."""
     from aeisu_amd import _lib as L
     kind = {"f16": torch.float16, "f32": torch.float32}
     m, state = model
@@ -229,19 +272,11 @@ def test_head_against_64_bits(model, size, dtypes):
     base, basis = state["base"].double(), state["basis"].double()
     ref = crop_output(M.reconstruct(padded, meta, base, basis), h, w)
     size_ = crop_output(M.reconstruct(padded.abs(), meta.abs(), base.abs(), basis.abs()), h, w)
-    bound = (2.0 ** -22 * 11 + 25 * 2.0 ** -24) * size_ + 1e-12
+    bound = 44 * 2.0 ** -24 * size_ + 1e-12
     if dtypes[1] == "f16":
         bound = bound + 2.0 ** -11 * ref.abs() + 2.0 ** -25
     over = (got - ref.clamp(0, 1)).abs() - bound
     assert over.max().item() <= 0, f"{over.max().item():.3g} over the bound"
-
-
-def chain(acc, pairs):
-    """acc + the products of `pairs`, one FP32 fused multiply-add after the other (a product of two FP32 values is
-    exact in 64 bits, where the sum's own rounding is 2^-29 of the FP32 one)."""
-    for a, b in pairs:
-        acc = (acc.double() + a.double() * b.double()).float()
-    return acc
 
 
 def head_chain(padded, meta, base, basis, y0, x0, h, w):
