@@ -315,6 +315,7 @@ struct ModeWeights {
   DeviceBuffer fp32;               // FP32 policy: project weights and every bias (kernels.hpp kF32*)
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
   DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail, f32_head;
+  float f32_head_unscale = 1.f;
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -342,7 +343,8 @@ struct ModeWeights {
     for (int l = 0; l < 4; ++l) W.grouped[l] = f32_grouped[l].ptr;
     W.compress = f32_compress.ptr;
     W.expand = f32_expand.ptr;
-    W.head = f32_head.as<float>();
+    W.head = f32_head.ptr;
+    W.head_unscale = f32_head_unscale;
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
     return W;
@@ -562,15 +564,30 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   split("refine", 64, 32, 3, kF32BiasRefine, 36, conv3, rt.f32_refine);
   split("tail", 64, 64, 1, kF32BiasTail, 8, [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; },
         rt.f32_tail);
-  // head: FP32 MFMA operands of the bank (taps past 24 are zero) and the base
-  std::vector<float> head(kF32HeadFloats, 0.f);
-  for (int tap = 0; tap < 25; ++tap)
-    for (int ph = 0; ph < 4; ++ph) {
-      for (int k = 0; k < 16; ++k)
-        head[((tap / 4) * 64 + 16 * (k / 4) + 4 * ph + tap % 4) * 4 + k % 4] = basis[(tap * 16 + k) * 4 + ph];
-      head[kF32HeadBase + ph * 28 + tap] = base[tap * 4 + ph];
-    }
-  rt.f32_head.upload(head);
+  // head bank, scaled so that the largest weight lies in [2^13, 2^14): row 4g + i of tile t is phase g of tap
+  // 4t + i (taps past 24 are zero); slots 0..15 the lo parts of the coefficients' weights and 16..31 the hi
+  // parts, or (fragments 7..13) the third and the hi parts; odd taps negated (k_fp32.hip)
+  float top = 0.f;
+  for (int i = 0; i < 1600; ++i) top = std::max(top, std::fabs(basis[i]));
+  const int e = top > 0.f ? std::min(13 - std::ilogb(top), 30) : 0;
+  auto bank = pack_frags<uint16_t>(14, 8, [&](int f, int m, int s) -> uint16_t {
+    const int tap = 4 * (f % 7) + m % 4;
+    if (tap > 24) return 0;
+    const float v = std::ldexp(basis[(tap * 16 + s % 16) * 4 + m / 4], e) * (tap % 2 ? -1.f : 1.f);
+    const uint16_t hi = f32_to_f16_bits(v);
+    const float rest = v - f16_bits_to_f32(hi);
+    const uint16_t lo = f32_to_f16_bits(rest);
+    if (f < 7) return s < 16 ? lo : hi;
+    return s < 16 ? f32_to_f16_bits(rest - f16_bits_to_f32(lo)) : hi;
+  });
+  std::vector<float> rows(4 * 7 * 4, 0.f);
+  for (int g = 0; g < 4; ++g)
+    for (int tap = 0; tap < 25; ++tap) rows[g * 28 + tap] = std::ldexp(base[tap * 4 + g], e);
+  const size_t halves = bank.size();
+  bank.resize(halves + 2 * rows.size());
+  std::memcpy(bank.data() + halves, rows.data(), rows.size() * sizeof(float));
+  rt.f32_head.upload(bank);
+  rt.f32_head_unscale = std::ldexp(1.f, -e);
   for (int i = 0; i < 24; ++i) img[kF32Analysis + i] = rt.analysis[i];
   rt.fp32.upload(img);
 }

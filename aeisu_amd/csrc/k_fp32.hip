@@ -7,9 +7,9 @@
 //   meta  [B][Hq][Wq][64]   refine 3x3 + LeakyReLU -> tail 1x1 (the packed coefficients)
 // and the head writes the clipped 2x frame.
 //
-// The project and the head's filter synthesis run as FP32 MFMAs, the layers between them as hi / lo FP16 splits
-// on the FP16 MFMA (below); all sums are FP32, in a fixed order that differs from the reference's convolution
-// order only by FP32 rounding.
+// The project runs as FP32 MFMAs, every other product as hi / lo FP16 splits on the FP16 MFMA (below);
+// all sums are FP32, in a fixed order that differs from the reference's convolution order only by FP32
+// rounding.
 #include <algorithm>
 
 #include "common.hpp"
@@ -696,14 +696,17 @@ __device__ __forceinline__ float clamp_coef(float a) {
 }
 
 // Persistent blocks over tiles of 64 x 4 LR pixels, one row per wave, in two chunks of 32 pixels.  The filter
-// weights of a chunk's even and odd pixels are products of 16 columns on the FP32 MFMA, laid out as in k_head.hip:
-// row 4g + i of row tile t is (phase g, tap 4t + i), so accumulator lane (n, g) holds all 25 taps of phase g of
-// pixels 2n and 2n + 1; K step j takes coefficient 4g + j from lane group g, so a lane reads four neighbouring
-// coefficients of each pixel.  The base is added to the sum of the 16 products, not taken as its first addend.
-// FP32 operands and sums rounded to nearest, no further from 64 bits than one FMA chain per weight: outputs (frames
-// of 33 x 65 to 1080p) 1.15e-7 (area) and 1.23e-7 (DIV2K), the chains 1.17e-7 and 1.26e-7.  Three-part FP16 splits
-// took 20 us less at 1080p (frame 339 against 359 us) and 0.3 us less for 256 x 256, but the FP16 MFMA cuts off the
-// bits of all terms below the largest of a pass, which darkens every output by 1.3e-8 on average (1.21e-7 and 1.20e-7).
+// weights of a chunk's even and odd pixels are two MFMA products of 16 columns, as in k_head.hip: row 4g + i of
+// row tile t is (phase g, tap 4t + i), so accumulator lane (n, g) holds all 25 taps of phase g of pixels 2n and
+// 2n + 1, with bank and coefficients in three FP16 parts each (exact to 2^-25),
+// [K_3 | K_hi] . [c_hi ; c_3] + [K_lo | K_hi] . [c_lo ; c_lo] + [K_lo | K_hi] . [c_hi ; c_hi], small terms
+// first, since the MFMA cuts off the bits of all terms below the largest of a pass; the FP32 base is added to
+// the sum, not taken as its first addend.  Cutting off lowers every sum, by 1e-9 on average, and the 25 taps add
+// that up: the bank of odd taps is negated and its sums are subtracted from the base, so that neighbouring taps take
+// it from each other (mean error of the output -1.3e-8 without, 4e-9 (area) and 4e-10 (DIV2K) with it).  Against 64
+// bits (frames of 33 x 65 to 1080p) the output's error is 1.08e-7 (area) and 1.17e-7 (DIV2K); one FP32 FMA chain
+// per weight gave 1.17e-7 and 1.26e-7, all sums of one sign 1.21e-7 and 1.20e-7, FP32 MFMAs 1.15e-7 and 1.23e-7 and
+// 113 us instead of 88 at 1080p.  Bank and base are scaled by a power of two, the RGB tile by its inverse.
 // The lane applies them with FP32 FMAs in tap order.  Two neighbouring pixels share 20 of their 25 window
 // positions: 30 LDS reads of 16 bytes instead of 50, which would take 46 us of LDS time at 1080p; the tile
 // holds even and odd columns apart, so that the lanes' reads are contiguous.  One thread per pixel took 168 us
@@ -714,6 +717,7 @@ constexpr int kF32HPos = kF32HLW * kF32HLH, kF32HPer = (kF32HPos + kF32Threads -
 constexpr int kF32HPlane = kF32HPos / 2;
 struct F32HeadGeom {
   int H, W, Hq, Wq, py, px, tiles_x, tiles_y, num;
+  float unscale;                                             // of the bank's power of two
 };
 struct F32HeadTile {
   int b, y0, x0;
@@ -735,16 +739,18 @@ __device__ __forceinline__ void f32_head_rgb(Tin (&v)[kF32HPer][3], const Tin* _
     for (int c = 0; c < 3; ++c) v[k][c] = s[c * plane + o];
   }
 }
-// The lane's four coefficients of pixels 2n and 2n + 1 of chunk j of the wave's row.  Pixels past the frame edge
+// The lane's eight coefficients of pixels 2n and 2n + 1 of chunk j of the wave's row.  Pixels past the frame edge
 // take the edge's (inside the tensor) and are not stored.
-__device__ __forceinline__ void f32_head_coef(float4 (&c)[2], const float* __restrict__ meta, F32HeadTile t,
+__device__ __forceinline__ void f32_head_coef(float4 (&c)[2][2], const float* __restrict__ meta, F32HeadTile t,
                                               const F32HeadGeom& G, int j, int wave, int lane) {
   const int n = lane & 15, Y = min(t.y0 + wave, G.H - 1) + G.py;
-  const float* row = meta + ((size_t)t.b * G.Hq + (Y >> 1)) * G.Wq * 64 + 32 * (Y & 1) + 4 * (lane >> 4);
+  const float* row = meta + ((size_t)t.b * G.Hq + (Y >> 1)) * G.Wq * 64 + 32 * (Y & 1) + 8 * ((lane >> 4) & 1);
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const int X = min(t.x0 + 32 * j + 2 * n + p, G.W - 1) + G.px;
-    c[p] = *reinterpret_cast<const float4*>(row + (size_t)(X >> 1) * 64 + 16 * (X & 1));
+    const float* q = row + (size_t)(X >> 1) * 64 + 16 * (X & 1);
+    c[p][0] = *reinterpret_cast<const float4*>(q);
+    c[p][1] = *reinterpret_cast<const float4*>(q + 4);
   }
 }
 // The output is written once and not read here: the non-temporal hint keeps it from displacing the coefficients
@@ -761,22 +767,24 @@ __device__ __forceinline__ void store_quad(_Float16* p, float a, float b, float 
 
 template <typename Tin, typename Tout>
 __global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __restrict__ src, const float* __restrict__ meta,
-                                                                  const float* __restrict__ bank, Tout* __restrict__ out,
+                                                                  const h8* __restrict__ bank, Tout* __restrict__ out,
                                                                   F32HeadGeom G, unsigned* __restrict__ nonfinite) {
   __shared__ float4 tiles[2][2][kF32HPlane];                 // [buffer][column parity]
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, n = lane & 15, g = lane >> 4;
-  __shared__ f4 base[4 * 7];                                 // [phase][t]; in registers it costs the third wave per SIMD
-  f4 A[7];                                                   // K step j of row tile t
+  __shared__ h8 bank3[7 * 64];                               // the third parts' fragments and the base: kept in
+  __shared__ f4 base[4 * 7];                                 // registers they cost the third wave per SIMD
+  h8 A[7];
 #pragma unroll
-  for (int t = 0; t < 7; ++t) A[t] = *reinterpret_cast<const f4*>(bank + (t * 64 + lane) * 4);
-  if (tid < 28) base[tid] = *reinterpret_cast<const f4*>(bank + kF32HeadBase + 4 * tid);
+  for (int t = 0; t < 7; ++t) A[t] = bank[t * 64 + lane];
+  for (int i = tid; i < 7 * 64; i += kF32Threads) bank3[i] = bank[7 * 64 + i];
+  if (tid < 28) base[tid] = reinterpret_cast<const f4*>(bank + 14 * 64)[tid];
   const size_t oplane = (size_t)4 * G.H * G.W;
   float chk = 0.f;                                           // NaN once an output was not finite
   const int iters = tile_iters(G.num);
   int tidx = tile_of(0, G.num);
   // in flight: the next tile's RGB and the next chunk's coefficients (read as soon as the last ones are used)
   Tin rgb[kF32HPer][3];
-  float4 coef[2];                                            // [pixel parity]
+  float4 coef[2][2];                                         // [pixel parity][half of the lane's eight]
   if (tidx < G.num) {
     const F32HeadTile t = f32_head_tile(tidx, G);
     f32_head_rgb(rgb, src, t, G, tid);
@@ -789,7 +797,7 @@ __global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __r
 #pragma unroll
     for (int k = 0; k < kF32HPer; ++k) {
       const int q = tid + kF32Threads * k;                   // positions of a row alternate between the planes
-      if (q < kF32HPos) buf[q & 1][q >> 1] = make_float4((float)rgb[k][0], (float)rgb[k][1], (float)rgb[k][2], 0.f);
+      if (q < kF32HPos) buf[q & 1][q >> 1] = make_float4((float)rgb[k][0] * G.unscale, (float)rgb[k][1] * G.unscale, (float)rgb[k][2] * G.unscale, 0.f);
     }
     const int next = tile_of(it + 1, G.num);
     const bool more = it + 1 < iters && next < G.num;
@@ -805,25 +813,36 @@ __global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __r
     for (int j = 0; j < 2; ++j) {
       const int lane_j = fresh(lane);
       f4 w[2][7];
-      f4 c[2];
+      h8 bh[2], bl[2], bt[2];
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
-        c[p] = f4{clamp_coef(coef[p].x), clamp_coef(coef[p].y), clamp_coef(coef[p].z), clamp_coef(coef[p].w)};
+      for (int p = 0; p < 2; ++p) {
+        const float4 c0 = coef[p][0], c1 = coef[p][1];
+        const float c[8] = {clamp_coef(c0.x), clamp_coef(c0.y), clamp_coef(c0.z), clamp_coef(c0.w),
+                            clamp_coef(c1.x), clamp_coef(c1.y), clamp_coef(c1.z), clamp_coef(c1.w)};
+        u4 hi, lo, third;
 #pragma unroll
-      for (int q = 0; q < 7; ++q)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) w[p][q] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int q = 0; q < 7; ++q)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) w[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[q][k], c[p][k], w[p][q], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+          hi[e] = pack_h2(c[2 * e], c[2 * e + 1]);
+          const float r0 = residual_lo(c[2 * e], hi[e]), r1 = residual_hi(c[2 * e + 1], hi[e]);
+          lo[e] = pack_h2(r0, r1);
+          const unsigned t3 = pack_h2(residual_lo(r0, lo[e]), residual_hi(r1, lo[e]));
+          third[e] = (lane_j >> 4) < 2 ? hi[e] : t3;
+        }
+        bh[p] = __builtin_bit_cast(h8, hi);
+        bl[p] = __builtin_bit_cast(h8, lo);
+        bt[p] = __builtin_bit_cast(h8, third);
+      }
 #pragma unroll
       for (int q = 0; q < 7; ++q) {
+        const h8 a3 = bank3[q * 64 + lane_j];
         const f4 bs = base[(lane_j >> 4) * 7 + q];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) w[p][q] += bs;
+        for (int p = 0; p < 2; ++p) {
+          w[p][q] = mfma_f16(a3, bt[p], f4{0.f, 0.f, 0.f, 0.f});
+          w[p][q] = mfma_f16(A[q], bl[p], w[p][q]);
+          w[p][q] = mfma_f16(A[q], bh[p], w[p][q]);
+          w[p][q] = f4{bs[0] + w[p][q][0], bs[1] - w[p][q][1], bs[2] + w[p][q][2], bs[3] - w[p][q][3]};
+        }
       }
       if (j == 0) f32_head_coef(coef, meta, t, G, 1, wave, lane_j);
       else if (more) f32_head_coef(coef, meta, tn, G, 0, wave, lane_j);
@@ -948,12 +967,12 @@ hipError_t launch_f32_controller(int in_fp32, const void* src, const F32Weights&
 hipError_t launch_f32_head(int in_fp32, int out_fp32, const void* src, const float* meta, const F32Weights& wts, void* out,
                            int H, int W, int Hq, int Wq, int py, int px, int batch, int cus, unsigned* nonfinite,
                            hipStream_t stream) {
-  F32HeadGeom G{H, W, Hq, Wq, py, px, (W + kF32HW - 1) / kF32HW, (H + kF32HH - 1) / kF32HH, 0};
+  F32HeadGeom G{H, W, Hq, Wq, py, px, (W + kF32HW - 1) / kF32HW, (H + kF32HH - 1) / kF32HH, 0, wts.head_unscale};
   G.num = batch * G.tiles_x * G.tiles_y;
   const int grid = persistent_grid(G.num, 3 * cus);
 #define AEISU_F32_HEAD(TI, TO)                                                                                        \
   hipLaunchKernelGGL((f32_head_kernel<TI, TO>), dim3(grid), dim3(kF32Threads), 0, stream, (const TI*)src, meta,       \
-                     wts.head, (TO*)out, G, nonfinite)
+                     (const h8*)wts.head, (TO*)out, G, nonfinite)
   if (in_fp32 && out_fp32) AEISU_F32_HEAD(float, float);
   else if (in_fp32) AEISU_F32_HEAD(float, _Float16);
   else if (out_fp32) AEISU_F32_HEAD(_Float16, float);

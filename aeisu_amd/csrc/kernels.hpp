@@ -135,14 +135,15 @@ constexpr int kF32Analysis = kF32BiasTail + 64;
 constexpr int kF32Rows = kF32Analysis + 24 - kF32BiasCompress;
 constexpr int kF32Floats = kF32Rows + kF32Analysis;
 constexpr int kF32Unscale = 24;
-constexpr int kF32HeadBase = 7 * 64 * 4, kF32HeadFloats = kF32HeadBase + 4 * 7 * 4;
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
   const float* image;
   const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
-  const float* head;                       // FP32 bank [t][lane][K step] (row 4g + i of tile t: phase g, tap 4t + i; step j
-                                           // of lane group g: coefficient 4g + j), then the base float4 [g][t]
+  const void* head;                        // fragments [K_lo | K_hi] x 7 (row 4g + i of tile t: phase g, tap 4t + i) and
+                                           // [K_3 | K_hi] x 7, odd taps negated; the FP32 base float4 [g][t]; all
+                                           // divided by head_unscale
+  float head_unscale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong

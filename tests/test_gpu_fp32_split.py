@@ -255,8 +255,9 @@ def test_rows_of_small_weights(R, tmp_path):
                          ids=lambda s: "x".join(map(str, s)))
 def test_head_against_64_bits(model, size, dtypes):
     """The head on the GPU's own coefficients, at ragged widths and heights, in every pair of layouts.  An
-    output is 25 filter weights (16 products and a base, 17 FP32 roundings, of coefficients that the clamp rounds
-    twice) applied to the window (25 roundings): 44 x 2^-24 of the terms, and the output's rounding."""
+    output is 25 filter weights (sums of 16 products of exact parts, of which the 4 MFMA passes at the main terms'
+    magnitude cut off up to 2^-24 in each of their 8 terms and the sum, 36 x 2^-24; the base; the clamp rounds a
+    coefficient twice) applied to the window (25 roundings): 64 x 2^-24 of the terms, and the output's rounding."""
     from aeisu_amd import _lib as L
     kind = {"f16": torch.float16, "f32": torch.float32}
     m, state = model
@@ -272,7 +273,7 @@ def test_head_against_64_bits(model, size, dtypes):
     base, basis = state["base"].double(), state["basis"].double()
     ref = crop_output(M.reconstruct(padded, meta, base, basis), h, w)
     size_ = crop_output(M.reconstruct(padded.abs(), meta.abs(), base.abs(), basis.abs()), h, w)
-    bound = 44 * 2.0 ** -24 * size_ + 1e-12
+    bound = 64 * 2.0 ** -24 * size_ + 1e-12
     if dtypes[1] == "f16":
         bound = bound + 2.0 ** -11 * ref.abs() + 2.0 ** -25
     over = (got - ref.clamp(0, 1)).abs() - bound
@@ -300,9 +301,8 @@ def head_chain(padded, meta, base, basis, y0, x0, h, w):
 
 def test_head_no_further_from_64_bits_than_fma_chains(model):
     """The error over a whole frame, not only a bound of every value: its norm is at most that of FP32 FMA chains
-    (0.98 of it on the GPU), and its mean is zero, as rounding to nearest leaves it.  An error of some 5e-8 in each of
-    270,000 outputs, alike over the windows of about 100 of them, has a mean of 1e-9 by chance; sums that cut bits
-    off instead of rounding shift it by 1.3e-8."""
+    (0.91 to 0.93 of it on the GPU), and its mean at most a tenth of its root mean square, a share of 0.5 % of the
+    norm.  Sums that all cut bits off in one direction have a mean of a quarter of it."""
     from aeisu_amd import _lib as L
     from aeisu_amd import frames as scenes
     m, state = model
@@ -320,4 +320,4 @@ def test_head_no_further_from_64_bits_than_fma_chains(model):
     ours, theirs = got.double() - ref, one.double() - ref
     print(f"  error norm {ours.norm():.4g}, FMA chains {theirs.norm():.4g}; mean {ours.mean():.3g}, {theirs.mean():.3g}", flush=True)
     assert ours.norm() <= theirs.norm()
-    assert ours.mean().abs() <= 3e-9
+    assert ours.mean().abs() <= 0.1 * ours.square().mean().sqrt()
