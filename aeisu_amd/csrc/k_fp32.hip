@@ -349,7 +349,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
   __shared__ __attribute__((aligned(16))) unsigned red[16];
   __shared__ __attribute__((aligned(16))) float rows[32];
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, grp = blockIdx.y;
-  if (tid < 32) rows[tid] = bias[kF32Rows + 32 * grp + tid];
+  const float row = bias[kF32Rows + 32 * grp + (tid & 31)];   // stored once the loads below are under way
   const int n = lane & 15, g = lane >> 4;
   float4 v[LY::Per];
   int tidx = tile_of(0, G.num);
@@ -359,6 +359,7 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
   f4 bs[2];
 #pragma unroll
   for (int T = 0; T < 2; ++T) bs[T] = *reinterpret_cast<const f4*>(bias + 32 * grp + 16 * T + 4 * g);
+  if (tid < 32) rows[tid] = row;                     // the loop's barriers are before the reads
   const int iters = tile_iters(G.num);
   for (int it = 0; it < iters; ++it) {
     if (tidx >= G.num) break;                        // block-uniform
@@ -425,15 +426,12 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
   __shared__ __attribute__((aligned(16))) float rb[128], tb[128];   // biases and row scales: in registers the kernel spills
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, role = wave & 1, half = wave >> 1;
   float4 v[LY::Per];
-  {
-    const int i = (tid & 63) + (tid & 64 ? kF32Rows : 0);
-    if (tid < 128) rb[tid] = rbias[i];
-    else tb[tid - 128] = tbias[i];
-  }
+  const float row = (tid < 128 ? rbias : tbias)[(tid & 63) + (tid & 64 ? kF32Rows : 0)];
   int tidx = tile_of(0, G.num);
   if (tidx < G.num) conv_fetch<LY::Per, 32>(v, work, G, tidx, TH, LY::Chunks, tid);
   h8 A[9][2][2];
   conv_weights(A, rfrag, role, lane);
+  (tid < 128 ? rb : tb)[tid & 127] = row;            // the loop's barriers are before the reads
   const int iters = tile_iters(G.num);
   for (int it = 0; it < iters; ++it) {
     if (tidx >= G.num) break;                        // block-uniform
@@ -455,6 +453,12 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
         const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
         f4 acc[R][2];
         conv_rows<R>(smem + (row * kConvPW + n) * kConvPix + 16 * g, A, acc);
+        f4 b0[2], sc[2];
+#pragma unroll
+        for (int T = 0; T < 2; ++T) {
+          b0[T] = *reinterpret_cast<const f4*>(rb + 32 * role + 16 * T + 4 * g);
+          sc[T] = *reinterpret_cast<const f4*>(rb + 64 + 32 * role + 16 * T + 4 * g);
+        }
 #pragma unroll
         for (int j = 0; j < R; ++j) {
           unsigned char* pix = smem + LY::SizeHalo + ((row + j) * kConvTW + n) * LY::RPix;
@@ -463,15 +467,14 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
           float m = 0.f;
 #pragma unroll
           for (int T = 0; T < 2; ++T) {
-            r[T] = *reinterpret_cast<const f4*>(rb + 32 * role + 16 * T + 4 * g);
-            const f4 sc = *reinterpret_cast<const f4*>(rb + 64 + 32 * role + 16 * T + 4 * g);
+            r[T] = b0[T];
             if (!first) {                            // the sum so far
               const f2 a = *reinterpret_cast<const f2*>(d + 32 * T), c = *reinterpret_cast<const f2*>(d + 32 * T + 128);
               r[T] = f4{a[0], a[1], c[0], c[1]};
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              r[T][i] = fmaf(acc[j][T][i] * inv, sc[i], r[T][i]);
+              r[T][i] = fmaf(acc[j][T][i] * inv, sc[T][i], r[T][i]);
               if (last) r[T][i] = leaky(r[T][i], 0.1f);
               m = fmaxf(m, fabsf(r[T][i]));
             }
@@ -509,9 +512,10 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
 #pragma unroll
       for (int part = 0; part < 2; ++part) At[k][part] = tf[(k * 2 + part) * 64];
     lds_barrier();
+    const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
+    const f4 bias = *reinterpret_cast<const f4*>(tb + 16 * wave + 4 * g), sc = *reinterpret_cast<const f4*>(tb + 64 + 16 * wave + 4 * g);
 #pragma unroll 2
     for (int row = 0; row < TH; ++row) {
-      const int ln = fresh(lane), n = ln & 15, g = ln >> 4;
       const unsigned char* pix = smem + LY::SizeHalo + (row * kConvTW + n) * LY::RPix;
       f4 acc[2];                                     // K chunk k: channels 32 k .. + 31, which share a scale
 #pragma unroll
@@ -522,8 +526,6 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
         acc[k] += mfma_f16(At[k][1], bh, small);
       }
       const float2 inv = *reinterpret_cast<const float2*>(pix + 256);
-      const f4 bias = *reinterpret_cast<const f4*>(tb + 16 * wave + 4 * g);
-      const f4 sc = *reinterpret_cast<const f4*>(tb + 64 + 16 * wave + 4 * g);
       const int qy = y0 + row, qx = x0 + n;
       if (qy < G.H && qx < G.W) {
         f4 o;
@@ -575,11 +577,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
       v[2 * k + 1] = *reinterpret_cast<const float4*>(q + 4);
     }
   };
+  __shared__ __attribute__((aligned(16))) float rows[64];
+  const float row = bias[kF32Rows + (threadIdx.x & 63)];
   float4 v[8];
   if (grp < groups) fetch(grp, v);
-  __shared__ __attribute__((aligned(16))) float rows[64];
-  if (threadIdx.x < 64) rows[threadIdx.x] = bias[kF32Rows + threadIdx.x];
-  lds_barrier();
   h8 A[4][4][2];
   f4 bs[4];
 #pragma unroll
@@ -590,6 +591,8 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_compress_kernel(const floa
 #pragma unroll
       for (int part = 0; part < 2; ++part) A[T][k][part] = frag[((T * 4 + k) * 2 + part) * 64 + lane];
   }
+  if (threadIdx.x < 64) rows[threadIdx.x] = row;
+  lds_barrier();
   for (; grp < groups; grp += waves) {
     const int ex = scale_exponent(as_float(max_of_rows(as_bits(chunk_max(v)))));
     const float s = pow2f(ex), inv = inverse_scale(ex);
@@ -635,14 +638,11 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
       v[2 * k + 1] = *reinterpret_cast<const float4*>(s + 32 * k + 4);
     }
   };
+  __shared__ __attribute__((aligned(16))) float sb[256];   // bias, then row scale, by row tile and row
+  const int rt = threadIdx.x >> 4 & 7;
+  const float row = bias[(threadIdx.x < 128 ? 0 : kF32Rows) + (16 * (rt >> 2) + (threadIdx.x & 15)) * 4 + (rt & 3)];
   float4 v[4];
   if (grp < groups) fetch(grp, v);
-  __shared__ __attribute__((aligned(16))) float sb[256];   // bias, then row scale, by row tile and row
-  {
-    const int T = threadIdx.x >> 4 & 7, m = threadIdx.x & 15;
-    sb[threadIdx.x] = bias[(threadIdx.x < 128 ? 0 : kF32Rows) + (16 * (T >> 2) + m) * 4 + (T & 3)];
-  }
-  lds_barrier();
   h8 A[8][2][2];
 #pragma unroll
   for (int T = 0; T < 8; ++T)
@@ -650,6 +650,8 @@ __global__ __launch_bounds__(kF32Threads, 2) void f32_expand_kernel(const float*
     for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int part = 0; part < 2; ++part) A[T][k][part] = frag[((T * 2 + k) * 2 + part) * 64 + lane];
+  sb[threadIdx.x] = row;
+  lds_barrier();
   for (; grp < groups; grp += waves) {
     const int idx = grp * 16 + n;
     const LowPixel p = low_pixel(min(idx, pixels - 1), Hl, Wl);
