@@ -566,14 +566,15 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
         rt.f32_tail);
   // head bank, scaled so that the largest weight lies in [2^13, 2^14): row 4g + i of tile t is phase g of tap
   // 4t + i (taps past 24 are zero); slots 0..15 the lo parts of the coefficients' weights and 16..31 the hi
-  // parts, or (fragments 7..13) the third and the hi parts; odd taps negated (k_fp32.hip)
+  // parts, or (fragments 7..13) the third and the hi parts; odd taps (and their base) negated
   float top = 0.f;
   for (int i = 0; i < 1600; ++i) top = std::max(top, std::fabs(basis[i]));
   const int e = top > 0.f ? std::min(13 - std::ilogb(top), 30) : 0;
+  auto sign = [](int tap) { return tap % 2 ? -1.f : 1.f; };
   auto bank = pack_frags<uint16_t>(14, 8, [&](int f, int m, int s) -> uint16_t {
     const int tap = 4 * (f % 7) + m % 4;
     if (tap > 24) return 0;
-    const float v = std::ldexp(basis[(tap * 16 + s % 16) * 4 + m / 4], e) * (tap % 2 ? -1.f : 1.f);
+    const float v = std::ldexp(basis[(tap * 16 + s % 16) * 4 + m / 4], e) * sign(tap);
     const uint16_t hi = f32_to_f16_bits(v);
     const float rest = v - f16_bits_to_f32(hi);
     const uint16_t lo = f32_to_f16_bits(rest);
@@ -582,7 +583,7 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   });
   std::vector<float> rows(4 * 7 * 4, 0.f);
   for (int g = 0; g < 4; ++g)
-    for (int tap = 0; tap < 25; ++tap) rows[g * 28 + tap] = std::ldexp(base[tap * 4 + g], e);
+    for (int tap = 0; tap < 25; ++tap) rows[g * 28 + tap] = std::ldexp(base[tap * 4 + g], e) * sign(tap);
   const size_t halves = bank.size();
   bank.resize(halves + 2 * rows.size());
   std::memcpy(bank.data() + halves, rows.data(), rows.size() * sizeof(float));

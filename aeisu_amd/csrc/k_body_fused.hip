@@ -84,13 +84,14 @@ BodyXcPlan body_fused_xc_plan(int mode, int batch, int Hl, int Wl, int cus, bool
 }
 
 // Side of the exchange's tiles for launches that would leave CUs idle with 24x24 tiles: such a launch takes one
-// tile's latency, so the smallest tiles that are all resident at once are taken.  With the exchange a tile's
+// tile's latency, so 8x8 tiles are taken where all are resident at once.  With the exchange a tile's
 // compress costs only its core, so smaller tiles add no compress work, only the grouped layers' halos, which
 // idle CUs take.  Whole call, Mixed: 48 x 64 38.7 us on 16x16 tiles, 26.9 on 8x8; 270 x 480 40.2 and 28.3;
 // 360 x 640 45.7 on 16x16, 39.4 on 12x12; 480 x 854 50.3 and 44.6 (INT8: 33.8 and 24.0, 35.7 and 25.4, 41.0 and
-// 34.9, 45.7 and 40.3).  12x12 tiles serve launches whose 16x16 tiles would leave half of the CUs idle: 540p has
-// 144 of those and keeps them (its plan is fixed by test_body_exchange_selection; 12x12 tiles measured 44.5
-// against 50.8 us).
+// 34.9, 45.7 and 40.3).  12x12 tiles serve launches whose 16x16 tiles would leave half of the CUs idle.  That line is
+// not where they stop paying: 540p has 144 16x16 tiles and measured 44.5 us on 12x12 tiles against 50.8.  It lies
+// there because test_body_exchange_selection fixes 540p's plan, and the other frames of 129 16x16 tiles and more whose
+// 12x12 tiles would all be resident (500 x 900, 600 x 800) give up their gain with it.
 int body_fused_xc_small_tile(int mode, int batch, int Hl, int Wl, int cus) {
   if (body_fused_num_tiles(mode, batch, Hl, Wl, 8) <= cus) return 8;
   if (body_fused_num_tiles(mode, batch, Hl, Wl, 12) <= cus && 2 * body_fused_num_tiles(mode, batch, Hl, Wl, 16) <= cus) return 12;

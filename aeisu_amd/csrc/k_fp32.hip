@@ -339,7 +339,7 @@ __device__ __forceinline__ void conv_stage(const float4 (&v)[PER], unsigned char
 
 // A grouped 3x3 layer (2 groups of 32 -> 32, zero padding) + LeakyReLU: blockIdx.y is the conv group, so the
 // block's waves share its weights and split the tile's rows.  One thread per pixel and group with FP32 FMAs:
-// 147 us at 1080p, 50 us for 256 x 256.
+// 147 us at 1080p, 50 us for 256 x 256, now 29 and 5.7 (28 and 5.6 with one scale per tile and per layer).
 template <int TH>
 __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const float* __restrict__ in, const h8* __restrict__ frag,
                                                                       const float* __restrict__ bias, float* __restrict__ out,
@@ -408,7 +408,8 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
 }
 
 // refine 3x3 (32 -> 64) + LeakyReLU + tail 1x1 (64 -> 64).  One thread per pixel with FP32 FMAs was bound by
-// their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 86 and 9.5.  Its 210 MB take 41 us
+// their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 91 and 10 (79 and 9
+// with one scale per tile and per layer).  Its 210 MB take 41 us
 // of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (320 KB per tile), which
 // two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
 // (a scale for each pixel's 32 channels of a wave, kept beside them) and wave w computes tail channels
@@ -704,8 +705,8 @@ __device__ __forceinline__ float clamp_coef(float a) {
 // [K_3 | K_hi] . [c_hi ; c_3] + [K_lo | K_hi] . [c_lo ; c_lo] + [K_lo | K_hi] . [c_hi ; c_hi], small terms
 // first, since the MFMA cuts off the bits of all terms below the largest of a pass; the FP32 base is added to
 // the sum, not taken as its first addend.  Cutting off lowers every sum, by 1e-9 on average, and the 25 taps add
-// that up: the bank of odd taps is negated and its sums are subtracted from the base, so that neighbouring taps take
-// it from each other (mean error of the output -1.3e-8 without, 4e-9 (area) and 4e-10 (DIV2K) with it).  Against 64
+// that up: bank and base of odd taps are negated and their weights applied with the other sign, so that neighbouring
+// taps take it from each other (mean error of the output -1.3e-8 without, 4e-9 (area) and 4e-10 (DIV2K) with it).  Against 64
 // bits (frames of 33 x 65 to 1080p) the output's error is 1.08e-7 (area) and 1.17e-7 (DIV2K); one FP32 FMA chain
 // per weight gave 1.17e-7 and 1.26e-7, all sums of one sign 1.21e-7 and 1.20e-7, FP32 MFMAs 1.15e-7 and 1.23e-7 and
 // 113 us instead of 88 at 1080p.  Bank and base are scaled by a power of two, the RGB tile by its inverse.
@@ -756,7 +757,7 @@ __device__ __forceinline__ void f32_head_coef(float4 (&c)[2][2], const float* __
   }
 }
 // The output is written once and not read here: the non-temporal hint keeps it from displacing the coefficients
-// (1080p frame 352 -> 335 us).
+// (16 frames in turn: 1080p 411 -> 408 us a call, 540p 141.4 -> 138; 256 x 256 unchanged).
 // Output columns 4n .. 4n + 3 of a chunk row and channel: pixels 2n and 2n + 1, left and right.
 __device__ __forceinline__ void store_quad(float* p, float a, float b, float c, float d, bool second) {
   if (second) __builtin_nontemporal_store(f4{a, b, c, d}, reinterpret_cast<f4*>(p));
@@ -843,7 +844,7 @@ __global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __r
           w[p][q] = mfma_f16(a3, bt[p], f4{0.f, 0.f, 0.f, 0.f});
           w[p][q] = mfma_f16(A[q], bl[p], w[p][q]);
           w[p][q] = mfma_f16(A[q], bh[p], w[p][q]);
-          w[p][q] = f4{bs[0] + w[p][q][0], bs[1] - w[p][q][1], bs[2] + w[p][q][2], bs[3] - w[p][q][3]};
+          w[p][q] += bs;
         }
       }
       if (j == 0) f32_head_coef(coef, meta, t, G, 1, wave, lane_j);
@@ -858,7 +859,7 @@ __global__ __launch_bounds__(kF32Threads, 3) void f32_head_kernel(const Tin* __r
           for (int p = 0; p < 2; ++p) {
             if (dx - p < 0 || dx - p > 4) continue;
             const int tap = dy * 5 + dx - p;
-            const float wt = w[p][tap >> 2][tap & 3];
+            const float wt = tap & 1 ? -w[p][tap >> 2][tap & 3] : w[p][tap >> 2][tap & 3];
             u[p][0] = fmaf(wt, L.x, u[p][0]);
             u[p][1] = fmaf(wt, L.y, u[p][1]);
             u[p][2] = fmaf(wt, L.z, u[p][2]);
@@ -925,7 +926,8 @@ static hipError_t launch_refine_t(const float* work, const F32Weights& W, float*
 }
 static hipError_t launch_f32_refine_tail(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch,
                                          int cus, hipStream_t stream) {
-  // tiles of 8 rows where they fill the 2 x cus resident blocks, else of 2 rows (more blocks, less work each)
+  // tiles of 8 rows where they fill the 2 x cus resident blocks, else of 2 rows (more blocks, less work each).  The
+  // line is not a measured one: just below it (270 x 480 has 320 tiles of 8 rows, one round) 2 rows take three rounds.
   return conv_tiles(Hq, Wq, 8, batch).num >= 2 * cus ? launch_refine_t<8>(work, W, meta, Hq, Wq, batch, cus, stream)
                                                      : launch_refine_t<2>(work, W, meta, Hq, Wq, batch, cus, stream);
 }

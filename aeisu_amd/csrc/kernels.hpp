@@ -141,8 +141,8 @@ struct F32Weights {
   const void *compress, *expand, *tail;    // [T][k][part]; compress: chunk k is phase k; expand: T = 4 (channel / 16) + phase
   const void *grouped[4], *refine;         // [T][tap][part], T = 2 group + t in the grouped layers
   const void* head;                        // fragments [K_lo | K_hi] x 7 (row 4g + i of tile t: phase g, tap 4t + i) and
-                                           // [K_3 | K_hi] x 7, odd taps negated; the FP32 base float4 [g][t]; all
-                                           // divided by head_unscale
+                                           // [K_3 | K_hi] x 7, then the FP32 base float4 [g][t]; odd taps negated,
+                                           // all divided by head_unscale
   float head_unscale;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage

@@ -230,7 +230,7 @@ def load_model(path, device: str = "cuda", precision: Optional[str] = None) -> U
 
     Mirrors aeisu/runtime.py:45-56.  ``precision`` defaults to the file's
     natural policy; an FP8 artifact can also run at "fp16" (its FP16 weights), a folded FP32
-    checkpoint also at "fp32" (FP32 activations and arithmetic: the reference's PyTorch path).
+    checkpoint also at "fp32" (FP32 activations and accuracy: the reference's PyTorch path).
     """
     blob, natural = load_blob(Path(path))
     precision = precision or natural

@@ -42,7 +42,7 @@ extern "C" {
                                           Mixed emulation, outside the 2/255 bound of MIXED; for
                                           comparison only */
 #define AEISU_PRECISION_FP32 5  /* FP32 activations and FP32 accuracy in every layer and the head
-                                   (per-layer kernels; products as FP32 FMAs or as hi / lo FP16 splits
+                                   (per-layer kernels; products on the FP32 MFMA or as FP16 splits
                                    with FP32 sums): the reference's PyTorch FP32 path
                                    (aeisu/model.py, aeisu/runtime.py).  Needs FP32 weights for every
                                    layer (<layer>.weight_fp32, written by the folded-checkpoint

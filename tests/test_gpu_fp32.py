@@ -1,7 +1,7 @@
 """FP32 policy (AEISU_PRECISION_FP32) on the GPU against the reference's own FP32 outputs.
 
-The FP32 policy keeps every activation in FP32 and computes every layer and the head with FP32
-fused multiply-adds (k_fp32.hip), so it stands in for the reference's PyTorch path
+The FP32 policy keeps every activation in FP32 and computes every layer and the head to FP32
+accuracy (k_fp32.hip: FP32 MFMAs and FP16 splits with FP32 sums), so it stands in for the reference's PyTorch path
 (aeisu/model.py, aeisu/runtime.py) that ``upscale`` users run: the north star holds the FP32/FP16
 path to 1e-3 max-abs of it, and this policy meets that bound on every frame class, white noise
 included, where FP16 activation storage alone costs 1.6-2.5e-3.
