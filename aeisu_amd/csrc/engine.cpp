@@ -316,6 +316,7 @@ struct ModeWeights {
   // FP32 policy, layers run as hi / lo FP16 splits: fragments and scales
   DeviceBuffer f32_compress, f32_grouped[4], f32_expand, f32_refine, f32_tail, f32_head;
   float f32_head_unscale = 1.f;
+  F32Bound f32_refine_bound{};
 
   // every device buffer, for commit() and byte accounting
   template <typename Fn>
@@ -345,6 +346,7 @@ struct ModeWeights {
     W.expand = f32_expand.ptr;
     W.head = f32_head.ptr;
     W.head_unscale = f32_head_unscale;
+    W.refine_bound = f32_refine_bound;
     W.refine = f32_refine.ptr;
     W.tail = f32_tail.ptr;
     return W;
@@ -562,6 +564,15 @@ static void pack_fp32(ModeWeights& rt, const Artifact& a, const float* base, con
   for (int l = 0; l < 4; ++l)
     split("bottleneck" + std::to_string(l), 64, 32, 3, kF32BiasGrouped + 64 * l, 36, conv3, rt.f32_grouped[l]);
   split("refine", 64, 32, 3, kF32BiasRefine, 36, conv3, rt.f32_refine);
+  const float* wr = w32("refine", 64, 32, 3);
+  double gain = 0, offset = 0;
+  for (int o = 0; o < 64; ++o) {
+    double sum = 0;
+    for (int i = 0; i < 288; ++i) sum += std::fabs((double)wr[o * 288 + i]);
+    gain = std::max(gain, sum);
+    offset = std::max(offset, std::fabs((double)img[kF32BiasRefine + o]));
+  }
+  rt.f32_refine_bound = {(float)(1.001 * gain), (float)(1.001 * offset)};   // the margin covers the sums' rounding
   split("tail", 64, 64, 1, kF32BiasTail, 8, [](int f, int m, int s) { return (16 * (f / 2) + m) * 64 + 32 * (f % 2) + s; },
         rt.f32_tail);
   // head bank, scaled so that the largest weight lies in [2^13, 2^14): row 4g + i of tile t is phase g of tap

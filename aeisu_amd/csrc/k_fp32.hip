@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64) void f32_project_kernel(const Tin* __restrict__
 // of their own: added to the main sum they would be rounded at its magnitude.
 //
 // The scale keeps FP32's range: the largest magnitude that shares it goes to [2^14, 2^15), so nothing overflows
-// FP16, and the lo halves end at 2^-39 of that.  The 1x1 layers and the tail take a scale per pixel.  The 3x3 layers
+// FP16, and the lo halves end at 2^-39 of that.  The 1x1 layers take a scale per pixel.  The 3x3 layers
 // take the tile's largest (finite) pixel, and pixels below 2^-14 of it in a pass of their own with their own
 // scale (bands): a pixel's values are thus held to 2^-22 of themselves or 2^-25 of its largest, whatever lies
 // beside it.  Weights are scaled by output (row): 2^e with the row's largest in [2^14, 2^15).  A sum is brought back
@@ -408,19 +408,20 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_grouped_kernel(const floa
 }
 
 // refine 3x3 (32 -> 64) + LeakyReLU + tail 1x1 (64 -> 64).  One thread per pixel with FP32 FMAs was bound by
-// their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 91 and 10 (79 and 9
-// with one scale per tile and per layer).  Its 210 MB take 41 us
+// their issue (22,528 per pixel): 511 us at 1080p, 98 us for 256 x 256, now 88 and 10 (81 and 9
+// with one scale per tile and per layer, 94 with a scale per pixel for the tail of every tile).  Its 210 MB take 41 us
 // of HBM time at 1080p and its MFMAs 34; the rest is the splitting and the LDS reads (320 KB per tile), which
 // two waves per SIMD do not hide.  The refine outputs go to LDS as hi and lo halves
-// (a scale for each pixel's 32 channels of a wave, kept beside them) and wave w computes tail channels
-// 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
+// (scaled by their bound from the tile's largest input and the weights; where a tile has several bands, a scale for
+// each pixel's 32 channels of a wave, kept beside them) and wave w computes tail channels 16 w .. + 15 from them; refine: channels 32 (w & 1) .. + 31 of the rows of half w >> 1.
 template <int TH>
 __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const float* __restrict__ work,
                                                                           const h8* __restrict__ rfrag,
                                                                           const h8* __restrict__ tfrag,
                                                                           const float* __restrict__ rbias,
                                                                           const float* __restrict__ tbias,
-                                                                          float* __restrict__ meta, F32ConvTiles G) {
+                                                                          float* __restrict__ meta, F32ConvTiles G,
+                                                                          F32Bound bound) {
   typedef ConvLayout<TH> LY;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LY::LdsRefine];
   __shared__ __attribute__((aligned(16))) unsigned red[16];
@@ -440,6 +441,9 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
     const int ty = rem / G.tiles_x, y0 = ty * TH, x0 = (rem - ty * G.tiles_x) * kConvTW;
     const int next = tile_of(it + 1, G.num);
     PixelRange rg = tile_range(v, red, wave, lane);
+    // a tile of one band scales its refine outputs by their bound
+    const bool single = rg.bottom >= rg.top * kBand;
+    const int eb = scale_exponent(fminf(fmaf(bound.gain, rg.top, bound.offset), 0x1p126f));
     for (float cap = __builtin_inff();;) {           // over the tile's bands
       const float low = rg.top * kBand;
       const bool first = cap == __builtin_inff(), last = rg.bottom >= low;
@@ -465,7 +469,6 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
           unsigned char* pix = smem + LY::SizeHalo + ((row + j) * kConvTW + n) * LY::RPix;
           unsigned char* d = pix + 64 * role + 8 * g;
           f4 r[2];
-          float m = 0.f;
 #pragma unroll
           for (int T = 0; T < 2; ++T) {
             r[T] = b0[T];
@@ -477,12 +480,17 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
             for (int i = 0; i < 4; ++i) {
               r[T][i] = fmaf(acc[j][T][i] * inv, sc[T][i], r[T][i]);
               if (last) r[T][i] = leaky(r[T][i], 0.1f);
-              m = fmaxf(m, fabsf(r[T][i]));
             }
           }
           if (last) {
-            const int er = scale_exponent(as_float(max_of_rows(as_bits(m))));   // of the pixel's 32 channels in this wave
-            const float s = pow2f(er);
+            float s = pow2f(eb);
+            if (!single) {                           // by the pixel's 32 channels in this wave
+              const float m = fmaxf(abs_max(make_float4(r[0][0], r[0][1], r[0][2], r[0][3])),
+                                    abs_max(make_float4(r[1][0], r[1][1], r[1][2], r[1][3])));
+              const int er = scale_exponent(as_float(max_of_rows(as_bits(m))));
+              s = pow2f(er);
+              if (g == 0) *reinterpret_cast<float*>(pix + 256 + 4 * role) = inverse_scale(er);
+            }
 #pragma unroll
             for (int T = 0; T < 2; ++T) {
               u2 hi, lo;
@@ -490,7 +498,6 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
               *reinterpret_cast<u2*>(d + 32 * T) = hi;
               *reinterpret_cast<u2*>(d + 32 * T + 128) = lo;
             }
-            if (g == 0) *reinterpret_cast<float*>(pix + 256 + 4 * role) = inverse_scale(er);
           } else {
 #pragma unroll
             for (int T = 0; T < 2; ++T) {
@@ -526,7 +533,8 @@ __global__ __launch_bounds__(kConvThreads, 2) void f32_refine_tail_kernel(const 
         acc[k] = mfma_f16(At[k][0], bh, f4{0.f, 0.f, 0.f, 0.f});
         acc[k] += mfma_f16(At[k][1], bh, small);
       }
-      const float2 inv = *reinterpret_cast<const float2*>(pix + 256);
+      float2 inv = make_float2(inverse_scale(eb), inverse_scale(eb));
+      if (!single) inv = *reinterpret_cast<const float2*>(pix + 256);
       const int qy = y0 + row, qx = x0 + n;
       if (qy < G.H && qx < G.W) {
         f4 o;
@@ -921,7 +929,7 @@ static hipError_t launch_refine_t(const float* work, const F32Weights& W, float*
                                   hipStream_t stream) {
   const F32ConvTiles G = conv_tiles(Hq, Wq, TH, batch);
   hipLaunchKernelGGL(f32_refine_tail_kernel<TH>, dim3(persistent_grid(G.num, 2 * cus)), dim3(kConvThreads), 0, stream, work,
-                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32BiasRefine, W.image + kF32BiasTail, meta, G);
+                     (const h8*)W.refine, (const h8*)W.tail, W.image + kF32BiasRefine, W.image + kF32BiasTail, meta, G, W.refine_bound);
   return hipGetLastError();
 }
 static hipError_t launch_f32_refine_tail(const float* work, const F32Weights& W, float* meta, int Hq, int Wq, int batch,

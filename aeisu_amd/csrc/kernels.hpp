@@ -135,6 +135,10 @@ constexpr int kF32Analysis = kF32BiasTail + 64;
 constexpr int kF32Rows = kF32Analysis + 24 - kF32BiasCompress;
 constexpr int kF32Floats = kF32Rows + kF32Analysis;
 constexpr int kF32Unscale = 24;
+// An output's magnitude is at most gain * (largest input magnitude) + offset.
+struct F32Bound {
+  float gain, offset;
+};
 // The image above and the split layers' MFMA fragments (hi then lo of each K chunk, FP16).
 struct F32Weights {
   const float* image;
@@ -144,6 +148,7 @@ struct F32Weights {
                                            // [K_3 | K_hi] x 7, then the FP32 base float4 [g][t]; odd taps negated,
                                            // all divided by head_unscale
   float head_unscale;
+  F32Bound refine_bound;
 };
 // project, compress, the four grouped layers, expand, refine + tail (events 1..5 after each stage
 // when ev is not null); lows: the five layer outputs when every layer is kept, else null (ping-pong
