@@ -179,7 +179,7 @@ def test_finite_outlier_stays_local(model, size, value):
 
 
 @pytest.mark.parametrize("size", [(1, 45, 70), (3, 150, 1030)], ids=lambda s: "x".join(map(str, s)))
-@pytest.mark.parametrize("values", [(1e8,), (-1e12, 3e5), (1e30, 1e-30, 1e10)], ids=str)
+@pytest.mark.parametrize("values", [(30.0,), (500.0, -5e3), (2e4,), (1e8,), (-1e12, 3e5), (1e30, 1e-30, 1e10)], ids=str)
 def test_stages_with_outliers(model, size, values):
     """Pixels far apart in magnitude within a tile: every stage within the bound of each pixel's own window."""
     print(f"case: FP32 stages {size} with pixels at {values}", flush=True)
